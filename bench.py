@@ -56,7 +56,8 @@ def parse():
     ap.add_argument("--autotune", type=int, default=1, help="pick the schedule with esl_plan_autotune first")
     ap.add_argument("--schedule", type=int, default=None,
                     help="pin a schedule instead of autotuning (0 per-set, 1 per-set global, 2 device-wide, "
-                         "3 per-set LDS with the basis in global memory, 4/5 per-set at 3/2 workgroups per CU)")
+                         "3 per-set LDS with the basis in global memory, 4 per-set at 3 workgroups per CU, 5 per-set on the "
+                         "parity-reduced system)")
     ap.add_argument("--restart", type=int, default=32, help="GMRES restart length of a pinned --schedule")
     ap.add_argument("--workload", default="n20", choices=["n20", "n16", "uneven", "n22", "warm", "seeds"],
                     help="n20 (default) is the headline metric; the others print their own JSON line")
@@ -148,7 +149,7 @@ def copy_calibration(L, ctx):
 
 
 SCHEDULE_NAMES = ["per-set LDS-resident", "per-set global", "device-wide", "per-set LDS, basis in memory",
-                  "per-set LDS-resident, 3 workgroups per CU", "per-set LDS-resident, 2 workgroups per CU"]
+                  "per-set LDS-resident, 3 workgroups per CU", "per-set, parity-reduced BiCGStab"]
 
 
 def host_cpu():

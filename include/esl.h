@@ -152,12 +152,14 @@ typedef struct
 	int precision;		 /* 0 = FP64 Krylov solves; 1 = FP32 inner solves + FP64 residual refinement */
 	double tol;			 /* relative residual target of every linear solve (default 1e-13) */
 	int max_iters;		 /* Krylov iterations per solve before ESL_E_NUMERIC (default 20000) */
-	int restart;		 /* GMRES restart length: at most 64 for the per-set solvers, 128 for the
-						  * device-wide solver; 0 (default): a plan's autotuned length, else 32 (the
-						  * device-wide solver halves it while its FP64 basis would exceed half the
-						  * free device memory) */
+	int restart;		 /* > 0 asks for restarted GMRES with this restart length: at most 64 for the
+						  * per-set solvers, 128 for the device-wide solver; 0 (default): a plan's
+						  * autotuned schedule, else the default method (per set, BiCGStab on the
+						  * parity-reduced system; device-wide, GMRES at 32, halved while its FP64
+						  * basis would exceed half the free device memory) */
 	int full;			 /* 1: also build solution_term / solution_nonterm (esl_solution_export) */
-	int preconditioner;	 /* 0 = default (ILU(0)), 1 = Jacobi, 2 = ILU(0) (level-scheduled) */
+	int preconditioner;	 /* 0 = default (ILU(0) where GMRES runs), 1 = Jacobi, 2 = ILU(0) (level-scheduled);
+						  * 1 and 2 ask for GMRES */
 	int graph;			 /* 1: capture the numeric sequence of a plan in a HIP graph and replay it */
 	const double* warm_pi; /* optional warm start of the terminal kernels: predicted final-vector values
 							* on the terminal states in canonical order (reordered_vertices[0, n_t)),
@@ -173,7 +175,7 @@ typedef struct
 typedef struct
 {
 	double residual;	 /* max relative FP64 residual over the linear systems solved */
-	int iterations;		 /* total Krylov iterations */
+	int iterations;		 /* total Krylov iterations (products by the system matrix) */
 	int refinements;	 /* FP64 refinement steps (precision 1) */
 	int64_t reachable;	 /* states reachable from supp(x0) */
 	int64_t unknowns;	 /* unknowns of the linear systems (terminal kernels + ambiguous transient states) */
@@ -264,9 +266,10 @@ esl_status esl_plan_gather_terminal(esl_ctx* ctx, const esl_plan* p, int n_sets,
 /* Autotuner: runs this batch under each candidate schedule -- 0 per-set solve with
  * the system in LDS (FP32 basis in registers where it fits), 1 per-set from global
  * memory, 2 device-wide, 3 per-set with the system in LDS and the basis in global
- * memory, 4 and 5 as 0 with 3 and 2 workgroups per CU (more registers: the basis of
- * systems up to 1024 unknowns then stays in registers) -- and restart length
- * 16 / 24 / 32 / 64, keeps the fastest that meets opts->tol in the plan, and returns
+ * memory, 4 as 0 with 3 workgroups per CU (more registers: the basis of systems up to
+ * 1024 unknowns then stays in registers), all GMRES at restart length 16 / 24 / 32 /
+ * 64, and 5 per-set BiCGStab on the parity-reduced system (the default method; no
+ * restart length: 32 is reported) -- keeps the fastest that meets opts->tol in the plan, and returns
  * it (choice[0] = schedule 0..5, choice[1] = restart; *best_ms = its time per
  * batch).
  * d_final receives the batch's results.  Later esl_plan_solve / esl_plan_solve_many

@@ -424,8 +424,9 @@ class solve_plan:
         return res, its, meth
 
     def set_schedule(self, schedule, restart=32):
-        """Pins a schedule (0 per-set LDS, 1 per-set global, 2 device-wide, 3 per-set LDS with
-        the basis in global memory; -1 forgets)."""
+        """Pins a schedule (GMRES: 0 per-set LDS, 1 per-set global, 2 device-wide, 3 per-set LDS with
+        the basis in global memory, 4 as 0 with 3 workgroups per CU; 5 the parity-reduced solver,
+        which is the default; -1 forgets)."""
         check(lib().esl_plan_set_schedule(self.handle, schedule, restart))
 
     def autotune(self, n_sets, d_rates, d_final, **opts):

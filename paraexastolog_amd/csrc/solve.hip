@@ -1384,6 +1384,8 @@ __global__ __launch_bounds__(pblock) void k_gmres_set(sys_t S, nbr_t G, int n_se
 	}
 }
 
+#include "reduced.hip.hpp"
+
 // ============================================================================
 // LDS-resident variant of k_gmres_set for systems of up to 2048 unknowns per
 // set (the common case: one terminal SCC of ~1000 states, many rate sets).
@@ -2187,19 +2189,11 @@ __global__ __launch_bounds__(pblock) __attribute__((amdgpu_waves_per_eu(4))) voi
 	gmres_lds_body<float, 4, MR>(S, G, n_seg, rhs, zio, sc, m, tol, max_iters, out, lp, inner_rtol);
 }
 
-// The same kernel with 170 or 256 registers (3 or 2 workgroups per CU): the
-// basis of restart 24 (100 floats per thread) then stays in registers, and a
-// batch of more sets than slots refills the slots that fast sets free.
+// The same kernel with 170 registers (3 workgroups per CU): the basis of restart
+// 24 (100 floats per thread) then stays in registers, and a batch of more sets
+// than slots refills the slots that fast sets free.
 template <int MR>
 __global__ __launch_bounds__(pblock) __attribute__((amdgpu_waves_per_eu(3))) void k_gmres_priv_o3(
-	sys_t S, nbr_t G, int n_seg, const double* __restrict__ rhs, double* __restrict__ zio, pgm_scratch_t sc, int m,
-	double tol, int max_iters, pgm_out_t out, lds_plan_t lp, double inner_rtol)
-{
-	gmres_lds_body<float, 4, MR>(S, G, n_seg, rhs, zio, sc, m, tol, max_iters, out, lp, inner_rtol);
-}
-
-template <int MR>
-__global__ __launch_bounds__(pblock) __attribute__((amdgpu_waves_per_eu(2))) void k_gmres_priv_o2(
 	sys_t S, nbr_t G, int n_seg, const double* __restrict__ rhs, double* __restrict__ zio, pgm_scratch_t sc, int m,
 	double tol, int max_iters, pgm_out_t out, lds_plan_t lp, double inner_rtol)
 {
@@ -3370,6 +3364,11 @@ struct nbr_store_t
 	mutable dbuf<int32_t> wptr, wmid, wnu;
 	mutable dbuf<uint8_t> wnr;
 	mutable bool wready = false;
+	// the same lists in parity-class order (reduced.hip.hpp)
+	dbuf<int32_t> rptr, rrow;
+	dbuf<uint4> rrec;
+	int64_t nE = 0, nR = 0, rgroups = 0;
+	rb_t rview() const { return rb_t{ (int)nE, (int)nR, rptr.get(), rrow.get(), rrec.get() }; }
 	nbr_t view() const
 	{
 		return nbr_t{ ptr.get(), mid.get(), nu.get(), nr.get(), lvl.get(), L,
@@ -3400,25 +3399,57 @@ void build_wnbr(ctx_t& c, int64_t nU, const nbr_store_t& st)
 	st.wready = true;
 }
 
+// coupling lists in parity-class order from the lists by unknown; opos: exclusive
+// scan of the odd-parity flags, n_odd their total
+void build_rb(ctx_t& c, const sys_t& S, nbr_store_t& st, const int32_t* opos, int64_t n_odd, int32_t* cnt)
+{
+	const int64_t nU = S.nU;
+	const int nb = ceil_div(nU, sblock);
+	const int elim = n_odd > nU - n_odd ? 1 : 0; // the larger class is eliminated
+	st.nE = elim ? n_odd : nU - n_odd;
+	st.nR = nU - st.nE;
+	dbuf<int32_t> inv;
+	inv.ensure(nU);
+	st.rptr.ensure(nU + 1);
+	st.rrow.ensure(nU);
+	k_rb_place<<<nb, sblock, 0, c.stream>>>(nU, (int)st.nE, elim, S.ulist, opos, st.ptr.get(), st.rrow.get(), inv.get(),
+											cnt);
+	exclusive_scan_i32(c, cnt, st.rptr.get(), nU);
+	int32_t groups = 0;
+	ESL_HIP(hipMemcpyAsync(&groups, st.rptr.get() + nU, sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
+	ESL_HIP(hipStreamSynchronize(c.stream));
+	st.rgroups = groups;
+	st.rrec.ensure(std::max(groups, 1));
+	k_rb_fill<<<nb, sblock, 0, c.stream>>>(nU, st.rrow.get(), inv.get(), st.ptr.get(), st.nu.get(), st.nr.get(),
+										   st.rptr.get(), st.rrec.get());
+	ESL_HIP(hipGetLastError());
+	ESL_HIP(hipStreamSynchronize(c.stream));
+}
+
 void build_nbr(ctx_t& c, const sys_t& S, nbr_store_t& st)
 {
 	const int64_t nU = S.nU;
 	const int nb = ceil_div(nU, sblock);
-	dbuf<int32_t> cnt, lvl_key;
+	dbuf<int32_t> cnt, lvl_key, opos;
 	cnt.ensure(nU);
 	lvl_key.ensure(nU);
+	opos.ensure(nU + 1);
 	st.ptr.ensure(nU + 1);
 	st.mid.ensure(nU);
 	st.lvl.ensure(nU);
+	k_rb_parity<<<nb, sblock, 0, c.stream>>>(nU, S.ulist, cnt.get());
+	exclusive_scan_i32(c, cnt.get(), opos.get(), nU);
 	k_nbr_count<<<nb, sblock, 0, c.stream>>>(S, cnt.get());
 	exclusive_scan_i32(c, cnt.get(), st.ptr.get(), nU);
-	int32_t nnz = 0;
+	int32_t nnz = 0, n_odd = 0;
 	ESL_HIP(hipMemcpyAsync(&nnz, st.ptr.get() + nU, sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
+	ESL_HIP(hipMemcpyAsync(&n_odd, opos.get() + nU, sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
 	ESL_HIP(hipStreamSynchronize(c.stream));
 	st.nnz = nnz;
 	st.nu.ensure(std::max(nnz, 1));
 	st.nr.ensure(std::max(nnz, 1));
 	k_nbr_fill<<<nb, sblock, 0, c.stream>>>(S, st.ptr.get(), st.nu.get(), st.nr.get(), st.mid.get(), lvl_key.get());
+	build_rb(c, S, st, opos.get(), n_odd, cnt.get());
 	// unknowns grouped by popcount level (counting sort on the host: N + 1 buckets)
 	std::vector<int32_t> h_key;
 	read_host(c, h_key, lvl_key.get(), (size_t)nU);
@@ -3782,6 +3813,7 @@ struct krylov_result_t
 	int iters = 0, cycles = 0;
 	int sets_iterated = 0; // sets whose initial iterate missed the tolerance
 	int fp64_fallback = 0; // sets finished in FP64 after their FP32 cycles stalled
+	int finished = 0;	   // sets that a second launch finished (their vectors changed after the first)
 	int missed = 0;		   // sets above the tolerance
 	int64_t iters_sum = 0; // iterations summed over the sets
 	int exact = 0;		   // sets solved by the exact dense LU
@@ -3791,6 +3823,7 @@ struct krylov_result_t
 struct pss_view_t
 {
 	double *r = nullptr, *udiag = nullptr, *res = nullptr, *t = nullptr;
+	double* xk = nullptr; // reduced solver: the iterate before the last cycle
 	int32_t *its = nullptr, *cyc = nullptr, *stl = nullptr;
 	uint64_t* tspan = nullptr; // [B][2] start / end wall clock of each set's workgroup
 	float* Vf = nullptr;  // FP32 basis (precision 1)
@@ -3891,12 +3924,13 @@ krylov_result_t collect_sets(ctx_t& c, const pss_view_t& sc, int B, double tol, 
 // scratch of the per-set GMRES kernel, grown on demand and reused
 struct per_set_scratch_t
 {
-	dbuf<double> r, udiag, res, t;
+	dbuf<double> r, udiag, res, t, xk;
 	dbuf<int32_t> its, cyc, stl;
 	dbuf<uint64_t> tspan;
 	dbuf<float> Vf;
 	dbuf<double> Vd;
-	void reserve(int B, int64_t nU, int m, int precision)
+	// reduced: for the reduced solver, which keeps no basis
+	void reserve(int B, int64_t nU, int m, int precision, bool reduced)
 	{
 		nU = std::max<int64_t>(nU, 1);
 		r.ensure((size_t)B * nU);
@@ -3907,23 +3941,45 @@ struct per_set_scratch_t
 		stl.ensure(B);
 		tspan.ensure((size_t)2 * B);
 		t.ensure((size_t)B * nU);
-		if (precision == 1)
+		if (reduced)
+			xk.ensure((size_t)B * nU);
+		else if (precision == 1)
 			Vf.ensure((size_t)B * (m + 1) * nU);
 		else
 			Vd.ensure((size_t)B * (m + 1) * nU);
 	}
 	pss_view_t view() const
 	{
-		return pss_view_t{ r.get(), udiag.get(), res.get(), t.get(), its.get(), cyc.get(), stl.get(),
-						   tspan.get(), Vf.get(), Vd.get() };
+		return pss_view_t{ r.get(),	  udiag.get(), res.get(),	t.get(),  xk.get(), its.get(),
+						   cyc.get(), stl.get(),   tspan.get(), Vf.get(), Vd.get() };
 	}
 };
 
-// one launch: GMRES of every set, one workgroup per set (no host synchronisation)
-// occ: workgroups per CU the private-basis kernel of small systems aims for (4, 3 or 2)
+// schedules of a plan (esl_plan_autotune): how a run solves its systems
+enum : int
+{
+	path_lds = 0,	  // per set, GMRES, system in LDS (private per-thread FP32 basis where it fits)
+	path_global = 1,  // per set, GMRES from global memory
+	path_wide = 2,	  // device-wide GMRES
+	path_lds_mem = 3, // as 0 with the basis in global memory
+	path_lds_o3 = 4,  // as 0 with 3 workgroups per CU
+	path_reduced = 5  // per set, BiCGStab on the parity-reduced system
+};
+
+// The reduced solver's kernel for this system and batch, or null when another
+// path or a preconditioner of GMRES is asked for by name, or none fits.
+const bicg_variant_t* reduced_variant(const ctx_t& c, const sys_t& S, const nbr_store_t& nb, const esl_solve_opts& o,
+									  int path)
+{
+	if (path != path_reduced || o.preconditioner != 0)
+		return nullptr;
+	return rb_variant(nb.nE, nb.nR, nb.rgroups, o.precision, S.B, (size_t)std::min(c.lds_per_block, 160 * 1024));
+}
+
+// one launch: the solve of every set, one workgroup per set (no host synchronisation)
+// path: the schedule; path_reduced falls back to path_lds where no reduced variant fits
 void launch_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, int n_seg, const double* rhs, double* z,
-					const esl_solve_opts& o, const pss_view_t& sc, bool allow_lds = true, bool allow_reg = true,
-					int occ = 4)
+					const esl_solve_opts& o, const pss_view_t& sc, int path)
 {
 	const int B = S.B;
 	const int m = std::min(std::max(o.restart > 0 ? o.restart : 32, 2), pm_max);
@@ -3932,7 +3988,21 @@ void launch_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, int n_seg, 
 	const nbr_t G = nb.view();
 	pgm_out_t po{ sc.its, sc.cyc, sc.res, sc.stl, sc.tspan };
 	const double by = gmres_set_bytes(S, nb.nnz);
-	if (allow_lds && ilu && nb.packed)
+	if (const bicg_variant_t* v = reduced_variant(c, S, nb, o, path))
+	{
+		const size_t lds = rb_lds_bytes(S.nU, nb.rgroups, o.precision, v->lrec);
+		const bicg_set_fn fn = v->fn[o.precision == 1];
+		if (lds > 48 * 1024)
+			ESL_HIP(hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+		const rb_scratch_t sp{ sc.r, sc.udiag, sc.t, sc.xk };
+		timed_launch(c, o.precision == 1 ? "k_bicg_set<float>" : "k_bicg_set<double>", by, [&] {
+			fn<<<B, v->blk, lds, c.stream>>>(S, nb.rview(), nseg1, rhs, z, sp, o.tol, o.max_iters, po, o.inner_rtol);
+		});
+		ESL_HIP(hipGetLastError());
+		return;
+	}
+	const bool allow_reg = path != path_lds_mem;
+	if (path != path_global && ilu && nb.packed)
 	{
 		// LDS-resident kernel when its structure, pivots and vector fit
 		const int psize = o.precision == 1 ? 4 : 8;
@@ -3942,14 +4012,13 @@ void launch_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, int n_seg, 
 			const bool small = S.nU <= 4 * pblock;
 			if (lp.bytes > 48 * 1024)
 			{
-				const void* fns[16] = { (const void*)k_gmres_lds<float, 4>,  (const void*)k_gmres_lds<float, 8>,
+				const void* fns[13] = { (const void*)k_gmres_lds<float, 4>,  (const void*)k_gmres_lds<float, 8>,
 										(const void*)k_gmres_lds<double, 4>, (const void*)k_gmres_lds<double, 8>,
 										(const void*)k_gmres_priv<32>,		 (const void*)k_gmres_priv<24>,
 										(const void*)k_gmres_priv<16>,		 (const void*)k_gmres_priv8<32>,
 										(const void*)k_gmres_priv8<24>,		 (const void*)k_gmres_priv8<16>,
 										(const void*)k_gmres_priv_o3<32>,	 (const void*)k_gmres_priv_o3<24>,
-										(const void*)k_gmres_priv_o3<16>,	 (const void*)k_gmres_priv_o2<32>,
-										(const void*)k_gmres_priv_o2<24>,	 (const void*)k_gmres_priv_o2<16> };
+										(const void*)k_gmres_priv_o3<16> };
 				for (const void* f : fns)
 					ESL_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lp.bytes));
 			}
@@ -3985,16 +4054,12 @@ void launch_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, int n_seg, 
 			KERNEL<32><<<B, pblock, lp.bytes, c.stream>>>(S, G, nseg1, rhs, z, sp, m, o.tol, o.max_iters, po, lp, \
 														  o.inner_rtol);                                      \
 	} while (0)
-				timed_launch(c, occ == 3 ? "k_gmres_priv_o3<float>" : occ == 2 ? "k_gmres_priv_o2<float>"
-																		: "k_gmres_priv<float>",
-							 by, [&] {
-								 if (occ == 3)
-									 ESL_PRIV_LAUNCH(k_gmres_priv_o3);
-								 else if (occ == 2)
-									 ESL_PRIV_LAUNCH(k_gmres_priv_o2);
-								 else
-									 ESL_PRIV_LAUNCH(k_gmres_priv);
-							 });
+				timed_launch(c, path == path_lds_o3 ? "k_gmres_priv_o3<float>" : "k_gmres_priv<float>", by, [&] {
+					if (path == path_lds_o3)
+						ESL_PRIV_LAUNCH(k_gmres_priv_o3);
+					else
+						ESL_PRIV_LAUNCH(k_gmres_priv);
+				});
 #undef ESL_PRIV_LAUNCH
 			}
 			else if (o.precision == 1)
@@ -4052,16 +4117,16 @@ void launch_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, int n_seg, 
 	ESL_HIP(hipGetLastError());
 }
 
-// Reads the per-set results of a launch_per_set.  In mixed precision, sets that
-// missed the tolerance (their FP32 cycles stalled) are finished by the FP64
-// kernel from their current iterate; sets that already converged leave it at
-// their first residual check.
+// Reads the per-set results of a launch_per_set.  Sets that missed the tolerance
+// in mixed precision (their FP32 cycles stalled) or in the reduced solver are
+// finished by FP64 GMRES with ILU(0) from their current iterate; sets that already
+// converged leave it at their first residual check.
 // fp64_view() gives the scratch with an FP64 basis (it may grow it).  Nothing
 // is thrown here: sets still above the tolerance are counted in kr.missed and
 // marked in `out` (method -1) for the caller's fallback.
 template <typename F>
 krylov_result_t finish_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, int n_seg, const double* rhs,
-							   double* z, esl_solve_opts o, const pss_view_t& sc, F&& fp64_view,
+							   double* z, esl_solve_opts o, const pss_view_t& sc, bool reduced, F&& fp64_view,
 							   set_results_t* out = nullptr, bool staged = false)
 {
 	ESL_HIP(hipStreamSynchronize(c.stream));
@@ -4069,23 +4134,27 @@ krylov_result_t finish_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, 
 	set_results_t sr;
 	sr.method.assign(B, 0);
 	krylov_result_t kr = collect_sets(c, sc, B, o.tol, false, &sr.res, &sr.its, &sr.tspan, staged);
-	if (o.precision == 1 && kr.missed > 0)
+	if ((o.precision == 1 || reduced) && kr.missed > 0)
 	{
+		const bool mixed = o.precision == 1;
 		o.precision = 0;
+		if (reduced)
+			o.preconditioner = 2;
 		const pss_view_t sd = fp64_view();
-		launch_per_set(c, S, nb, n_seg, rhs, z, o, sd);
+		launch_per_set(c, S, nb, n_seg, rhs, z, o, sd, path_lds);
 		ESL_HIP(hipStreamSynchronize(c.stream));
 		std::vector<double> res2;
 		std::vector<int32_t> its2;
 		const krylov_result_t k2 = collect_sets(c, sd, B, o.tol, false, &res2, &its2);
 		for (int b = 0; b < B; ++b)
 		{
-			if (!(sr.res[b] <= o.tol))
+			if (!(sr.res[b] <= o.tol) && mixed)
 				sr.method[b] = 1;
 			sr.res[b] = res2[b];
 			sr.its[b] += its2[b];
 		}
-		kr.fp64_fallback = kr.missed;
+		kr.finished = kr.missed;
+		kr.fp64_fallback = mixed ? kr.missed : 0;
 		kr.missed = k2.missed;
 		kr.resid = k2.resid;
 		kr.iters += k2.iters;
@@ -4146,13 +4215,10 @@ struct plan_t
 	struct tune_t
 	{
 		bool set = false;
-		int path = 0; // 0 per-set (LDS-resident, private per-thread basis when it fits), 1 per-set from global
-					  // memory, 2 device-wide, 3 per-set LDS-resident with the basis in global memory
+		int path = 0; // path_lds ... path_reduced
 		int m = 32;
 	} tune;
-	bool allow_lds = true; // the schedule of the run being enqueued
-	bool allow_reg = true;
-	int occ = 4;		   // workgroups per CU of the private-basis kernel (schedules 4 and 5: 3 and 2)
+	int path = 0; // the schedule of the run being enqueued
 	set_results_t results; // per-set outcome of the last run (esl_plan_set_results)
 	double ms[3] = { 0, 0, 0 };
 	// captured numeric sequence and the arguments it was captured with
@@ -4166,14 +4232,12 @@ struct plan_t
 		double tol = 0, inner_rtol = 0;
 		int max_iters = 0;
 		int64_t epoch = 0;
-		bool allow_lds = true, allow_reg = true;
-		int occ = 4;
+		int path = 0;
 		bool operator==(const gkey_t& o) const
 		{
 			return B == o.B && rates == o.rates && fin == o.fin && warm == o.warm && precision == o.precision &&
 				   preconditioner == o.preconditioner && m == o.m && tol == o.tol && inner_rtol == o.inner_rtol &&
-				   max_iters == o.max_iters && epoch == o.epoch && allow_lds == o.allow_lds &&
-				   allow_reg == o.allow_reg && occ == o.occ;
+				   max_iters == o.max_iters && epoch == o.epoch && path == o.path;
 		}
 	};
 	gkey_t gkey{};
@@ -4241,14 +4305,16 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 			build_nbr(c, S, local);
 		const nbr_store_t& nb = prebuilt ? *prebuilt : local;
 		per_set_scratch_t sc;
-		sc.reserve(B, nU, m, opts.precision);
 		esl_solve_opts o = opts;
 		o.tol = tol;
 		o.max_iters = max_iters;
 		o.restart = m;
-		launch_per_set(c, S, nb, n_seg, rhs_p, z_p, o, sc.view());
-		kr = finish_per_set(c, S, nb, n_seg, rhs_p, z_p, o, sc.view(), [&] {
-			sc.reserve(B, nU, m, 0);
+		const int path = opts.restart <= 0 ? path_reduced : path_lds;
+		const bool reduced = reduced_variant(c, S, nb, o, path) != nullptr;
+		sc.reserve(B, nU, m, opts.precision, reduced);
+		launch_per_set(c, S, nb, n_seg, rhs_p, z_p, o, sc.view(), path);
+		kr = finish_per_set(c, S, nb, n_seg, rhs_p, z_p, o, sc.view(), reduced, [&] {
+			sc.reserve(B, nU, m, 0, false);
 			return sc.view();
 		});
 		if (kr.missed && throw_on_miss)
@@ -4731,33 +4797,50 @@ void plan_enqueue(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_f
 	}
 	plan_enqueue_setup(c, P, B, d_rates, o);
 	if (P.nU)
-		launch_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, o, P.rb.ps, P.allow_lds,
-					   P.allow_reg, P.occ);
+		launch_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, o, P.rb.ps, P.path);
 	if (fork)
 		ESL_HIP(hipStreamWaitEvent(c.stream, c.fill_ev[1], 0));
 	plan_enqueue_post(c, P, B, d_rates, d_final, !fork);
 }
 
-void plan_reserve_(plan_t& P, int B, int m, int precision);
+void plan_reserve_(plan_t& P, int B, int m, int precision, bool reduced);
+
+// The schedule of a run: the tuned one when the caller asks for restart 0, else
+// the reduced solver -- unless a restart length asks for GMRES.
+int run_path(const plan_t& P, const esl_solve_opts& o)
+{
+	if (o.restart == 0 && P.tune.set)
+		return P.tune.path;
+	return o.restart <= 0 ? path_reduced : path_lds;
+}
+
+// whether a per-set run of the plan takes the reduced solver
+bool plan_reduced(const ctx_t& c, const plan_t& P, int B, const esl_solve_opts& o)
+{
+	sys_t S{};
+	S.nU = P.nU;
+	S.B = B;
+	return P.nU > 0 && reduced_variant(c, S, P.nbr, o, P.path) != nullptr;
+}
 
 // grows the per-run buffers; a captured graph holds their addresses, so any
 // reallocation bumps the plan's epoch (part of every graph key)
-void plan_reserve(plan_t& P, int B, int m, int precision)
+void plan_reserve(plan_t& P, int B, int m, int precision, bool reduced)
 {
 	auto ptrs = [&] {
 		return std::vector<const void*>{ P.p0.get(),	 P.p1.get(),	  P.anchor.get(), P.invd.get(),
 										 P.rhs.get(),	 P.z.get(),		  P.y.get(),	  P.segsum.get(),
 										 P.scr.r.get(),	  P.scr.udiag.get(), P.scr.res.get(),
 										 P.scr.t.get(), P.scr.its.get(), P.scr.cyc.get(), P.scr.stl.get(),
-										 P.scr.tspan.get(), P.scr.Vf.get(), P.scr.Vd.get() };
+										 P.scr.tspan.get(), P.scr.xk.get(), P.scr.Vf.get(), P.scr.Vd.get() };
 	};
 	const auto before = ptrs();
-	plan_reserve_(P, B, m, precision);
+	plan_reserve_(P, B, m, precision, reduced);
 	if (ptrs() != before)
 		++P.epoch;
 }
 
-void plan_reserve_(plan_t& P, int B, int m, int precision)
+void plan_reserve_(plan_t& P, int B, int m, int precision, bool reduced)
 {
 	const int64_t nU = std::max<int64_t>(P.nU, 1), nUt = std::max<int64_t>(P.nUt, 1);
 	P.p0.ensure((size_t)B * nUt);
@@ -4768,7 +4851,7 @@ void plan_reserve_(plan_t& P, int B, int m, int precision)
 	P.z.ensure((size_t)B * nU);
 	P.y.ensure((size_t)B * std::max(P.Tr, 1));
 	P.segsum.ensure((size_t)B * std::max(P.n_seg, 1));
-	P.scr.reserve(B, nU, m, precision);
+	P.scr.reserve(B, nU, m, precision, reduced);
 	P.use_own_bufs();
 }
 
@@ -4968,9 +5051,7 @@ void plan_run(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_final
 	const bool tuned = o.restart == 0 && P.tune.set;
 	if (tuned)
 		o.restart = P.tune.m;
-	P.allow_lds = !(tuned && P.tune.path == 1);
-	P.allow_reg = !(tuned && P.tune.path == 3);
-	P.occ = tuned && P.tune.path == 4 ? 3 : tuned && P.tune.path == 5 ? 2 : 4;
+	P.path = run_path(P, o_in);
 	const int m = std::min(std::max(o.restart > 0 ? o.restart : 32, 2), pm_max);
 	const bool per_set = P.nU == 0 || (tuned ? P.tune.path != 2 : P.nU <= per_set_max_unknowns(B));
 	rep.terminals_reached = P.Tr;
@@ -4979,13 +5060,14 @@ void plan_run(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_final
 	krylov_result_t kr;
 	if (per_set)
 	{
-		plan_reserve(P, B, m, o.precision);
+		const bool reduced = plan_reduced(c, P, B, o);
+		plan_reserve(P, B, m, o.precision, reduced);
 		const bool use_graph = o.graph != 0;
 		if (use_graph)
 		{
 			const plan_t::gkey_t key{ B,		   d_rates,	  d_final,	   o.warm_pi,  o.precision,
 									  o.preconditioner, m,		  o.tol,	   o.inner_rtol, o.max_iters,
-									  P.epoch,		   P.allow_lds, P.allow_reg, P.occ };
+									  P.epoch,		   P.path };
 			if (!P.gexec || !(P.gkey == key) || P.gprof != c.prof.on)
 			{
 				P.drop_graph();
@@ -5032,13 +5114,13 @@ void plan_run(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_final
 			esl_solve_opts of = o;
 			of.restart = m;
 			set_results_t sr;
-			kr = finish_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, of, P.rb.ps, [&] {
-				P.scr.reserve(B, P.nU, m, 0);
+			kr = finish_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, of, P.rb.ps, reduced, [&] {
+				P.scr.reserve(B, P.nU, m, 0, false);
 				P.use_own_bufs();
 				return P.rb.ps;
 			}, &sr, staged);
-			// the final vectors are rebuilt when FP64 iterates replaced FP32 ones
-			plan_finish_sets(c, P, B, d_rates, d_final, of, kr, std::move(sr), kr.fp64_fallback > 0, true);
+			// the final vectors are rebuilt when a second launch finished sets
+			plan_finish_sets(c, P, B, d_rates, d_final, of, kr, std::move(sr), kr.finished > 0, true);
 		}
 		else
 			P.results = trivial_results(B);
@@ -5046,7 +5128,7 @@ void plan_run(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_final
 	else
 	{
 		// one large system: device-wide GMRES (host-driven restarts)
-		plan_reserve(P, B, 2, 0);
+		plan_reserve(P, B, 2, 0, true);
 		plan_enqueue_setup(c, P, B, d_rates, o);
 		set_results_t sr;
 		kr = krylov_solve(c, P.sys(B, d_rates), P.n_seg, P.rb.rhs, P.rb.z, o, &P.nbr, true, false, &sr.res);
@@ -5164,6 +5246,7 @@ plan_t::run_bufs_t carve_run_bufs(const plan_t& P, int B, int m, carve_t& cv)
 	rb.ps.tspan = cv.take<uint64_t>((size_t)2 * B);
 	rb.ps.Vd = cv.take<double>((size_t)B * (m + 1) * nU);
 	rb.ps.Vf = reinterpret_cast<float*>(rb.ps.Vd);
+	rb.ps.xk = rb.ps.Vd; // the reduced solver keeps no basis
 	return rb;
 }
 
@@ -5191,9 +5274,6 @@ void plan_solve_noalloc(ctx_t& c, void* p, int B, const double* d_rates, double*
 	const bool tuned = o.restart == 0 && P.tune.set;
 	if (tuned)
 		o.restart = P.tune.m;
-	const bool allow_lds = !(tuned && P.tune.path == 1);
-	const bool allow_reg = !(tuned && P.tune.path == 3);
-	const int occ = tuned && P.tune.path == 4 ? 3 : tuned && P.tune.path == 5 ? 2 : 4;
 	const int m = std::min(std::max(o.restart > 0 ? o.restart : 32, 2), pm_max);
 	o.restart = m;
 	const bool per_set = P.nU == 0 || (tuned ? P.tune.path != 2 : P.nU <= per_set_max_unknowns(B));
@@ -5210,9 +5290,7 @@ void plan_solve_noalloc(ctx_t& c, void* p, int B, const double* d_rates, double*
 	carve_t cv{ base, base };
 	prof_pause_t pause(c);
 	P.rb = carve_run_bufs(P, B, m, cv);
-	P.allow_lds = allow_lds;
-	P.allow_reg = allow_reg;
-	P.occ = occ;
+	P.path = run_path(P, o_in);
 	rep.terminals_reached = P.Tr;
 	rep.unknowns = P.nU;
 	rep.reachable = -1;
@@ -5225,10 +5303,10 @@ void plan_solve_noalloc(ctx_t& c, void* p, int B, const double* d_rates, double*
 		{
 			const pss_view_t ps = P.rb.ps;
 			set_results_t sr;
-			kr = finish_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, o, ps, [&] { return ps; },
-								&sr);
+			kr = finish_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, o, ps,
+								plan_reduced(c, P, B, o), [&] { return ps; }, &sr);
 			// no exact fallback here (its dense matrix would need an allocation)
-			plan_finish_sets(c, P, B, d_rates, d_final, o, kr, std::move(sr), kr.fp64_fallback > 0, false);
+			plan_finish_sets(c, P, B, d_rates, d_final, o, kr, std::move(sr), kr.finished > 0, false);
 		}
 		else
 			P.results = trivial_results(B);
@@ -5261,7 +5339,7 @@ struct multi_graph_t
 	std::vector<const double*> rates;
 	std::vector<double*> fin;
 	std::vector<int64_t> epochs;
-	std::vector<int> ms, lds;
+	std::vector<int> ms, paths;
 	int precision = 0, preconditioner = 0, max_iters = 0;
 	double tol = 0, inner_rtol = 0;
 	bool prof = false;
@@ -5271,7 +5349,7 @@ struct multi_graph_t
 	bool same(const multi_graph_t& o) const
 	{
 		return plans == o.plans && B == o.B && rates == o.rates && fin == o.fin && epochs == o.epochs &&
-			   ms == o.ms && lds == o.lds && precision == o.precision && preconditioner == o.preconditioner &&
+			   ms == o.ms && paths == o.paths && precision == o.precision && preconditioner == o.preconditioner &&
 			   max_iters == o.max_iters && tol == o.tol &&
 			   inner_rtol == o.inner_rtol && prof == o.prof;
 	}
@@ -5364,9 +5442,7 @@ void plan_solve_many(ctx_t& c, int np, void* const* plans, const int* B, const d
 		plan_t& P = *static_cast<plan_t*>(plans[i]);
 		reps[i] = esl_solve_report{};
 		const bool tuned = o_in.restart == 0 && P.tune.set;
-		P.allow_lds = !(tuned && P.tune.path == 1);
-		P.allow_reg = !(tuned && P.tune.path == 3);
-		P.occ = tuned && P.tune.path == 4 ? 3 : tuned && P.tune.path == 5 ? 2 : 4;
+		P.path = run_path(P, o_in);
 		po[i].restart = std::min(std::max(tuned ? P.tune.m : (o.restart > 0 ? o.restart : 32), 2), pm_max);
 		if (P.nU == 0 || (tuned ? P.tune.path != 2 : P.nU <= per_set_max_unknowns(B[i])))
 			conc.push_back(i);
@@ -5421,7 +5497,8 @@ void many_per_set(ctx_t& c, const std::vector<int>& conc, void* const* plans, co
 	if (conc.empty())
 		return;
 	for (int i : conc)
-		plan_reserve(*static_cast<plan_t*>(plans[i]), B[i], po[i].restart, o.precision);
+		plan_reserve(*static_cast<plan_t*>(plans[i]), B[i], po[i].restart, o.precision,
+					 plan_reduced(c, *static_cast<plan_t*>(plans[i]), B[i], po[i]));
 	ensure_aux(c, (int)conc.size());
 	timer_t tm_(c);
 	auto enqueue_all = [&] {
@@ -5457,9 +5534,7 @@ void many_per_set(ctx_t& c, const std::vector<int>& conc, void* const* plans, co
 			key.fin.push_back(d_final[i]);
 			key.epochs.push_back(static_cast<plan_t*>(plans[i])->epoch);
 			key.ms.push_back(po[i].restart);
-			key.lds.push_back((static_cast<plan_t*>(plans[i])->allow_lds ? 1 : 0) +
-							  (static_cast<plan_t*>(plans[i])->allow_reg ? 2 : 0) +
-							  4 * static_cast<plan_t*>(plans[i])->occ);
+			key.paths.push_back(static_cast<plan_t*>(plans[i])->path);
 		}
 		key.precision = o.precision;
 		key.preconditioner = o.preconditioner;
@@ -5530,12 +5605,13 @@ void many_per_set(ctx_t& c, const std::vector<int>& conc, void* const* plans, co
 			const esl_solve_opts& of = po[i];
 			set_results_t sr;
 			krylov_result_t kr =
-				finish_per_set(c, P.sys(B[i], d_rates[i]), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, of, P.rb.ps, [&] {
-					P.scr.reserve(B[i], P.nU, of.restart, 0);
+				finish_per_set(c, P.sys(B[i], d_rates[i]), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, of, P.rb.ps,
+							   plan_reduced(c, P, B[i], of), [&] {
+					P.scr.reserve(B[i], P.nU, of.restart, 0, false);
 					P.use_own_bufs();
 					return P.rb.ps;
 				}, &sr);
-			plan_finish_sets(c, P, B[i], d_rates[i], d_final[i], of, kr, std::move(sr), kr.fp64_fallback > 0, true);
+			plan_finish_sets(c, P, B[i], d_rates[i], d_final[i], of, kr, std::move(sr), kr.finished > 0, true);
 			rep.exact_solves = kr.exact;
 			rep.residual = kr.resid;
 			rep.iterations = kr.iters;
@@ -5608,13 +5684,12 @@ void plan_autotune(ctx_t& c, void* p, int B, const double* d_rates, double* d_fi
 				cands.push_back({ 1, m });
 			if (ilu && o.precision == 1 && P.nU <= lds_max_unknowns && m <= 32) // otherwise path 3 is path 0
 				cands.push_back({ 3, m });
-			if (ilu && o.precision == 1 && P.nU <= 4 * pblock && m <= 32) // the private-basis kernel at 3 / 2 WG per CU
-			{
+			if (ilu && o.precision == 1 && P.nU <= 4 * pblock && m <= 32) // the private-basis kernel at 3 WG per CU
 				cands.push_back({ 4, m });
-				cands.push_back({ 5, m });
-			}
 			cands.push_back({ 2, m });
 		}
+	if (P.nU > 0 && o.preconditioner == 0)
+		cands.push_back({ path_reduced, 32 }); // keeps no basis: the restart length does not matter
 	const plan_t::tune_t saved = P.tune;
 	plan_t::tune_t best_t{};
 	double best = 1e300;
