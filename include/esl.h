@@ -149,14 +149,16 @@ esl_status esl_graph_export(esl_ctx* ctx, const esl_graph* g, int32_t* reordered
 
 typedef struct
 {
-	int precision;		 /* 0 = FP64 Krylov solves; 1 = FP32 inner solves + FP64 residual refinement */
+	int precision;		 /* 0 = FP64 Krylov solves; 1 = FP32 inner solves + FP64 residual refinement (where
+						  * GMRES runs; the default method holds its vectors in FP64 either way) */
 	double tol;			 /* relative residual target of every linear solve (default 1e-13) */
 	int max_iters;		 /* Krylov iterations per solve before ESL_E_NUMERIC (default 20000) */
 	int restart;		 /* > 0 asks for restarted GMRES with this restart length: at most 64 for the
 						  * per-set solvers, 128 for the device-wide solver; 0 (default): a plan's
-						  * autotuned schedule, else the default method (per set, BiCGStab on the
-						  * parity-reduced system; device-wide, GMRES at 32, halved while its FP64
-						  * basis would exceed half the free device memory) */
+						  * autotuned schedule, else the default method, BiCGStab on the
+						  * parity-reduced system in FP64 (per set or device-wide); GMRES with ILU(0)
+						  * finishes what stalls there, device-wide at 32, halved while its FP64
+						  * basis would exceed half the free device memory */
 	int full;			 /* 1: also build solution_term / solution_nonterm (esl_solution_export) */
 	int preconditioner;	 /* 0 = default (ILU(0) where GMRES runs), 1 = Jacobi, 2 = ILU(0) (level-scheduled);
 						  * 1 and 2 ask for GMRES */
@@ -268,8 +270,8 @@ esl_status esl_plan_gather_terminal(esl_ctx* ctx, const esl_plan* p, int n_sets,
  * memory, 2 device-wide, 3 per-set with the system in LDS and the basis in global
  * memory, 4 as 0 with 3 workgroups per CU (more registers: the basis of systems up to
  * 1024 unknowns then stays in registers), all GMRES at restart length 16 / 24 / 32 /
- * 64, and 5 per-set BiCGStab on the parity-reduced system (the default method; no
- * restart length: 32 is reported) -- keeps the fastest that meets opts->tol in the plan, and returns
+ * 64, and 5 BiCGStab on the parity-reduced system (the default method, per set or
+ * device-wide by the system's size; no restart length: 32 is reported) -- keeps the fastest that meets opts->tol in the plan, and returns
  * it (choice[0] = schedule 0..5, choice[1] = restart; *best_ms = its time per
  * batch).
  * d_final receives the batch's results.  Later esl_plan_solve / esl_plan_solve_many

@@ -15,12 +15,15 @@
 // It replaces restarted GMRES with ILU(0) as the default method of the per-set
 // solver (that one stays for sets on which this method stalls, and for callers
 // that ask for a restart length or a preconditioner).  At 1e-12 a set of N = 20
-// seed 0 (1,022 unknowns) takes 66-90 products by S against 30 by M with ILU(0),
+// seed 0 (1,022 unknowns) takes 40-90 products by S against 30 by M with ILU(0),
 // but a product costs three barriers and one reduction where a preconditioned step
 // has 22 levels and a Gram-Schmidt pass.  Bound: the latency of that chain.
+// Vectors are FP64 in both precisions: in FP32 the recurrences lose so much that
+// the same sets take 90 products on average and up to 288 instead of 62 and 158
+// (1,024 sets: 912 us against 453), and larger systems up to three times as many.
 // Measured on MI355X, GMRES with ILU(0) -> this: one set in FP64 853 -> 89 us; 250
 // sets of 2,048 unknowns in FP64 6,600 -> 385 us; 1,024 sets of 1,022 unknowns in
-// mixed precision, beside the fill of the final vectors, 2,130 -> 912 us.
+// mixed precision, beside the fill of the final vectors, 2,130 -> 453 us.
 
 // coupling lists with rows in class order: row q < nE is an eliminated unknown,
 // row nE + o a kept one; a neighbour is named by its index inside the other
@@ -34,7 +37,6 @@ struct rb_t
 	const int32_t* row = nullptr; // [nU] row -> unknown
 	const uint4* rec = nullptr;	  // neighbour | rate code << 25 | mirrored << 31
 };
-constexpr int rb_null = 63; // 2N <= 52 rate codes are in use
 constexpr uint32_t rb_index = (1u << 25) - 1; // a parity class has at most 2^25 states (N <= 26)
 __device__ __forceinline__ int rb_code(uint32_t r) { return (r >> 25) & 63; }
 
@@ -64,7 +66,7 @@ __global__ __launch_bounds__(sblock) void k_rb_place(int64_t nU, int nE, int eli
 	cnt[q] = (gptr[u + 1] - gptr[u] + 3) / 4;
 }
 
-__global__ __launch_bounds__(sblock) void k_rb_fill(int64_t nU, const int32_t* __restrict__ row,
+__global__ __launch_bounds__(sblock) void k_rb_fill(int64_t nU, int null_code, const int32_t* __restrict__ row,
 													const int32_t* __restrict__ inv, const int32_t* __restrict__ gptr,
 													const int32_t* __restrict__ gnu, const uint8_t* __restrict__ gnr,
 													const int32_t* __restrict__ rptr, uint4* __restrict__ rec)
@@ -80,7 +82,7 @@ __global__ __launch_bounds__(sblock) void k_rb_fill(int64_t nU, const int32_t* _
 		uint32_t r[4];
 		for (int k = 0; k < 4; ++k, ++e)
 		{
-			r[k] = (uint32_t)rb_null << 25;
+			r[k] = (uint32_t)null_code << 25;
 			if (e < e1)
 			{
 				const uint32_t code = gnr[e];
@@ -92,9 +94,8 @@ __global__ __launch_bounds__(sblock) void k_rb_fill(int64_t nU, const int32_t* _
 }
 
 // s + sum over the groups of a row (first group | groups << 24) of rate * y[neighbour], in list order
-template <typename Y>
 __device__ __forceinline__ double rb_sum(const uint4* __restrict__ rec, const double* __restrict__ rates, uint32_t h,
-										 const Y* __restrict__ y, double s)
+										 const double* __restrict__ y, double s)
 {
 	const int g1 = (int)(h & 0xffffff) + (int)(h >> 24);
 	for (int g = (int)(h & 0xffffff); g < g1; ++g)
@@ -102,14 +103,14 @@ __device__ __forceinline__ double rb_sum(const uint4* __restrict__ rec, const do
 		const uint4 q = rec[g];
 		const double r0 = rates[rb_code(q.x)], r1 = rates[rb_code(q.y)];
 		const double r2 = rates[rb_code(q.z)], r3 = rates[rb_code(q.w)];
-		const Y y0 = y[q.x & rb_index], y1 = y[q.y & rb_index];
-		const Y y2 = y[q.z & rb_index], y3 = y[q.w & rb_index];
+		const double y0 = y[q.x & rb_index], y1 = y[q.y & rb_index];
+		const double y2 = y[q.z & rb_index], y3 = y[q.w & rb_index];
 		// the eight loads together: one LDS round trip per group instead of one per term
 		__builtin_amdgcn_sched_barrier(0);
-		s += r0 * (double)y0;
-		s += r1 * (double)y1;
-		s += r2 * (double)y2;
-		s += r3 * (double)y3;
+		s += r0 * y0;
+		s += r1 * y1;
+		s += r2 * y2;
+		s += r3 * y3;
 	}
 	return s;
 }
@@ -216,30 +217,21 @@ struct rb_scratch_t
 	double* xk; // [B][nU] iterate before the last cycle
 };
 
-// Where a cycle that starts at the relative residual rel stops: a tenth of the
-// tolerance, in as many equal drops as cycles that each reduce by inner_rtol
-// would need (what FP32 vectors can deliver; 0: in one).  Aiming at the tolerance
-// itself leaves the last cycle's residual just below it; the extra decade costs
-// one product in twelve and keeps the error of the result where GMRES had it.
-__device__ __forceinline__ double rb_target(double rel, double tol, double inner_rtol)
-{
-	const double end = 0.1 * tol;
-	if (!(inner_rtol > 0.0) || rel * inner_rtol <= end)
-		return end;
-	const double cycles = ceil(log(rel / end) / -log(inner_rtol) - 1e-3);
-	return rel * exp(-log(rel / end) / fmax(cycles, 1.0));
-}
+// A cycle ends at a tenth of the tolerance: aiming at the tolerance itself leaves
+// the residual just below it, and the extra decade costs one product in twelve and
+// keeps the error of the result below what GMRES left.
+constexpr double rb_aim = 0.1;
 
 constexpr int rb_max_fails = 3;		 // cycles without progress before a set is left to GMRES
-constexpr int rb_cycle_products = 200; // products by S per cycle, so that rounding cannot drift for long
+constexpr int rb_cycle_products = 500; // products by S per cycle, so that rounding cannot drift for long
 
 // One workgroup of BLK threads solves one rate set; thread t owns the rows
 // t + i BLK (i < RPT) of both classes.  LREC: the coupling records are copied to
 // LDS, else they are read from global memory (shared by all sets, so from L2).
-template <typename T, int BLK, int RPT, bool LREC>
+template <int BLK, int RPT, bool LREC>
 __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int n_seg, const double* __restrict__ rhs,
 											  double* __restrict__ zio, const rb_scratch_t& sc, double tol,
-											  int max_iters, const pgm_out_t& out, double inner_rtol)
+											  int max_iters, const pgm_out_t& out)
 {
 	extern __shared__ __align__(16) unsigned char smem[];
 	__shared__ double s_part[2][rb_part];
@@ -248,9 +240,9 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 	const uint64_t t_begin = wall_clock64();
 	const int nE = G.nE, nR = G.nR, nU = nE + nR;
 	const int64_t off = (int64_t)b * nU;
-	T* s_g = (T*)smem;	 // [nR] the vector being multiplied
-	T* s_te = s_g + nR;	 // [nE] its image on the eliminated rows
-	uint4* s_rec = (uint4*)(smem + ((size_t)nU * sizeof(T) + 15) / 16 * 16);
+	double* s_g = (double*)smem;	 // [nR] the vector being multiplied
+	double* s_te = s_g + nR;	 // [nE] its image on the eliminated rows
+	uint4* s_rec = (uint4*)(smem + ((size_t)nU * sizeof(double) + 15) / 16 * 16);
 	double* __restrict__ xp = sc.x + off;
 	double* __restrict__ bp = sc.b + off;
 	double* __restrict__ rEp = sc.rE + off;
@@ -287,7 +279,7 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 			const double r = rhs[off + u];
 			bp[e] = r;
 			bb += r * r;
-			s_te[e] = anc ? (T)0 : (T)cE[i];
+			s_te[e] = anc ? 0.0 : cE[i];
 		}
 	}
 	__syncthreads();
@@ -318,7 +310,7 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 #pragma unroll
 				for (int k = 0; k < 4; ++k)
 					if (qq[k] >> 31)
-						d -= s_rates[rb_code(qq[k])] * s_rates[rb_code(qq[k]) ^ 1] * (double)s_te[qq[k] & rb_index];
+						d -= s_rates[rb_code(qq[k])] * s_rates[rb_code(qq[k]) ^ 1] * s_te[qq[k] & rb_index];
 			}
 			jR[i] = 1.0 / (d > 0.0 ? d : dR[i]);
 		}
@@ -398,7 +390,6 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 			fails = compare ? 0 : fails;
 		compare = true;
 		rel_prev = rel;
-		const double inner_target = rb_target(rel, tol, sizeof(T) == 4 ? inner_rtol : 0.0);
 		++cycles;
 		const double inv_beta = 1.0 / beta;
 #pragma unroll
@@ -406,21 +397,21 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 		{
 			const int e = tid + i * BLK;
 			if (e < nE)
-				s_te[e] = (T)(cE[i] * rEp[e] * inv_beta);
+				s_te[e] = cE[i] * rEp[e] * inv_beta;
 		}
 		__syncthreads();
-		T r[RPT], rh[RPT], p[RPT], v[RPT], x[RPT];
+		double r[RPT], rh[RPT], p[RPT], v[RPT], x[RPT];
 		double s2[2] = { 0.0, 0.0 };
 #pragma unroll
 		for (int i = 0; i < RPT; ++i)
 		{
 			const int o = tid + i * BLK;
-			r[i] = (T)(jR[i] * rb_sum(rec, s_rates, hR[i], s_te, ro[i] * inv_beta));
-			rh[i] = o < nR ? (T)rb_shadow(o, fails, (double)r[i]) : (T)0;
+			r[i] = jR[i] * rb_sum(rec, s_rates, hR[i], s_te, ro[i] * inv_beta);
+			rh[i] = o < nR ? rb_shadow(o, fails, r[i]) : 0.0;
 			p[i] = r[i];
-			x[i] = (T)0;
-			s2[0] += (double)r[i] * (double)r[i];
-			s2[1] += (double)rh[i] * (double)r[i];
+			x[i] = 0.0;
+			s2[0] += r[i] * r[i];
+			s2[1] += rh[i] * r[i];
 		}
 		rb_block_sums<BLK>(s2, s_part[1]);
 		double rho = s2[1];
@@ -437,14 +428,14 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 #pragma unroll
 			for (int i = 0; i < RPT; ++i)
 				if (tid + i * BLK < nE)
-					s_te[tid + i * BLK] = (T)(cE[i] * rb_sum(rec, s_rates, hE[i], s_g, 0.0));
+					s_te[tid + i * BLK] = cE[i] * rb_sum(rec, s_rates, hE[i], s_g, 0.0);
 			__syncthreads();
 			double s1[1] = { 0.0 };
 #pragma unroll
 			for (int i = 0; i < RPT; ++i)
 			{
-				v[i] = (T)(jR[i] * (dR[i] * (double)p[i] - rb_sum(rec, s_rates, hR[i], s_te, 0.0)));
-				s1[0] += (double)rh[i] * (double)v[i];
+				v[i] = jR[i] * (dR[i] * p[i] - rb_sum(rec, s_rates, hR[i], s_te, 0.0));
+				s1[0] += rh[i] * v[i];
 			}
 			rb_block_sums<BLK>(s1, s_part[0]);
 			++iters;
@@ -456,7 +447,7 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 #pragma unroll
 			for (int i = 0; i < RPT; ++i)
 			{
-				r[i] = (T)((double)r[i] - alpha * (double)v[i]);
+				r[i] -= alpha * v[i];
 				if (tid + i * BLK < nR)
 					s_g[tid + i * BLK] = r[i];
 			}
@@ -464,17 +455,17 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 #pragma unroll
 			for (int i = 0; i < RPT; ++i)
 				if (tid + i * BLK < nE)
-					s_te[tid + i * BLK] = (T)(cE[i] * rb_sum(rec, s_rates, hE[i], s_g, 0.0));
+					s_te[tid + i * BLK] = cE[i] * rb_sum(rec, s_rates, hE[i], s_g, 0.0);
 			__syncthreads();
-			T t[RPT];
+			double t[RPT];
 #pragma unroll
 			for (int k = 0; k < 5; ++k)
 				sums[k] = 0.0;
 #pragma unroll
 			for (int i = 0; i < RPT; ++i)
 			{
-				t[i] = (T)(jR[i] * (dR[i] * (double)r[i] - rb_sum(rec, s_rates, hR[i], s_te, 0.0)));
-				const double td = (double)t[i], sd = (double)r[i], hd = (double)rh[i];
+				t[i] = jR[i] * (dR[i] * r[i] - rb_sum(rec, s_rates, hR[i], s_te, 0.0));
+				const double td = t[i], sd = r[i], hd = rh[i];
 				sums[0] += td * sd;
 				sums[1] += td * td;
 				sums[2] += sd * sd;
@@ -490,15 +481,15 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 			const double rr2 = fmax(sums[2] - omega * (2.0 * sums[0] - omega * sums[1]), 0.0);
 			const double rho1 = sums[3] - omega * sums[4];
 			const double beta_b = (rho1 / rho) * (alpha / omega);
-			const bool stop = sqrt(rr2) * est <= inner_target || omega == 0.0 || !rb_finite(beta_b) || beta_b == 0.0 ||
+			const bool stop = sqrt(rr2) * est <= rb_aim * tol || omega == 0.0 || !rb_finite(beta_b) || beta_b == 0.0 ||
 							  iters >= max_iters;
 			rho = rho1;
 #pragma unroll
 			for (int i = 0; i < RPT; ++i)
 			{
-				x[i] = (T)((double)x[i] + alpha * (double)p[i] + omega * (double)r[i]);
-				r[i] = (T)((double)r[i] - omega * (double)t[i]);
-				p[i] = (T)((double)r[i] + beta_b * ((double)p[i] - omega * (double)v[i]));
+				x[i] += alpha * p[i] + omega * r[i];
+				r[i] -= omega * t[i];
+				p[i] = r[i] + beta_b * (p[i] - omega * v[i]);
 			}
 			if (stop)
 				break;
@@ -514,7 +505,7 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 				s_g[o] = x[i];
 				const double x0 = xp[nE + o];
 				xk[nE + o] = x0;
-				xp[nE + o] = x0 + beta * (double)x[i];
+				xp[nE + o] = x0 + beta * x[i];
 			}
 		}
 		__syncthreads();
@@ -549,19 +540,19 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 	}
 }
 
-template <typename T, int BLK, int RPT, bool LREC>
-__global__ __launch_bounds__(BLK, BLK >= 1024 || LREC ? 4 : 2) void k_bicg_set(
+template <int BLK, int RPT, bool LREC>
+__global__ __launch_bounds__(BLK, 4) void k_bicg_set(
 	sys_t S, rb_t G, int n_seg, const double* __restrict__ rhs, double* __restrict__ zio, rb_scratch_t sc, double tol,
-	int max_iters, pgm_out_t out, double inner_rtol)
+	int max_iters, pgm_out_t out)
 {
-	bicg_set_body<T, BLK, RPT, LREC>(S, G, n_seg, rhs, zio, sc, tol, max_iters, out, inner_rtol);
+	bicg_set_body<BLK, RPT, LREC>(S, G, n_seg, rhs, zio, sc, tol, max_iters, out);
 }
 
-using bicg_set_fn = void (*)(sys_t, rb_t, int, const double*, double*, rb_scratch_t, double, int, pgm_out_t, double);
+using bicg_set_fn = void (*)(sys_t, rb_t, int, const double*, double*, rb_scratch_t, double, int, pgm_out_t);
 struct bicg_variant_t
 {
-	bicg_set_fn fn[2]; // FP64, FP32 vectors
-	int blk, rows;	   // threads, rows of the larger class at most
+	bicg_set_fn fn;
+	int blk, rows; // threads, rows of the larger class at most
 	bool lrec;
 };
 
@@ -571,14 +562,14 @@ struct bicg_variant_t
 constexpr int rb_cus = 256;
 constexpr size_t rb_lds_static = 3072; // upper bound of the kernel's static LDS
 // dynamic LDS of one set: the vector being multiplied, its image, the records
-inline size_t rb_lds_bytes(int64_t nU, int64_t groups, int precision, bool lrec)
+inline size_t rb_lds_bytes(int64_t nU, int64_t groups, bool lrec)
 {
-	return ((size_t)nU * (precision == 1 ? 4 : 8) + 15) / 16 * 16 + (lrec ? (size_t)groups * 16 : 0);
+	return ((size_t)nU * 8 + 15) / 16 * 16 + (lrec ? (size_t)groups * 16 : 0);
 }
-inline const bicg_variant_t* rb_variant(int64_t nE, int64_t nR, int64_t groups, int precision, int B, size_t lds_max)
+inline const bicg_variant_t* rb_variant(int64_t nE, int64_t nR, int64_t groups, int B, size_t lds_max)
 {
 #define ESL_RB(BLK, RPT, LREC)                                                                                       \
-	{ { k_bicg_set<double, BLK, RPT, LREC>, k_bicg_set<float, BLK, RPT, LREC> }, BLK, BLK * RPT, LREC }
+	{ k_bicg_set<BLK, RPT, LREC>, BLK, BLK * RPT, LREC }
 	static const bicg_variant_t few[] = { ESL_RB(64, 1, true),	 ESL_RB(256, 1, true),	 ESL_RB(512, 1, true),
 										  ESL_RB(1024, 1, true), ESL_RB(1024, 2, false), ESL_RB(1024, 4, false) };
 	static const bicg_variant_t many[] = { ESL_RB(64, 2, true), ESL_RB(256, 2, true), ESL_RB(512, 2, true),
@@ -587,9 +578,881 @@ inline const bicg_variant_t* rb_variant(int64_t nE, int64_t nR, int64_t groups, 
 	const int64_t rows = nE > nR ? nE : nR;
 	auto pick = [&](const bicg_variant_t* v, int n) -> const bicg_variant_t* {
 		for (int i = 0; i < n; ++i)
-			if (rows <= v[i].rows && rb_lds_bytes(nE + nR, groups, precision, v[i].lrec) + rb_lds_static <= lds_max)
+			if (rows <= v[i].rows && rb_lds_bytes(nE + nR, groups, v[i].lrec) + rb_lds_static <= lds_max)
 				return v + i;
 		return nullptr;
 	};
 	return B <= rb_cus ? pick(few, sizeof few / sizeof *few) : pick(many, sizeof many / sizeof *many);
+}
+
+// ============================================================================
+// The same method device-wide, for systems too large for one workgroup.  Vectors
+// are [row][set] with rows in class order; a lane takes W (2, or 1 for an odd batch)
+// neighbouring sets of a row, a block up to 64 sets of R rows at a time.  A row's
+// records are read once per set pair, its neighbours' values are contiguous
+// 16-byte loads, and the rates of the block's sets sit in LDS.  A block owns a
+// contiguous range of rows, and blocks are dealt to the eight XCDs in contiguous
+// runs: most neighbours of a row (its low bits) then lie in what the same XCD's L2
+// holds.  Two products by S are eight launches and no host round trip; a step of
+// GMRES with ILU(0) was two launches per popcount level, a product by M and two
+// passes over up to 32 basis vectors.  Measured: 64 sets of 221,184 unknowns 138 ms
+// -> 59 ms, 16 sets of 524,288 unknowns 73 -> 24 ms.  Bound: the products' gathers
+// (64 sets of 221,184 unknowns: 78 us for 113 MB of compulsory vectors and eleven
+// neighbours a row), then the vector updates at 7 TB/s through the Infinity Cache.
+// One set per lane with rates from global memory took 110 us.
+
+constexpr int rbw_threads = 256; // threads of a block at most
+constexpr int rbw_sets = 64;	 // sets of a block at most
+
+struct rbw_geo_t
+{
+	int B, bs, L, R; // sets, sets per block, lanes per row, rows per step; block = L * R threads
+	int ncode;		 // 2N
+	const double* rates;
+	int64_t rstride;
+};
+
+// contiguous share of `rows` for this block; XCD i (blockIdx.x % 8) gets the i-th eighth of the blocks
+__device__ __forceinline__ void rbw_rows(int64_t rows, int64_t& q0, int64_t& q1)
+{
+	const int64_t nb = gridDim.x;
+	int64_t k = blockIdx.x;
+	if (nb % 8 == 0)
+		k = (k % 8) * (nb / 8) + k / 8;
+	q0 = rows * k / nb;
+	q1 = rows * (k + 1) / nb;
+}
+
+// the thread's row of a step, its first set, and whether that set exists (W divides B)
+#define ESL_RBW_THREAD                                                                                               \
+	const int t_row = (int)threadIdx.x / geo.L, bl = (int)threadIdx.x % geo.L * W;                                   \
+	const int b = (int)blockIdx.y * geo.bs + bl, B = geo.B;                                                          \
+	const bool in = bl < geo.bs && b < B
+
+template <int W>
+struct rbw_vec_t
+{
+	double v[W];
+};
+template <int W>
+__device__ __forceinline__ rbw_vec_t<W> rbw_load(const double* __restrict__ p)
+{
+	rbw_vec_t<W> r;
+	if constexpr (W == 2)
+	{
+		const double2 d = *(const double2*)p;
+		r.v[0] = d.x;
+		r.v[1] = d.y;
+	}
+	else
+		r.v[0] = *p;
+	return r;
+}
+template <int W>
+__device__ __forceinline__ void rbw_store(double* __restrict__ p, const rbw_vec_t<W>& r)
+{
+	if constexpr (W == 2)
+		*(double2*)p = make_double2(r.v[0], r.v[1]);
+	else
+		*p = r.v[0];
+}
+
+// rates of the block's sets into LDS, [code][set of the block]; code 2N (null records) is zero
+__device__ __forceinline__ double* rbw_lds_rates(const rbw_geo_t& geo)
+{
+	extern __shared__ __align__(16) unsigned char smem[];
+	double* s = (double*)smem;
+	for (int i = threadIdx.x; i < (geo.ncode + 1) * geo.bs; i += blockDim.x)
+	{
+		const int k = i % geo.bs, code = i / geo.bs, b = (int)blockIdx.y * geo.bs + k;
+		s[i] = code < geo.ncode && b < geo.B ? geo.rates[(int64_t)b * geo.rstride + code] : 0.0;
+	}
+	__syncthreads();
+	return s;
+}
+
+// sum over the couplings of row q for W sets; the next group's records are loaded
+// while this one's values are
+template <int W>
+__device__ __forceinline__ rbw_vec_t<W> rbw_sum(const rb_t& G, int64_t q, int b, int bl, const rbw_geo_t& geo,
+												const double* __restrict__ rt, const double* __restrict__ y)
+{
+	rbw_vec_t<W> s{};
+	int g = G.ptr[q];
+	const int g1 = G.ptr[q + 1];
+	uint4 c = G.rec[g];
+	const double* __restrict__ yb = y + b;
+	const double* __restrict__ rb = rt + bl;
+	const uint32_t B = (uint32_t)geo.B, bs = (uint32_t)geo.bs;
+	while (g < g1)
+	{
+		const uint4 nx = G.rec[++g];
+		const auto y0 = rbw_load<W>(yb + (uint64_t)(c.x & rb_index) * B), y1 = rbw_load<W>(yb + (uint64_t)(c.y & rb_index) * B);
+		const auto y2 = rbw_load<W>(yb + (uint64_t)(c.z & rb_index) * B), y3 = rbw_load<W>(yb + (uint64_t)(c.w & rb_index) * B);
+		const auto r0 = rbw_load<W>(rb + rb_code(c.x) * bs), r1 = rbw_load<W>(rb + rb_code(c.y) * bs);
+		const auto r2 = rbw_load<W>(rb + rb_code(c.z) * bs), r3 = rbw_load<W>(rb + rb_code(c.w) * bs);
+#pragma unroll
+		for (int w = 0; w < W; ++w)
+			s.v[w] += r0.v[w] * y0.v[w] + r1.v[w] * y1.v[w] + (r2.v[w] * y2.v[w] + r3.v[w] * y3.v[w]);
+		c = nx;
+	}
+	return s;
+}
+
+// per-set sums of a block: the R partials of a set folded in halves (a fixed
+// order), into part[blk][b][k].  Reuses the dynamic LDS from its start.
+template <int W, int K>
+__device__ __forceinline__ void rbw_block_sums(const rbw_geo_t& geo, const double (&v)[K][W], bool on, int b, int t_row,
+											   double* __restrict__ part)
+{
+	extern __shared__ __align__(16) unsigned char smem[];
+	double* s = (double*)smem; // [K][W][blockDim]
+	const int nt = blockDim.x;
+	__syncthreads();
+#pragma unroll
+	for (int k = 0; k < K; ++k)
+#pragma unroll
+		for (int w = 0; w < W; ++w)
+			s[(k * W + w) * nt + threadIdx.x] = on ? v[k][w] : 0.0;
+	for (int r = geo.R; r > 1;)
+	{
+		const int h = (r + 1) / 2;
+		__syncthreads();
+		if (t_row < r - h)
+#pragma unroll
+			for (int k = 0; k < K * W; ++k)
+				s[k * nt + threadIdx.x] += s[k * nt + threadIdx.x + h * geo.L];
+		r = h;
+	}
+	__syncthreads();
+	if (t_row == 0 && on)
+#pragma unroll
+		for (int w = 0; w < W; ++w)
+#pragma unroll
+			for (int k = 0; k < K; ++k)
+				part[((int64_t)blockIdx.x * geo.B + b + w) * K + k] = s[(k * W + w) * nt + threadIdx.x];
+}
+
+// state of a set through a cycle
+struct rbw_set_t
+{
+	double rho, alpha, omega, beta; // BiCGStab
+	double est;						// |r| -> relative residual
+	double scale;					// norm of the FP64 residual (the cycle solves for x / scale)
+	int32_t live, upd, fails, pad;
+};
+
+// ---- start
+
+// c = 1 / D of every row, and the masses the anchor sweeps start from (1 on
+// terminal rows, 0 on ambiguous ones)
+template <int W>
+__global__ void k_rbw_coef(sys_t S, rb_t G, rbw_geo_t geo, double* __restrict__ c, double* __restrict__ mE,
+						   double* __restrict__ mR)
+{
+	const double* rt = rbw_lds_rates(geo);
+	ESL_RBW_THREAD;
+	int64_t q0, q1;
+	rbw_rows(S.nU, q0, q1);
+	if (!in)
+		return;
+	for (int64_t q = q0 + t_row; q < q1; q += geo.R)
+	{
+		const int32_t u = G.row[q];
+		const uint32_t s = (uint32_t)S.ulist[u];
+		rbw_vec_t<W> d{}, m;
+		for (uint32_t k = S.mask[s]; k; k &= k - 1)
+		{
+			const int i = __ffs(k) - 1;
+#pragma unroll
+			for (int w = 0; w < W; ++w)
+				d.v[w] += rt[(2 * i + ((s >> i) & 1u)) * geo.bs + bl + w];
+		}
+#pragma unroll
+		for (int w = 0; w < W; ++w)
+		{
+			d.v[w] = 1.0 / d.v[w];
+			m.v[w] = S.ucls[u] >= 0 ? 1.0 : 0.0;
+		}
+		rbw_store<W>(c + q * B + b, d);
+		rbw_store<W>((q < G.nE ? mE + q * B : mR + (q - G.nE) * B) + b, m);
+	}
+}
+
+// Anchor sweeps: the damped Jacobi sweeps of k_anchor_sweep taken class by class.
+// E rows: m = inflow / D; R rows: m = (m + inflow / D) / 2.  One pair moves the mass
+// as far as two sweeps over all rows, so half as many do.
+constexpr int rbw_sweeps = 16;
+template <int W, bool KEPT>
+__global__ void k_rbw_sweep(rb_t G, rbw_geo_t geo, const double* __restrict__ c, const double* __restrict__ from,
+							double* __restrict__ to)
+{
+	const double* rt = rbw_lds_rates(geo);
+	ESL_RBW_THREAD;
+	int64_t q0, q1;
+	rbw_rows(KEPT ? G.nR : G.nE, q0, q1);
+	if (!in)
+		return;
+	for (int64_t o = q0 + t_row; o < q1; o += geo.R)
+	{
+		const int64_t q = KEPT ? G.nE + o : o;
+		auto s = rbw_sum<W>(G, q, b, bl, geo, rt, from);
+		const auto cc = rbw_load<W>(c + q * B + b);
+		rbw_vec_t<W> m{};
+		if (KEPT)
+			m = rbw_load<W>(to + o * B + b);
+#pragma unroll
+		for (int w = 0; w < W; ++w)
+			s.v[w] = KEPT ? 0.5 * m.v[w] + 0.5 * (cc.v[w] * s.v[w]) : cc.v[w] * s.v[w];
+		rbw_store<W>(to + o * B + b, s);
+	}
+}
+
+// index inside its class of the first unknown >= u, for each segment's bounds:
+// off[0][k] eliminated rows, off[1][k] kept rows
+__global__ __launch_bounds__(sblock) void k_rbw_seg_rows(rb_t G, int n_seg, const int32_t* __restrict__ seg_off,
+														 int32_t* __restrict__ off)
+{
+	const int k = blockIdx.x * sblock + threadIdx.x;
+	if (k > n_seg)
+		return;
+	for (int cls = 0; cls < 2; ++cls)
+	{
+		// rows of a class ascend in the unknowns
+		const int32_t* r = G.row + (cls ? G.nE : 0);
+		int lo = 0, hi = cls ? G.nR : G.nE;
+		while (lo < hi)
+		{
+			const int mid = (lo + hi) / 2;
+			if (r[mid] < seg_off[k])
+				lo = mid + 1;
+			else
+				hi = mid;
+		}
+		off[cls * (n_seg + 1) + k] = lo;
+	}
+}
+
+// largest mass of a slice of a segment per set, ties to the smallest unknown:
+// block (segment and slice, set chunk) -> pv / pu[slice][seg][b]
+template <int W>
+__global__ void k_rbw_pick(rb_t G, rbw_geo_t geo, int n_seg, int slices, const int32_t* __restrict__ off,
+						   const double* __restrict__ mE, const double* __restrict__ mR, double* __restrict__ pv,
+						   int32_t* __restrict__ pu)
+{
+	extern __shared__ __align__(16) unsigned char smem[];
+	ESL_RBW_THREAD;
+	const int k = blockIdx.x / slices, sl = blockIdx.x % slices, nt = blockDim.x;
+	double* s_v = (double*)smem;				   // [W][blockDim]
+	int32_t* s_u = (int32_t*)(s_v + W * nt); // [W][blockDim]
+	double best[W];
+	int32_t bu[W];
+#pragma unroll
+	for (int w = 0; w < W; ++w)
+	{
+		best[w] = -1.0;
+		bu[w] = INT32_MAX;
+	}
+	for (int cls = 0; cls < 2 && in; ++cls)
+	{
+		const int64_t a = off[cls * (n_seg + 1) + k], n = off[cls * (n_seg + 1) + k + 1] - a;
+		const int64_t o0 = a + n * sl / slices, o1 = a + n * (sl + 1) / slices;
+		for (int64_t o = o0 + t_row; o < o1; o += geo.R)
+		{
+			const auto m = rbw_load<W>((cls ? mR : mE) + o * B + b);
+			const int32_t u = G.row[cls ? G.nE + o : o];
+#pragma unroll
+			for (int w = 0; w < W; ++w)
+				if (m.v[w] > best[w] || (m.v[w] == best[w] && u < bu[w]))
+				{
+					best[w] = m.v[w];
+					bu[w] = u;
+				}
+		}
+	}
+#pragma unroll
+	for (int w = 0; w < W; ++w)
+	{
+		s_v[w * nt + threadIdx.x] = best[w];
+		s_u[w * nt + threadIdx.x] = bu[w];
+	}
+	__syncthreads();
+	if (t_row == 0 && in)
+#pragma unroll
+		for (int w = 0; w < W; ++w)
+		{
+			for (int r = 1; r < geo.R; ++r)
+			{
+				const double v = s_v[w * nt + threadIdx.x + r * geo.L];
+				const int32_t u = s_u[w * nt + threadIdx.x + r * geo.L];
+				if (v > best[w] || (v == best[w] && u < bu[w]))
+				{
+					best[w] = v;
+					bu[w] = u;
+				}
+			}
+			const int64_t at = ((int64_t)sl * n_seg + k) * B + b + w;
+			pv[at] = best[w];
+			pu[at] = bu[w];
+		}
+}
+
+// slices -> anchor[b][seg] and its mass pa[seg][b]
+__global__ __launch_bounds__(sblock) void k_rbw_anchor(int B, int n_seg, int slices, const double* __restrict__ pv,
+													   const int32_t* __restrict__ pu, int32_t* __restrict__ anchor,
+													   double* __restrict__ pa)
+{
+	const int i = blockIdx.x * sblock + threadIdx.x;
+	if (i >= n_seg * B)
+		return;
+	const int k = i / B, b = i - k * B;
+	double best = -1.0;
+	int32_t bu = INT32_MAX;
+	for (int s = 0; s < slices; ++s)
+	{
+		const int64_t at = ((int64_t)s * n_seg + k) * B + b;
+		if (pv[at] > best || (pv[at] == best && pu[at] < bu))
+		{
+			best = pv[at];
+			bu = pu[at];
+		}
+	}
+	anchor[(int64_t)b * n_seg + k] = bu;
+	pa[i] = best;
+}
+
+// start vector, right-hand side and anchors (c <- 0: the row is the identity).
+// Terminal rows start from their masses relative to the anchor's, ambiguous ones
+// from zero.  A start from the anchor alone would leave a residual with one or two
+// nonzeros, on which the first cycle breaks down.
+template <int W>
+__global__ void k_rbw_start(sys_t S, rb_t G, rbw_geo_t geo, int n_seg, const double* __restrict__ x0,
+							const double* __restrict__ mE, const double* __restrict__ mR, const double* __restrict__ pa,
+							double* __restrict__ c, double* __restrict__ x, double* __restrict__ wb)
+{
+	ESL_RBW_THREAD;
+	int64_t q0, q1;
+	rbw_rows(S.nU, q0, q1);
+	if (!in)
+		return;
+	for (int64_t q = q0 + t_row; q < q1; q += geo.R)
+	{
+		const int32_t u = G.row[q], k = S.ucls[u];
+		rbw_vec_t<W> xv{}, bv{};
+		if (k < 0)
+		{
+			const double v = x0[S.ulist[u]];
+#pragma unroll
+			for (int w = 0; w < W; ++w)
+				bv.v[w] = v;
+		}
+		else
+		{
+			const auto m = rbw_load<W>((q < G.nE ? mE + q * B : mR + (q - G.nE) * B) + b);
+#pragma unroll
+			for (int w = 0; w < W; ++w)
+			{
+				const double p = pa[(int64_t)k * B + b + w];
+				xv.v[w] = p > 0.0 ? m.v[w] / p : 0.0;
+				if (S.anchor[(int64_t)(b + w) * n_seg + k] == u)
+				{
+					xv.v[w] = bv.v[w] = 1.0;
+					c[q * B + b + w] = 0.0;
+				}
+			}
+		}
+		rbw_store<W>(x + q * B + b, xv);
+		rbw_store<W>(wb + q * B + b, bv);
+	}
+}
+
+constexpr int rbw_tile = 32; // rows (and sets) of a transposed tile
+
+// the warm start's counterpart: plan vectors (set-major) -> solver vectors, through
+// LDS tiles so that both sides are read and written along their rows
+__global__ __launch_bounds__(sblock) void k_rbw_enter(sys_t S, rb_t G, int n_seg, const double* __restrict__ rhs,
+													  const double* __restrict__ z, double* __restrict__ wx,
+													  double* __restrict__ wb, double* __restrict__ wc)
+{
+	__shared__ double s_x[rbw_tile][rbw_tile + 1], s_b[rbw_tile][rbw_tile + 1], s_c[rbw_tile][rbw_tile + 1];
+	const int64_t nU = S.nU, q0 = (int64_t)blockIdx.x * rbw_tile;
+	const int b0 = blockIdx.y * rbw_tile, tx = threadIdx.x % rbw_tile, ty = threadIdx.x / rbw_tile;
+	constexpr int step = sblock / rbw_tile;
+	const int64_t q = q0 + tx;
+	const int32_t u = q < nU ? G.row[q] : 0;
+	for (int j = ty; j < rbw_tile && q < nU; j += step)
+		if (b0 + j < S.B)
+		{
+			const int b = b0 + j;
+			const int64_t o = (int64_t)b * nU + u;
+			const double iv = S.invd[o];
+			s_x[j][tx] = z[o] * iv;
+			s_b[j][tx] = rhs[o];
+			s_c[j][tx] = is_anchor(S, n_seg, b, u) ? 0.0 : iv;
+		}
+	__syncthreads();
+	for (int j = ty; j < rbw_tile; j += step)
+		if (q0 + j < nU && b0 + tx < S.B)
+		{
+			const int64_t i = (q0 + j) * S.B + b0 + tx;
+			wx[i] = s_x[tx][j];
+			wb[i] = s_b[tx][j];
+			wc[i] = s_c[tx][j];
+		}
+}
+
+// z = D' x and 1 / D' (1 for anchors) back into the plan's layout
+__global__ __launch_bounds__(sblock) void k_rbw_leave(sys_t S, rb_t G, const double* __restrict__ wx,
+													  const double* __restrict__ wc, const double* __restrict__ dj,
+													  double* __restrict__ z, double* __restrict__ invd)
+{
+	__shared__ double s_x[rbw_tile][rbw_tile + 1], s_c[rbw_tile][rbw_tile + 1];
+	const int64_t nU = S.nU, q0 = (int64_t)blockIdx.x * rbw_tile;
+	const int b0 = blockIdx.y * rbw_tile, tx = threadIdx.x % rbw_tile, ty = threadIdx.x / rbw_tile;
+	constexpr int step = sblock / rbw_tile;
+	for (int j = ty; j < rbw_tile; j += step)
+		if (q0 + j < nU && b0 + tx < S.B)
+		{
+			const int64_t i = (q0 + j) * S.B + b0 + tx;
+			double cc = wc[i];
+			if (cc != 0.0 && q0 + j >= G.nE)
+				cc /= dj[i - (int64_t)G.nE * S.B]; // J / (D J)
+			s_x[j][tx] = wx[i];
+			s_c[j][tx] = cc != 0.0 ? cc : 1.0;
+		}
+	__syncthreads();
+	const int64_t q = q0 + tx;
+	const int32_t u = q < nU ? G.row[q] : 0;
+	for (int j = ty; j < rbw_tile && q < nU; j += step)
+		if (b0 + j < S.B)
+		{
+			const int64_t o = (int64_t)(b0 + j) * nU + u;
+			z[o] = s_x[tx][j] / s_c[tx][j];
+			if (invd)
+				invd[o] = s_c[tx][j];
+		}
+}
+
+// kept rows: J = 1 / diag(S) in place of 1 / D (0 for an anchor), and D J (1 for an anchor)
+template <int W>
+__global__ void k_rbw_diag(rb_t G, rbw_geo_t geo, double* __restrict__ c, double* __restrict__ dj)
+{
+	const double* rt = rbw_lds_rates(geo);
+	ESL_RBW_THREAD;
+	int64_t q0, q1;
+	rbw_rows(G.nR, q0, q1);
+	if (!in)
+		return;
+	for (int64_t o = q0 + t_row; o < q1; o += geo.R)
+	{
+		const int64_t q = G.nE + o;
+		auto cc = rbw_load<W>(c + q * B + b);
+		rbw_vec_t<W> back{}, dv;
+		for (int g = G.ptr[q]; g < G.ptr[q + 1]; ++g)
+		{
+			const uint4 r4 = G.rec[g];
+			const uint32_t r[4] = { r4.x, r4.y, r4.z, r4.w };
+#pragma unroll
+			for (int k = 0; k < 4; ++k)
+				if (r[k] >> 31) // an anchor's coefficient is zero, so its mirrored entry counts nothing
+				{
+					const auto ce = rbw_load<W>(c + (int64_t)(r[k] & rb_index) * B + b);
+#pragma unroll
+					for (int w = 0; w < W; ++w)
+						back.v[w] += rt[rb_code(r[k]) * geo.bs + bl + w] * rt[(rb_code(r[k]) ^ 1) * geo.bs + bl + w] * ce.v[w];
+				}
+		}
+#pragma unroll
+		for (int w = 0; w < W; ++w)
+		{
+			const bool anchor = cc.v[w] == 0.0;
+			const double D = 1.0 / cc.v[w], d = D - back.v[w];
+			const double J = 1.0 / (d > 0.0 ? d : D);
+			cc.v[w] = anchor ? 0.0 : J;
+			dv.v[w] = anchor ? 1.0 : D * J;
+		}
+		rbw_store<W>(c + q * B + b, cc);
+		rbw_store<W>(dj + o * B + b, dv);
+	}
+}
+
+// ---- cycles
+
+// FP64 residual of every row; partial sums of r^2 and b^2
+template <int W>
+__global__ void k_rbw_residual(rb_t G, rbw_geo_t geo, const double* __restrict__ c, const double* __restrict__ dj,
+							   const double* __restrict__ wb, const double* __restrict__ x, double* __restrict__ r,
+							   double* __restrict__ part)
+{
+	const double* rt = rbw_lds_rates(geo);
+	ESL_RBW_THREAD;
+	const int64_t nE = G.nE, nU = nE + G.nR;
+	int64_t q0, q1;
+	rbw_rows(nU, q0, q1);
+	double sum[2][W] = {};
+	if (in)
+		for (int64_t q = q0 + t_row; q < q1; q += geo.R)
+		{
+			const int64_t i = q * B + b;
+			const auto cc = rbw_load<W>(c + i), bv = rbw_load<W>(wb + i), xv = rbw_load<W>(x + i);
+			const auto s = rbw_sum<W>(G, q, b, bl, geo, rt, q < nE ? x + nE * B : x);
+			rbw_vec_t<W> d, res;
+			if (q >= nE)
+				d = rbw_load<W>(dj + i - nE * B);
+#pragma unroll
+			for (int w = 0; w < W; ++w)
+			{
+				const double D = q < nE ? 1.0 / cc.v[w] : d.v[w] / cc.v[w];
+				res.v[w] = cc.v[w] != 0.0 ? bv.v[w] - (D * xv.v[w] - s.v[w]) : bv.v[w] - xv.v[w];
+				sum[0][w] += res.v[w] * res.v[w];
+				sum[1][w] += bv.v[w] * bv.v[w];
+			}
+			rbw_store<W>(r + i, res);
+		}
+	rbw_block_sums<W, 2>(geo, sum, in, b, t_row, part);
+}
+
+// whether any of the thread's sets is in the cycle (others run along, unused)
+template <int W>
+__device__ __forceinline__ bool rbw_live(const rbw_set_t* __restrict__ st, int b)
+{
+	bool l = st[b].live != 0;
+	if constexpr (W == 2)
+		l = l || st[b + 1].live != 0;
+	return l;
+}
+
+// t_E at the start of a cycle: r_E / (D scale)
+template <int W>
+__global__ void k_rbw_te0(rb_t G, rbw_geo_t geo, const double* __restrict__ c, const double* __restrict__ r,
+						  double* __restrict__ te, const rbw_set_t* __restrict__ st)
+{
+	ESL_RBW_THREAD;
+	int64_t q0, q1;
+	rbw_rows(G.nE, q0, q1);
+	if (!in || !rbw_live<W>(st, b))
+		return;
+	double inv[W];
+#pragma unroll
+	for (int w = 0; w < W; ++w)
+		inv[w] = st[b + w].live ? 1.0 / st[b + w].scale : 0.0;
+	for (int64_t q = q0 + t_row; q < q1; q += geo.R)
+	{
+		const int64_t i = q * B + b;
+		const auto cc = rbw_load<W>(c + i);
+		auto rv = rbw_load<W>(r + i);
+#pragma unroll
+		for (int w = 0; w < W; ++w)
+			rv.v[w] *= (cc.v[w] != 0.0 ? cc.v[w] : 1.0) * inv[w];
+		rbw_store<W>(te + i, rv);
+	}
+}
+
+// start of a cycle: r = J (r_R + A t_E) / scale, shadow vector, p = r, x = 0; sums of r.r and rh.r
+template <int W>
+__global__ void k_rbw_init(rb_t G, rbw_geo_t geo, const double* __restrict__ c, const double* __restrict__ res,
+						   const double* __restrict__ te, double* __restrict__ r, double* __restrict__ rh,
+						   double* __restrict__ p, double* __restrict__ x, const rbw_set_t* __restrict__ st,
+						   double* __restrict__ part)
+{
+	const double* rt = rbw_lds_rates(geo);
+	ESL_RBW_THREAD;
+	int64_t q0, q1;
+	rbw_rows(G.nR, q0, q1);
+	double sum[2][W] = {};
+	if (in && rbw_live<W>(st, b))
+	{
+		double inv[W];
+		int fails[W];
+#pragma unroll
+		for (int w = 0; w < W; ++w)
+		{
+			inv[w] = st[b + w].live ? 1.0 / st[b + w].scale : 0.0;
+			fails[w] = st[b + w].fails;
+		}
+		for (int64_t o = q0 + t_row; o < q1; o += geo.R)
+		{
+			const int64_t q = G.nE + o, i = o * B + b;
+			const auto J = rbw_load<W>(c + q * B + b), rv = rbw_load<W>(res + q * B + b);
+			const auto s = rbw_sum<W>(G, q, b, bl, geo, rt, te);
+			rbw_vec_t<W> g, h;
+#pragma unroll
+			for (int w = 0; w < W; ++w)
+			{
+				g.v[w] = rv.v[w] * inv[w];
+				if (J.v[w] != 0.0)
+					g.v[w] = J.v[w] * (g.v[w] + s.v[w]);
+				h.v[w] = rb_shadow((int)o, fails[w], g.v[w]);
+				sum[0][w] += g.v[w] * g.v[w];
+				sum[1][w] += h.v[w] * g.v[w];
+			}
+			rbw_store<W>(r + i, g);
+			rbw_store<W>(p + i, g);
+			rbw_store<W>(rh + i, h);
+			rbw_store<W>(x + i, rbw_vec_t<W>{});
+		}
+	}
+	rbw_block_sums<W, 2>(geo, sum, in, b, t_row, part);
+}
+
+// t_E = 1/D (A y) on the eliminated rows
+template <int W>
+__global__ void k_rbw_te(rb_t G, rbw_geo_t geo, const double* __restrict__ c, const double* __restrict__ y,
+						 double* __restrict__ te, const rbw_set_t* __restrict__ st)
+{
+	const double* rt = rbw_lds_rates(geo);
+	ESL_RBW_THREAD;
+	int64_t q0, q1;
+	rbw_rows(G.nE, q0, q1);
+	if (!in || !rbw_live<W>(st, b))
+		return;
+	for (int64_t q = q0 + t_row; q < q1; q += geo.R)
+	{
+		const auto cc = rbw_load<W>(c + q * B + b);
+		auto s = rbw_sum<W>(G, q, b, bl, geo, rt, y);
+#pragma unroll
+		for (int w = 0; w < W; ++w)
+			s.v[w] *= cc.v[w];
+		rbw_store<W>(te + q * B + b, s);
+	}
+}
+
+// out = J S y on the kept rows.  FULL false: with the sum rh.out (v of the step);
+// true: with out.y, out.out, y.y, rh.y, rh.out (t of the step)
+template <int W, bool FULL>
+__global__ void k_rbw_mul(rb_t G, rbw_geo_t geo, const double* __restrict__ c, const double* __restrict__ dj,
+						  const double* __restrict__ te, const double* __restrict__ y, const double* __restrict__ rh,
+						  double* __restrict__ out, const rbw_set_t* __restrict__ st, double* __restrict__ part)
+{
+	constexpr int K = FULL ? 5 : 1;
+	const double* rt = rbw_lds_rates(geo);
+	ESL_RBW_THREAD;
+	int64_t q0, q1;
+	rbw_rows(G.nR, q0, q1);
+	double sum[K][W] = {};
+	if (in && rbw_live<W>(st, b))
+		for (int64_t o = q0 + t_row; o < q1; o += geo.R)
+		{
+			const int64_t q = G.nE + o, i = o * B + b;
+			const auto J = rbw_load<W>(c + q * B + b), d = rbw_load<W>(dj + i), yv = rbw_load<W>(y + i),
+					   hv = rbw_load<W>(rh + i);
+			auto s = rbw_sum<W>(G, q, b, bl, geo, rt, te);
+#pragma unroll
+			for (int w = 0; w < W; ++w)
+			{
+				const double t = d.v[w] * yv.v[w] - J.v[w] * s.v[w];
+				s.v[w] = t;
+				if constexpr (FULL)
+				{
+					sum[0][w] += t * yv.v[w];
+					sum[1][w] += t * t;
+					sum[2][w] += yv.v[w] * yv.v[w];
+					sum[3][w] += hv.v[w] * yv.v[w];
+					sum[4][w] += hv.v[w] * t;
+				}
+				else
+					sum[0][w] += hv.v[w] * t;
+			}
+			rbw_store<W>(out + i, s);
+		}
+	rbw_block_sums<W, K>(geo, sum, in, b, t_row, part);
+}
+
+// s = r - alpha v, in place
+template <int W>
+__global__ void k_rbw_s(int64_t nR, rbw_geo_t geo, double* __restrict__ r, const double* __restrict__ v,
+						const rbw_set_t* __restrict__ st)
+{
+	ESL_RBW_THREAD;
+	int64_t q0, q1;
+	rbw_rows(nR, q0, q1);
+	if (!in || !rbw_live<W>(st, b))
+		return;
+	double alpha[W];
+#pragma unroll
+	for (int w = 0; w < W; ++w)
+		alpha[w] = st[b + w].live ? st[b + w].alpha : 0.0;
+	for (int64_t o = q0 + t_row; o < q1; o += geo.R)
+	{
+		const auto vv = rbw_load<W>(v + o * B + b);
+		auto rv = rbw_load<W>(r + o * B + b);
+#pragma unroll
+		for (int w = 0; w < W; ++w)
+			if (alpha[w] != 0.0)
+				rv.v[w] -= alpha[w] * vv.v[w];
+		rbw_store<W>(r + o * B + b, rv);
+	}
+}
+
+// x += alpha p + omega s;  r = s - omega t;  p = r + beta (p - omega v)
+template <int W>
+__global__ void k_rbw_update(int64_t nR, rbw_geo_t geo, double* __restrict__ x, double* __restrict__ r,
+							 double* __restrict__ p, const double* __restrict__ v, const double* __restrict__ t,
+							 const rbw_set_t* __restrict__ st)
+{
+	ESL_RBW_THREAD;
+	int64_t q0, q1;
+	rbw_rows(nR, q0, q1);
+	if (!in)
+		return;
+	bool upd[W], any = false;
+	double alpha[W], omega[W], beta[W];
+#pragma unroll
+	for (int w = 0; w < W; ++w)
+	{
+		upd[w] = st[b + w].upd != 0;
+		any = any || upd[w];
+		alpha[w] = st[b + w].alpha;
+		omega[w] = st[b + w].omega;
+		beta[w] = st[b + w].beta;
+	}
+	if (!any)
+		return;
+	for (int64_t o = q0 + t_row; o < q1; o += geo.R)
+	{
+		const int64_t i = o * B + b;
+		auto xv = rbw_load<W>(x + i), rv = rbw_load<W>(r + i), pv = rbw_load<W>(p + i);
+		const auto vv = rbw_load<W>(v + i), tv = rbw_load<W>(t + i);
+#pragma unroll
+		for (int w = 0; w < W; ++w)
+			if (upd[w])
+			{
+				xv.v[w] += alpha[w] * pv.v[w] + omega[w] * rv.v[w];
+				rv.v[w] -= omega[w] * tv.v[w];
+				pv.v[w] = rv.v[w] + beta[w] * (pv.v[w] - omega[w] * vv.v[w]);
+			}
+		rbw_store<W>(x + i, xv);
+		rbw_store<W>(r + i, rv);
+		rbw_store<W>(p + i, pv);
+	}
+}
+
+// end of a cycle, FP64: KEPT: x_R += scale dx, else x_E += 1/D (r_E + scale A dx);
+// keep receives the iterate before
+template <int W, bool KEPT>
+__global__ void k_rbw_correct(rb_t G, rbw_geo_t geo, const double* __restrict__ c, const double* __restrict__ res,
+							  const double* __restrict__ dx, double* __restrict__ x, double* __restrict__ keep,
+							  const rbw_set_t* __restrict__ st)
+{
+	const double* rt = KEPT ? nullptr : rbw_lds_rates(geo);
+	ESL_RBW_THREAD;
+	int64_t q0, q1;
+	rbw_rows(KEPT ? G.nR : G.nE, q0, q1);
+	if (!in)
+		return;
+	double scale[W];
+	bool any = false;
+#pragma unroll
+	for (int w = 0; w < W; ++w)
+	{
+		scale[w] = st[b + w].scale;
+		any = any || scale[w] > 0.0;
+	}
+	if (!any)
+		return;
+	for (int64_t o = q0 + t_row; o < q1; o += geo.R)
+	{
+		const int64_t i = (KEPT ? G.nE + o : o) * B + b;
+		auto xv = rbw_load<W>(x + i);
+		rbw_store<W>(keep + i, xv);
+		rbw_vec_t<W> d, cc{}, rv{};
+		if (KEPT)
+			d = rbw_load<W>(dx + o * B + b);
+		else
+		{
+			cc = rbw_load<W>(c + i);
+			rv = rbw_load<W>(res + i);
+			d = rbw_sum<W>(G, o, b, bl, geo, rt, dx);
+		}
+#pragma unroll
+		for (int w = 0; w < W; ++w)
+			if (scale[w] > 0.0)
+				xv.v[w] += KEPT			   ? scale[w] * d.v[w]
+						   : cc.v[w] != 0.0 ? cc.v[w] * (rv.v[w] + scale[w] * d.v[w])
+											: rv.v[w];
+		rbw_store<W>(x + i, xv);
+	}
+}
+
+// the iterate before the last cycle, for the sets of `undo`
+__global__ __launch_bounds__(sblock) void k_rbw_undo(int64_t count, int B, const double* __restrict__ keep,
+													 double* __restrict__ x, const int32_t* __restrict__ undo)
+{
+	const int64_t i = (int64_t)blockIdx.x * sblock + threadIdx.x;
+	if (i < count && undo[i % B])
+		x[i] = keep[i];
+}
+
+// sums over the blocks of part[blk][b][K] (one workgroup per set, fixed order),
+// then that set's scalars.  STEP 0: residual norms to out[b][2]; 1: start of a
+// cycle; 2: alpha; 3: omega, beta and whether the set goes on, also into the
+// host's mirror.
+template <int STEP>
+__global__ __launch_bounds__(sblock) void k_rbw_reduce(const double* __restrict__ part, int nblk, int B,
+													   rbw_set_t* __restrict__ st, double* __restrict__ out,
+													   int32_t* __restrict__ h_live, double aim)
+{
+	constexpr int K = STEP == 2 ? 1 : STEP == 3 ? 5 : 2;
+	__shared__ double s_part[rb_part];
+	const int b = blockIdx.x;
+	const bool on = STEP == 0 || st[b].live;
+	if (STEP == 3 && !on)
+	{
+		if (threadIdx.x == 0)
+		{
+			st[b].upd = 0;
+			h_live[b] = 0;
+		}
+		return;
+	}
+	if (!on)
+		return;
+	double v[K];
+#pragma unroll
+	for (int k = 0; k < K; ++k)
+		v[k] = 0.0;
+	for (int i = threadIdx.x; i < nblk; i += sblock)
+#pragma unroll
+		for (int k = 0; k < K; ++k)
+			v[k] += part[((int64_t)i * B + b) * K + k];
+	rb_block_sums<sblock>(v, s_part);
+	if (threadIdx.x != 0)
+		return;
+	if constexpr (STEP == 0)
+	{
+		out[2 * b] = v[0];
+		out[2 * b + 1] = v[1];
+	}
+	else if constexpr (STEP == 1)
+	{
+		rbw_set_t& s = st[b];
+		s.rho = v[1];
+		s.est = v[0] > 0.0 ? s.est / sqrt(v[0]) : 0.0; // the host left the relative residual here
+		if (!(v[0] > 0.0))
+			s.live = 0; // nothing left on the kept rows: the correction solves the eliminated ones
+	}
+	else if constexpr (STEP == 2)
+	{
+		rbw_set_t& s = st[b];
+		s.alpha = s.rho / v[0];
+		if (!rb_finite(s.alpha))
+			s.live = 0;
+	}
+	else
+	{
+		rbw_set_t& s = st[b];
+		double omega = v[1] > 0.0 ? v[0] / v[1] : 0.0;
+		if (!rb_finite(omega))
+			omega = 0.0;
+		const double rr = fmax(v[2] - omega * (2.0 * v[0] - omega * v[1]), 0.0);
+		const double rho1 = v[3] - omega * v[4];
+		const double beta = (rho1 / s.rho) * (s.alpha / omega);
+		const bool stop = sqrt(rr) * s.est <= aim || omega == 0.0 || !rb_finite(beta) || beta == 0.0;
+		s.omega = omega;
+		s.beta = stop ? 0.0 : beta;
+		s.rho = rho1;
+		s.upd = 1;
+		s.live = stop ? 0 : 1;
+		h_live[b] = s.live;
+	}
 }

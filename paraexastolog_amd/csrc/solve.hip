@@ -50,6 +50,7 @@
 #include <memory>
 #include <mutex>
 #include <thread>
+#include <type_traits>
 
 #include "common.hip.hpp"
 #include "esl_internal.hpp"
@@ -3419,8 +3420,8 @@ void build_rb(ctx_t& c, const sys_t& S, nbr_store_t& st, const int32_t* opos, in
 	ESL_HIP(hipMemcpyAsync(&groups, st.rptr.get() + nU, sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
 	ESL_HIP(hipStreamSynchronize(c.stream));
 	st.rgroups = groups;
-	st.rrec.ensure(std::max(groups, 1));
-	k_rb_fill<<<nb, sblock, 0, c.stream>>>(nU, st.rrow.get(), inv.get(), st.ptr.get(), st.nu.get(), st.nr.get(),
+	st.rrec.ensure((size_t)groups + 1); // a group past the last, for loads ahead
+	k_rb_fill<<<nb, sblock, 0, c.stream>>>(nU, 2 * S.N, st.rrow.get(), inv.get(), st.ptr.get(), st.nu.get(), st.nr.get(),
 										   st.rptr.get(), st.rrec.get());
 	ESL_HIP(hipGetLastError());
 	ESL_HIP(hipStreamSynchronize(c.stream));
@@ -3786,6 +3787,336 @@ struct gmres_w_t
 	}
 };
 
+// buffers of the device-wide reduced solver, kept with the plan between solves
+struct rbw_ws_t
+{
+	dbuf<double> x, b, c, dj, res, keep, part, norms, pick_v, pa;
+	dbuf<double> vec; // the vectors of the cycle: six on the kept rows, one on the others
+	dbuf<rbw_set_t> st;
+	dbuf<int32_t> undo, pick_u, seg_rows;
+	// liveness after each iteration, written by the device (two iterations deep)
+	int32_t* h_live = nullptr;
+	size_t n_live = 0;
+	hipEvent_t ev[2] = { nullptr, nullptr };
+	rbw_ws_t() = default;
+	rbw_ws_t(const rbw_ws_t&) = delete;
+	rbw_ws_t& operator=(const rbw_ws_t&) = delete;
+	void reset()
+	{
+		for (dbuf<double>* d : { &x, &b, &c, &dj, &res, &keep, &part, &norms, &pick_v, &pa, &vec })
+			d->reset();
+		st.reset();
+		for (dbuf<int32_t>* d : { &undo, &pick_u, &seg_rows })
+			d->reset();
+		if (h_live)
+			(void)hipHostFree(h_live);
+		h_live = nullptr;
+		n_live = 0;
+		for (hipEvent_t& e : ev)
+		{
+			if (e)
+				(void)hipEventDestroy(e);
+			e = nullptr;
+		}
+	}
+	~rbw_ws_t() { reset(); }
+	void reserve(int64_t nE, int64_t nR, int B, int nblk, int n_seg, int slices)
+	{
+		const size_t cU = (size_t)(nE + nR) * B, cR = (size_t)nR * B, cE = (size_t)nE * B;
+		for (dbuf<double>* d : { &x, &b, &c, &res, &keep })
+			d->ensure(cU);
+		dj.ensure(cR);
+		part.ensure((size_t)nblk * B * 5);
+		norms.ensure((size_t)2 * B);
+		vec.ensure(6 * cR + cE);
+		pick_v.ensure((size_t)slices * n_seg * B);
+		pick_u.ensure((size_t)slices * n_seg * B);
+		pa.ensure((size_t)n_seg * B);
+		seg_rows.ensure((size_t)2 * (n_seg + 1));
+		st.ensure(B);
+		undo.ensure(B);
+		if (n_live < (size_t)2 * B)
+		{
+			if (h_live)
+				ESL_HIP(hipHostFree(h_live));
+			h_live = nullptr;
+			ESL_HIP(hipHostMalloc((void**)&h_live, (size_t)2 * B * sizeof(int32_t), hipHostMallocDefault));
+			n_live = (size_t)2 * B;
+		}
+		for (hipEvent_t& e : ev)
+			if (!e)
+				ESL_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+	}
+};
+
+// Device-wide BiCGStab on the parity-reduced system (the k_rbw_* kernels) for up
+// to 1024 sets.  The host drives the cycles: it reads the FP64 residuals, decides
+// per set (converged, another cycle, undone, stalled) and enqueues the iterations,
+// checking liveness one iteration late so that the device never waits for it.
+struct bicg_w_t
+{
+	ctx_t& c;
+	const sys_t& S;
+	const nbr_store_t& NB;
+	rbw_ws_t& ws;
+	int n_seg, B, W;
+	rb_t G;
+	rbw_geo_t geo{};
+	int nbR, nbE, nbU, chunks, slices = 1;
+	double *X, *R, *RH, *P, *V, *T2, *TE;
+	std::vector<double> h_res; // relative residuals of the last check
+	int iters = 0, cycles = 0;
+	double final_res = 0.0;
+
+	bicg_w_t(ctx_t& ctx, const sys_t& sys, const nbr_store_t& nb, rbw_ws_t& w, int nseg)
+		: c(ctx), S(sys), NB(nb), ws(w), n_seg(nseg), B(sys.B), G(nb.rview())
+	{
+		// up to 64 sets (an even share) side by side, two to a lane where the batch is
+		// even, and as many rows as fill the block
+		W = B % 2 ? 1 : 2;
+		geo.B = B;
+		geo.bs = ceil_div(ceil_div(B, ceil_div(B, rbw_sets)), W) * W;
+		chunks = ceil_div(B, geo.bs);
+		geo.L = geo.bs / W;
+		geo.R = std::max(1, rbw_threads / geo.L);
+		geo.ncode = 2 * S.N;
+		geo.rates = S.rates;
+		geo.rstride = S.rate_stride;
+		auto blocks = [&](int64_t rows) {
+			const int64_t k = std::max<int64_t>(1, std::min<int64_t>(ceil_div(rows, geo.R), std::max(8, 2048 / chunks)));
+			return (int)(k > 8 ? k / 8 * 8 : k);
+		};
+		nbR = blocks(G.nR);
+		nbE = blocks(G.nE);
+		nbU = blocks((int64_t)G.nE + G.nR);
+		slices = (int)std::max<int64_t>(1, std::min<int64_t>(64, S.nUt / (64 * std::max(1, n_seg))));
+		ws.reserve(G.nE, G.nR, B, std::max(nbR, nbU), n_seg, slices);
+		const size_t cR = (size_t)G.nR * B;
+		X = ws.vec.get();
+		R = X + cR;
+		RH = R + cR;
+		P = RH + cR;
+		V = P + cR;
+		T2 = V + cR;
+		TE = T2 + cR;
+		h_res.assign(B, 0.0);
+	}
+
+	// a kernel over row blocks, for W sets per lane (pick(W) names it); K sums per set
+	// go through LDS, over the rates' place
+	template <typename F, typename... A>
+	void rows(int nb, int K, bool rates, F pick, A... args)
+	{
+		const int nt = geo.L * geo.R;
+		const size_t lds = std::max((size_t)K * W * nt, rates ? (size_t)(geo.ncode + 1) * geo.bs : 0) * sizeof(double);
+		if (W == 2)
+			pick(two{})<<<dim3(nb, chunks), nt, lds, c.stream>>>(args...);
+		else
+			pick(one{})<<<dim3(nb, chunks), nt, lds, c.stream>>>(args...);
+	}
+	using one = std::integral_constant<int, 1>;
+	using two = std::integral_constant<int, 2>;
+
+	// set-up from the rates alone: coefficients, anchors (into anchor[b][seg]), start
+	// vector and right-hand side
+	void enter(const double* x0, const int32_t* seg_off, int segs, int32_t* anchor)
+	{
+		rows(nbU, 0, true, [](auto w) { return k_rbw_coef<decltype(w)::value>; }, S, G, geo, ws.c.get(), TE, P);
+		if (segs)
+		{
+			for (int it = 0; it < rbw_sweeps; ++it)
+			{
+				timed_launch(c, "k_rbw_sweep", 24.0 * G.nE * B, [&] {
+					rows(nbE, 0, true, [](auto w) { return k_rbw_sweep<decltype(w)::value, false>; }, G, geo, ws.c.get(), P, TE);
+				});
+				timed_launch(c, "k_rbw_sweep", 32.0 * G.nR * B, [&] {
+					rows(nbR, 0, true, [](auto w) { return k_rbw_sweep<decltype(w)::value, true>; }, G, geo, ws.c.get(), TE, P);
+				});
+			}
+			k_rbw_seg_rows<<<ceil_div(segs + 1, sblock), sblock, 0, c.stream>>>(G, segs, seg_off, ws.seg_rows.get());
+			const int nt = geo.L * geo.R;
+			const size_t lds = (size_t)W * nt * 12;
+			const dim3 gp(slices * segs, chunks);
+			if (W == 2)
+				k_rbw_pick<2><<<gp, nt, lds, c.stream>>>(G, geo, segs, slices, ws.seg_rows.get(), TE, P, ws.pick_v.get(),
+														 ws.pick_u.get());
+			else
+				k_rbw_pick<1><<<gp, nt, lds, c.stream>>>(G, geo, segs, slices, ws.seg_rows.get(), TE, P, ws.pick_v.get(),
+														 ws.pick_u.get());
+			k_rbw_anchor<<<ceil_div(segs * B, sblock), sblock, 0, c.stream>>>(B, segs, slices, ws.pick_v.get(),
+																			   ws.pick_u.get(), anchor, ws.pa.get());
+		}
+		rows(nbU, 0, false, [](auto w) { return k_rbw_start<decltype(w)::value>; }, S, G, geo, n_seg, x0, TE, P, ws.pa.get(), ws.c.get(), ws.x.get(), ws.b.get());
+		diag();
+	}
+
+	// from the plan's vectors (a warm start, or another system set up set-major)
+	void enter(const double* rhs, const double* z)
+	{
+		const dim3 gt(ceil_div(S.nU, rbw_tile), ceil_div(B, rbw_tile));
+		k_rbw_enter<<<gt, sblock, 0, c.stream>>>(S, G, n_seg, rhs, z, ws.x.get(), ws.b.get(), ws.c.get());
+		diag();
+	}
+
+	void diag()
+	{
+		rows(nbR, 0, true, [](auto w) { return k_rbw_diag<decltype(w)::value>; }, G, geo, ws.c.get(), ws.dj.get());
+		ESL_HIP(hipGetLastError());
+	}
+
+	void leave(double* z, double* invd)
+	{
+		const dim3 gt(ceil_div(S.nU, rbw_tile), ceil_div(B, rbw_tile));
+		k_rbw_leave<<<gt, sblock, 0, c.stream>>>(S, G, ws.x.get(), ws.c.get(), ws.dj.get(), z, invd);
+		ESL_HIP(hipGetLastError());
+	}
+
+	bool live_after(int j)
+	{
+		ESL_HIP(hipEventSynchronize(ws.ev[j & 1]));
+		const int32_t* f = ws.h_live + (size_t)(j & 1) * B;
+		return std::any_of(f, f + B, [](int32_t v) { return v != 0; });
+	}
+
+	// two products by S for every live set
+	void iteration(int j, double aim)
+	{
+		const rbw_set_t* st = ws.st.get();
+		const double *cc = ws.c.get(), *dj = ws.dj.get();
+		double* part = ws.part.get();
+		int32_t* live = ws.h_live + (size_t)(j & 1) * B;
+		// algorithmic bytes: each vector and coefficient the step reads or writes once
+		const double eb = 8.0 * G.nE * B, rb = 8.0 * G.nR * B, st_b = 16.0 * NB.rgroups;
+		for (int half = 0; half < 2; ++half)
+		{
+			timed_launch(c, "k_rbw_te", rb + 2.0 * eb + st_b, [&] {
+				rows(nbE, 0, true, [](auto w) { return k_rbw_te<decltype(w)::value>; }, G, geo, cc, half ? R : P, TE, st);
+			});
+			timed_launch(c, "k_rbw_mul", eb + 5.0 * rb + st_b, [&] {
+				if (half)
+				{
+					rows(nbR, 5, true, [](auto w) { return k_rbw_mul<decltype(w)::value, true>; }, G, geo, cc, dj, TE, R, RH, T2, st, part);
+				}
+				else
+				{
+					rows(nbR, 1, true, [](auto w) { return k_rbw_mul<decltype(w)::value, false>; }, G, geo, cc, dj, TE, P, RH, V, st, part);
+				}
+			});
+			if (half)
+			{
+				k_rbw_reduce<3><<<B, sblock, 0, c.stream>>>(part, nbR, B, ws.st.get(), nullptr, live, aim);
+				timed_launch(c, "k_rbw_update", 8.0 * rb, [&] {
+					rows(nbR, 0, false, [](auto w) { return k_rbw_update<decltype(w)::value>; }, (int64_t)G.nR, geo, X, R, P, V, T2, st);
+				});
+			}
+			else
+			{
+				k_rbw_reduce<2><<<B, sblock, 0, c.stream>>>(part, nbR, B, ws.st.get(), nullptr, nullptr, 0.0);
+				timed_launch(c, "k_rbw_s", 3.0 * rb, [&] {
+					rows(nbR, 0, false, [](auto w) { return k_rbw_s<decltype(w)::value>; }, (int64_t)G.nR, geo, R, V, st);
+				});
+			}
+		}
+		ESL_HIP(hipGetLastError());
+		ESL_HIP(hipEventRecord(ws.ev[j & 1], c.stream));
+	}
+
+	// false when sets are left above the tolerance
+	bool solve(double tol, int max_iters)
+	{
+		std::vector<double> norms, prev(B, 0.0);
+		std::vector<rbw_set_t> hs(B);
+		std::vector<int32_t> undo(B, 0), fails(B, 0), compare(B, 0);
+		const double* cc = ws.c.get();
+		for (;;)
+		{
+			rows(nbU, 2, true, [](auto w) { return k_rbw_residual<decltype(w)::value>; }, G, geo, cc, ws.dj.get(), ws.b.get(), ws.x.get(), ws.res.get(), ws.part.get());
+			k_rbw_reduce<0><<<B, sblock, 0, c.stream>>>(ws.part.get(), nbU, B, ws.st.get(), ws.norms.get(), nullptr, 0.0);
+			ESL_HIP(hipGetLastError());
+			read_host(c, norms, ws.norms.get(), (size_t)2 * B);
+			bool any_undo = false, any_live = false, all = true;
+			final_res = 0.0;
+			for (int b = 0; b < B; ++b)
+			{
+				const double beta = std::sqrt(norms[2 * b]), bn = norms[2 * b + 1] > 0.0 ? std::sqrt(norms[2 * b + 1]) : 1.0;
+				double rel = beta / bn;
+				undo[b] = 0;
+				hs[b] = rbw_set_t{};
+				bool go = false;
+				if (!(rel <= tol))
+				{
+					if (compare[b] && !(rel < 0.9 * prev[b]))
+					{
+						++fails[b];
+						if (!(rel <= prev[b])) // worse: back to the iterate before the cycle
+						{
+							undo[b] = 1;
+							any_undo = true;
+							rel = prev[b];
+						}
+					}
+					else if (compare[b])
+						fails[b] = 0;
+					go = fails[b] < rb_max_fails && !undo[b];
+				}
+				compare[b] = go;
+				prev[b] = rel;
+				h_res[b] = rel;
+				all = all && rel <= tol;
+				final_res = std::max(final_res, std::isnan(rel) ? 1e300 : rel);
+				if (go)
+				{
+					hs[b].est = rel;
+					hs[b].scale = beta;
+					hs[b].live = 1;
+					hs[b].fails = fails[b];
+					any_live = true;
+				}
+			}
+			if (any_undo)
+			{
+				write_dev(c, ws.undo.get(), undo);
+				k_rbw_undo<<<ceil_div(S.nU * B, sblock), sblock, 0, c.stream>>>(S.nU * B, B, ws.keep.get(), ws.x.get(),
+																				ws.undo.get());
+				ESL_HIP(hipGetLastError());
+				ESL_HIP(hipStreamSynchronize(c.stream));
+				bool more = false;
+				for (int b = 0; b < B; ++b)
+				{
+					compare[b] = 0; // every set's residual is taken again before the next cycle
+					more = more || (h_res[b] > tol && fails[b] < rb_max_fails);
+				}
+				if (more)
+					continue;
+			}
+			if (all || !any_live || iters >= max_iters)
+				return all;
+			++cycles;
+			write_dev(c, ws.st.get(), hs);
+			const rbw_set_t* st = ws.st.get();
+			rows(nbE, 0, false, [](auto w) { return k_rbw_te0<decltype(w)::value>; }, G, geo, cc, ws.res.get(), TE, st);
+			rows(nbR, 2, true, [](auto w) { return k_rbw_init<decltype(w)::value>; }, G, geo, cc, ws.res.get(), TE, R, RH, P, X, st, ws.part.get());
+			k_rbw_reduce<1><<<B, sblock, 0, c.stream>>>(ws.part.get(), nbR, B, ws.st.get(), nullptr, nullptr, 0.0);
+			ESL_HIP(hipGetLastError());
+			for (int j = 0; 2 * j < rb_cycle_products; ++j)
+			{
+				iteration(j, rb_aim * tol);
+				iters += 2;
+				if (j > 0 && !live_after(j - 1))
+				{
+					iters -= 2; // every set had stopped before iteration j
+					break;
+				}
+				if (iters >= max_iters)
+					break;
+			}
+			rows(nbR, 0, false, [](auto w) { return k_rbw_correct<decltype(w)::value, true>; }, G, geo, cc, ws.res.get(), X, ws.x.get(), ws.keep.get(), st);
+			rows(nbE, 0, true, [](auto w) { return k_rbw_correct<decltype(w)::value, false>; }, G, geo, cc, ws.res.get(), X, ws.x.get(), ws.keep.get(), st);
+			ESL_HIP(hipGetLastError());
+		}
+	}
+};
+
 // Systems up to this size per set run as one workgroup per set; larger ones
 // device-wide.  Measured on MI355X: 128 sets of 32,724 unknowns take 115 ms per
 // set-workgroup and 50 ms device-wide, 128 sets of 239,616 unknowns 2.4 s and
@@ -3973,7 +4304,7 @@ const bicg_variant_t* reduced_variant(const ctx_t& c, const sys_t& S, const nbr_
 {
 	if (path != path_reduced || o.preconditioner != 0)
 		return nullptr;
-	return rb_variant(nb.nE, nb.nR, nb.rgroups, o.precision, S.B, (size_t)std::min(c.lds_per_block, 160 * 1024));
+	return rb_variant(nb.nE, nb.nR, nb.rgroups, S.B, (size_t)std::min(c.lds_per_block, 160 * 1024));
 }
 
 // one launch: the solve of every set, one workgroup per set (no host synchronisation)
@@ -3990,13 +4321,13 @@ void launch_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, int n_seg, 
 	const double by = gmres_set_bytes(S, nb.nnz);
 	if (const bicg_variant_t* v = reduced_variant(c, S, nb, o, path))
 	{
-		const size_t lds = rb_lds_bytes(S.nU, nb.rgroups, o.precision, v->lrec);
-		const bicg_set_fn fn = v->fn[o.precision == 1];
+		const size_t lds = rb_lds_bytes(S.nU, nb.rgroups, v->lrec);
+		const bicg_set_fn fn = v->fn;
 		if (lds > 48 * 1024)
 			ESL_HIP(hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
 		const rb_scratch_t sp{ sc.r, sc.udiag, sc.t, sc.xk };
-		timed_launch(c, o.precision == 1 ? "k_bicg_set<float>" : "k_bicg_set<double>", by, [&] {
-			fn<<<B, v->blk, lds, c.stream>>>(S, nb.rview(), nseg1, rhs, z, sp, o.tol, o.max_iters, po, o.inner_rtol);
+		timed_launch(c, "k_bicg_set", by, [&] {
+			fn<<<B, v->blk, lds, c.stream>>>(S, nb.rview(), nseg1, rhs, z, sp, o.tol, o.max_iters, po);
 		});
 		ESL_HIP(hipGetLastError());
 		return;
@@ -4193,6 +4524,7 @@ struct plan_t
 	dbuf<double> p0, p1, invd, rhs, z, y, segsum;
 	dbuf<int32_t> anchor;
 	per_set_scratch_t scr;
+	rbw_ws_t wide_ws; // device-wide reduced solver
 	// the buffers the run being enqueued uses: the ones above (plan_reserve), or
 	// slices of the library's static scratch (plan_run_noalloc)
 	struct run_bufs_t
@@ -4286,10 +4618,24 @@ int dw_restart(int requested, int64_t nU, int cb)
 	return m;
 }
 
-// throw_on_miss = false leaves sets above the tolerance to the caller (kr.missed)
+// what the device-wide reduced solver sets up by itself: anchors [B][n_seg], and
+// from them 1 / D' and the right-hand side that other methods and checks read
+struct rb_setup_t
+{
+	const double* x0;
+	const int32_t* seg_off;
+	int n_seg;
+	int32_t* anchor;
+	double *invd, *rhs;
+};
+
+// throw_on_miss = false leaves sets above the tolerance to the caller (kr.missed);
+// cold: the reduced solver starts from the rates (rhs, z and S.invd need no values)
 krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* rhs_p, double* z_p,
 							 const esl_solve_opts& opts, const nbr_store_t* prebuilt = nullptr, bool device_wide = false,
-							 bool throw_on_miss = true, std::vector<double>* set_res = nullptr)
+							 bool throw_on_miss = true, std::vector<double>* set_res = nullptr,
+							 int path = path_reduced, rbw_ws_t* plan_ws = nullptr,
+							 const rb_setup_t* cold = nullptr)
 {
 	krylov_result_t kr;
 	const int64_t nU = S.nU;
@@ -4297,6 +4643,8 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 	const double tol = opts.tol > 0 ? opts.tol : 1e-13;
 	const int max_iters = opts.max_iters > 0 ? opts.max_iters : 20000;
 	const int restart = std::min(std::max(opts.restart > 0 ? opts.restart : 32, 2), dw_max);
+	if (opts.restart > 0 && path == path_reduced)
+		path = path_lds;
 	if (!device_wide && nU <= per_set_max_unknowns(B))
 	{
 		const int m = std::min(restart, pm_max);
@@ -4309,7 +4657,6 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 		o.tol = tol;
 		o.max_iters = max_iters;
 		o.restart = m;
-		const int path = opts.restart <= 0 ? path_reduced : path_lds;
 		const bool reduced = reduced_variant(c, S, nb, o, path) != nullptr;
 		sc.reserve(B, nU, m, opts.precision, reduced);
 		launch_per_set(c, S, nb, n_seg, rhs_p, z_p, o, sc.view(), path);
@@ -4345,7 +4692,36 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 			int it = 0, cy = 0;
 			std::vector<double> cres;
 			double cmax = 0.0;
-			if (opts.precision == 1)
+			const bool reduced = path == path_reduced && opts.preconditioner == 0;
+			if (reduced)
+			{
+				rbw_ws_t own;
+				rbw_ws_t& ws = plan_ws ? *plan_ws : own;
+				bicg_w_t gm(c, Sc, nb, ws, nseg1);
+				if (cold)
+				{
+					gm.enter(cold->x0, cold->seg_off, cold->n_seg, cold->anchor + (int64_t)b0 * nseg1);
+					k_rhs<<<dim3(ceil_div(nU, sblock), cb), sblock, 0, c.stream>>>(Sc, nseg1, cold->x0,
+																				   cold->rhs + (int64_t)b0 * nU);
+				}
+				else
+					gm.enter(rhs_c, z_c);
+				done = gm.solve(tol, max_iters);
+				gm.leave(z_c, cold ? cold->invd + (int64_t)b0 * nU : nullptr);
+				cres = std::move(gm.h_res);
+				cmax = gm.final_res;
+				it = gm.iters;
+				cy = gm.cycles;
+				if (!done)
+				{
+					// sets that stalled: GMRES below, which needs the room
+					ESL_HIP(hipStreamSynchronize(c.stream));
+					ws.reset();
+					if (opts.precision == 1)
+						kr.fp64_fallback += cb;
+				}
+			}
+			else if (opts.precision == 1)
 			{
 				gmres_w_t<float> gm(c, Sc, nb, nseg1, dw_restart(opts.restart, nU, cb), ilu);
 				gm.enter(rhs_c, z_c);
@@ -4814,6 +5190,14 @@ int run_path(const plan_t& P, const esl_solve_opts& o)
 	return o.restart <= 0 ? path_reduced : path_lds;
 }
 
+// whether a run is per set (one workgroup per rate set) or device-wide
+bool runs_per_set(const plan_t& P, int B, bool tuned)
+{
+	if (P.nU == 0 || (tuned && P.tune.path != path_wide && P.tune.path != path_reduced))
+		return true;
+	return !(tuned && P.tune.path == path_wide) && P.nU <= per_set_max_unknowns(B);
+}
+
 // whether a per-set run of the plan takes the reduced solver
 bool plan_reduced(const ctx_t& c, const plan_t& P, int B, const esl_solve_opts& o)
 {
@@ -4851,7 +5235,8 @@ void plan_reserve_(plan_t& P, int B, int m, int precision, bool reduced)
 	P.z.ensure((size_t)B * nU);
 	P.y.ensure((size_t)B * std::max(P.Tr, 1));
 	P.segsum.ensure((size_t)B * std::max(P.n_seg, 1));
-	P.scr.reserve(B, nU, m, precision, reduced);
+	if (m > 0) // 0: the device-wide solvers keep their own buffers
+		P.scr.reserve(B, nU, m, precision, reduced);
 	P.use_own_bufs();
 }
 
@@ -5049,11 +5434,11 @@ void plan_run(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_final
 	// would add their creation and one more host round trip to every solve
 	const auto t_start = std::chrono::steady_clock::now();
 	const bool tuned = o.restart == 0 && P.tune.set;
-	if (tuned)
+	if (tuned && P.tune.path != path_reduced)
 		o.restart = P.tune.m;
 	P.path = run_path(P, o_in);
 	const int m = std::min(std::max(o.restart > 0 ? o.restart : 32, 2), pm_max);
-	const bool per_set = P.nU == 0 || (tuned ? P.tune.path != 2 : P.nU <= per_set_max_unknowns(B));
+	const bool per_set = runs_per_set(P, B, tuned);
 	rep.terminals_reached = P.Tr;
 	rep.unknowns = P.nU;
 	rep.reachable = -1;
@@ -5128,10 +5513,14 @@ void plan_run(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_final
 	else
 	{
 		// one large system: device-wide GMRES (host-driven restarts)
-		plan_reserve(P, B, 2, 0, true);
-		plan_enqueue_setup(c, P, B, d_rates, o);
+		plan_reserve(P, B, 0, 0, true);
+		const rb_setup_t cold{ P.x0.get(), P.d_seg_off.get(), P.n_seg, P.rb.anchor, P.rb.invd, P.rb.rhs };
+		const bool reduced = P.path == path_reduced && o.preconditioner == 0 && o.warm_pi == nullptr;
+		if (!reduced)
+			plan_enqueue_setup(c, P, B, d_rates, o);
 		set_results_t sr;
-		kr = krylov_solve(c, P.sys(B, d_rates), P.n_seg, P.rb.rhs, P.rb.z, o, &P.nbr, true, false, &sr.res);
+		kr = krylov_solve(c, P.sys(B, d_rates), P.n_seg, P.rb.rhs, P.rb.z, o, &P.nbr, true, false, &sr.res, P.path,
+						  &P.wide_ws, reduced ? &cold : nullptr);
 		plan_enqueue_post(c, P, B, d_rates, d_final);
 		if ((int)sr.res.size() != B)
 			sr.res = set_residuals(c, P.sys(B, d_rates), P.n_seg, P.rb.rhs, P.rb.z);
@@ -5272,11 +5661,11 @@ void plan_solve_noalloc(ctx_t& c, void* p, int B, const double* d_rates, double*
 	if (o.max_iters <= 0)
 		o.max_iters = 20000;
 	const bool tuned = o.restart == 0 && P.tune.set;
-	if (tuned)
+	if (tuned && P.tune.path != path_reduced)
 		o.restart = P.tune.m;
 	const int m = std::min(std::max(o.restart > 0 ? o.restart : 32, 2), pm_max);
 	o.restart = m;
-	const bool per_set = P.nU == 0 || (tuned ? P.tune.path != 2 : P.nU <= per_set_max_unknowns(B));
+	const bool per_set = runs_per_set(P, B, tuned);
 	if (!per_set)
 		throw error(ESL_E_ARG, "the no-allocation solve runs the per-set solvers only; this plan's system (" +
 								   std::to_string(P.nU) + " unknowns per set) needs the device-wide solver");
@@ -5444,7 +5833,7 @@ void plan_solve_many(ctx_t& c, int np, void* const* plans, const int* B, const d
 		const bool tuned = o_in.restart == 0 && P.tune.set;
 		P.path = run_path(P, o_in);
 		po[i].restart = std::min(std::max(tuned ? P.tune.m : (o.restart > 0 ? o.restart : 32), 2), pm_max);
-		if (P.nU == 0 || (tuned ? P.tune.path != 2 : P.nU <= per_set_max_unknowns(B[i])))
+		if (runs_per_set(P, B[i], tuned))
 			conc.push_back(i);
 		else // one large system: its device-wide solver is driven from the host
 			wide.push_back(i);

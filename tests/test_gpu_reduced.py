@@ -2,7 +2,8 @@
 restarted GMRES with ILU(0) on the full one, which an explicit restart length
 asks for: systems of 8 to 3,944 unknowns, so that every workgroup size and the
 rows past a workgroup's last full one are met; one set per compute unit and
-more; both precisions."""
+more; both precisions.  And the same method device-wide on larger systems, for odd
+and even batches within and beyond one block's sets, from a warm start too."""
 import numpy as np
 import pytest
 
@@ -62,3 +63,32 @@ def test_reduced_matches_gmres(ctx, unknowns, B, precision):
         red2 = DeviceArray(ctx, (B, n), np.float64)
         p.solve(B, dr.ptr, red2.ptr, precision=precision, tol=1e-12, graph=graph)
         np.testing.assert_array_equal(red2.download(), x)
+
+
+# terminal segment of 12 states and 12,256 undecided ones (its first cycle breaks down
+# for some rate sets); 32,768 terminal states; 32,636 undecided between four attractors
+WIDE = {12268: (2, 14, 5, 0), 32768: (0, 15, 0, 5), 32636: (0, 15, 1, 5)}
+
+
+@pytest.mark.parametrize("unknowns", sorted(WIDE))
+@pytest.mark.parametrize("B", [1, 2, 3, 70, 131])
+def test_device_wide_reduced_matches_gmres(ctx, unknowns, B):
+    p, dr, n = kept(ctx, *WIDE[unknowns], B)
+    assert p.info()["unknowns"] == unknowns
+    red, ref = DeviceArray(ctx, (B, n), np.float64), DeviceArray(ctx, (B, n), np.float64)
+    p.set_schedule(2, 32)  # device-wide GMRES, to 1e-13: at 1e-12 it is itself 1.5e-10 off on one of these
+    p.solve(B, dr.ptr, ref.ptr, precision=0, tol=1e-13)
+    p.set_schedule(-1)
+    y = ref.download()
+    for precision in (0, 1):
+        rep = p.solve(B, dr.ptr, red.ptr, precision=precision, tol=1e-12)
+        assert rep["residual"] <= 1e-12 and rep["exact_solves"] == 0
+        x = red.download()
+        assert np.abs(x - y).sum(axis=1).max() <= 1e-10
+        assert np.abs(x.sum(axis=1) - 1.0).max() <= 1e-11
+    # a warm start from the answer converges at once and to the same vectors
+    nt = p.info()["n_t"]
+    warm = DeviceArray(ctx, (B, nt), np.float64)
+    p.gather_terminal(B, red.ptr, warm.ptr)
+    rep = p.solve(B, dr.ptr, ref.ptr, precision=0, tol=1e-12, warm=warm.ptr)
+    assert np.abs(ref.download() - x).sum(axis=1).max() <= 1e-10
