@@ -307,7 +307,8 @@ esl_status esl_plan_set_schedule(esl_plan* p, int schedule, int restart);
  * n_sets[i] rate sets d_rates[i] -> d_final[i]; the per-set solves of all plans run
  * concurrently on forked streams (opts->graph = 1: captured once as one HIP graph and
  * replayed while plans, sizes, pointers and options stay the same).  Plans whose system
- * needs the device-wide solver run one after another first.  reports[n_plans].
+ * needs the device-wide solver run beside them, each on a host thread of its own; nothing
+ * is captured then.  reports[n_plans].
  * No reference counterpart (the reference solves one network per process); it serves
  * batches over several networks. */
 esl_status esl_plan_solve_many(esl_ctx* ctx, int n_plans, esl_plan* const* plans, const int* n_sets,

@@ -44,6 +44,7 @@
 // while the sets stream through.
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -4503,6 +4504,12 @@ krylov_result_t finish_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, 
 // everything a solve needs that does not depend on the rates
 struct plan_t
 {
+	static uint64_t next_id()
+	{
+		static std::atomic<uint64_t> n{ 0 };
+		return ++n;
+	}
+	const uint64_t id = next_id();
 	graph_t* g = nullptr;
 	dbuf<double> x0;
 	dbuf<uint8_t> reach;
@@ -5723,7 +5730,7 @@ void plan_solve_noalloc(ctx_t& c, void* p, int B, const double* d_rates, double*
 // concurrently on forked streams, optionally captured as one HIP graph
 struct multi_graph_t
 {
-	std::vector<void*> plans;
+	std::vector<uint64_t> plans; // plan_t::id: an address may name another plan later
 	std::vector<int> B;
 	std::vector<const double*> rates;
 	std::vector<double*> fin;
@@ -5838,6 +5845,12 @@ void plan_solve_many(ctx_t& c, int np, void* const* plans, const int* B, const d
 		else // one large system: its device-wide solver is driven from the host
 			wide.push_back(i);
 	}
+	// No capture beside the host threads below, which allocate and free: a program
+	// that alternates between such batches would capture anew on every call while
+	// they run (one such run ended in a host segmentation fault), and what a replay
+	// saves is microseconds beside milliseconds of device-wide solves.
+	if (!wide.empty())
+		o.graph = 0;
 	// the device-wide plans, each on a host thread of its own, joined before return
 	std::vector<std::unique_ptr<child_ctx_t>> kids;
 	for (size_t k = 0; k < wide.size(); ++k)
@@ -5917,7 +5930,7 @@ void many_per_set(ctx_t& c, const std::vector<int>& conc, void* const* plans, co
 		multi_graph_t key;
 		for (int i : conc)
 		{
-			key.plans.push_back(plans[i]);
+			key.plans.push_back(static_cast<plan_t*>(plans[i])->id);
 			key.B.push_back(B[i]);
 			key.rates.push_back(d_rates[i]);
 			key.fin.push_back(d_final[i]);
