@@ -225,13 +225,75 @@ constexpr double rb_aim = 0.1;
 constexpr int rb_max_fails = 3;		 // cycles without progress before a set is left to GMRES
 constexpr int rb_cycle_products = 500; // products by S per cycle, so that rounding cannot drift for long
 
+// What a solve that starts from the rates alone sets up by itself: the anchors
+// [B][n_seg], and from them 1 / D' and the right-hand side that other methods and
+// checks read.
+struct rb_setup_t
+{
+	const double* x0; // [2^N]; null: anchors, 1 / D', right-hand side and start vector are given
+	const int32_t* seg_off;
+	int n_seg;
+	int32_t* anchor;
+	double *invd, *rhs;
+	const double* warm;	 // [B][n_t] predicted final vectors on the terminal states, or null
+	const int32_t* tpos; // terminal unknown -> its place there
+	int64_t n_t;
+	// mass that the sweeps start from on a terminal unknown
+	__device__ __forceinline__ double mass(int b, int32_t u) const
+	{
+		return warm ? fmax(warm[(int64_t)b * n_t + tpos[u]], 0.0) : 1.0;
+	}
+};
+
+// Anchor sweeps: damped Jacobi sweeps (as in k_anchor_sweep) taken class by class.
+// E rows: m = inflow / D; R rows: m = (m + inflow / D) / 2.  One pair moves the mass
+// as far as two sweeps over all rows, so half as many do.  They start from equal
+// masses or from a prediction, which they smooth (a stationary vector stays as it is).
+// Inside the solve kernel, on the records it holds anyway, they and the set-up cost
+// 10 us of its 98 (one set of 1,022 unknowns) where the anchor kernel took 78 and the
+// set-up 6; 250 sets of 2,048 unknowns: 0 of 384 against 180 and 10.
+constexpr int rb_sweeps = 16;
+
+// the largest mass of the workgroup and its unknown, ties to the smallest unknown
+template <int BLK>
+__device__ __forceinline__ void rb_block_argmax(double& v, int32_t& u, double* s_v, int32_t* s_u)
+{
+#pragma unroll
+	for (int o = wave / 2; o > 0; o >>= 1)
+	{
+		const double v2 = __shfl_xor(v, o, wave);
+		const int32_t u2 = __shfl_xor(u, o, wave);
+		if (v2 > v || (v2 == v && u2 < u))
+		{
+			v = v2;
+			u = u2;
+		}
+	}
+	if constexpr (BLK > wave)
+	{
+		__syncthreads();
+		if (lane_id() == 0)
+		{
+			s_v[threadIdx.x / wave] = v;
+			s_u[threadIdx.x / wave] = u;
+		}
+		__syncthreads();
+		for (int w = 0; w < BLK / wave; ++w)
+			if (s_v[w] > v || (s_v[w] == v && s_u[w] < u))
+			{
+				v = s_v[w];
+				u = s_u[w];
+			}
+	}
+}
+
 // One workgroup of BLK threads solves one rate set; thread t owns the rows
 // t + i BLK (i < RPT) of both classes.  LREC: the coupling records are copied to
 // LDS, else they are read from global memory (shared by all sets, so from L2).
 template <int BLK, int RPT, bool LREC>
 __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int n_seg, const double* __restrict__ rhs,
-											  double* __restrict__ zio, const rb_scratch_t& sc, double tol,
-											  int max_iters, const pgm_out_t& out)
+											  double* __restrict__ zio, const rb_scratch_t& sc,
+											  const rb_setup_t& su, double tol, int max_iters, const pgm_out_t& out)
 {
 	extern __shared__ __align__(16) unsigned char smem[];
 	__shared__ double s_part[2][rb_part];
@@ -262,45 +324,182 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 	uint32_t hE[RPT], hR[RPT];
 	double cE[RPT], dR[RPT], jR[RPT];
 	double bb = 0.0;
+	auto groups_of = [&](int q) { return (uint32_t)G.ptr[q] | (uint32_t)(G.ptr[q + 1] - G.ptr[q]) << 24; };
+	if (su.x0)
+	{
+		// from the rates alone: the anchor of a segment is its row of largest mass
+		// after the sweeps, and the masses relative to it are the start vector (a start
+		// from the anchor alone leaves a residual with one or two nonzeros, on which
+		// the first cycle breaks down); undecided states start from zero
+		int32_t uE[RPT], uR[RPT], kE[RPT], kR[RPT];
+		__syncthreads(); // the rates
+#pragma unroll
+		for (int i = 0; i < RPT; ++i)
+		{
+			const int e = tid + i * BLK;
+			hE[i] = hR[i] = 0;
+			cE[i] = dR[i] = 0.0;
+			kE[i] = kR[i] = -1;
+			if (e < nE)
+			{
+				uE[i] = G.row[e];
+				kE[i] = S.ucls[uE[i]];
+				const uint32_t st = (uint32_t)S.ulist[uE[i]];
+				cE[i] = 1.0 / out_rate_s(st, S.mask[st], s_rates);
+				hE[i] = groups_of(e);
+			}
+			if (e < nR)
+			{
+				uR[i] = G.row[nE + e];
+				kR[i] = S.ucls[uR[i]];
+				const uint32_t st = (uint32_t)S.ulist[uR[i]];
+				dR[i] = out_rate_s(st, S.mask[st], s_rates);
+				hR[i] = groups_of(nE + e);
+				s_g[e] = kR[i] >= 0 ? su.mass(b, uR[i]) : 0.0;
+			}
+		}
+		__syncthreads();
+		for (int it = 0; it < (su.n_seg ? rb_sweeps : 0); ++it)
+		{
+#pragma unroll
+			for (int i = 0; i < RPT; ++i)
+				if (tid + i * BLK < nE)
+					s_te[tid + i * BLK] = cE[i] * rb_sum(rec, s_rates, hE[i], s_g, 0.0);
+			__syncthreads();
+#pragma unroll
+			for (int i = 0; i < RPT; ++i)
+				if (tid + i * BLK < nR)
+				{
+					const int o = tid + i * BLK;
+					s_g[o] = 0.5 * s_g[o] + 0.5 * (rb_sum(rec, s_rates, hR[i], s_te, 0.0) / dR[i]);
+				}
+			__syncthreads();
+		}
+		// undecided states
+#pragma unroll
+		for (int i = 0; i < RPT; ++i)
+		{
+			const int e = tid + i * BLK;
+			if (e < nE && kE[i] < 0)
+			{
+				const double r = su.x0[S.ulist[uE[i]]];
+				su.invd[off + uE[i]] = cE[i];
+				su.rhs[off + uE[i]] = bp[e] = r;
+				xp[e] = 0.0;
+				bb += r * r;
+			}
+			if (e < nR && kR[i] < 0)
+			{
+				const double r = su.x0[S.ulist[uR[i]]];
+				su.invd[off + uR[i]] = 1.0 / dR[i];
+				su.rhs[off + uR[i]] = bp[nE + e] = r;
+				xp[nE + e] = 0.0;
+				bb += r * r;
+			}
+		}
+		// segments
+		for (int k = 0; k < su.n_seg; ++k)
+		{
+			double best = -1.0;
+			int32_t bu = INT32_MAX;
+#pragma unroll
+			for (int i = 0; i < RPT; ++i)
+			{
+				const int e = tid + i * BLK;
+				if (kE[i] == k && (s_te[e] > best || (s_te[e] == best && uE[i] < bu)))
+				{
+					best = s_te[e];
+					bu = uE[i];
+				}
+				if (kR[i] == k && (s_g[e] > best || (s_g[e] == best && uR[i] < bu)))
+				{
+					best = s_g[e];
+					bu = uR[i];
+				}
+			}
+			rb_block_argmax<BLK>(best, bu, s_part[0], (int32_t*)s_part[1]);
+			if (tid == 0)
+				su.anchor[(int64_t)b * su.n_seg + k] = bu;
+			const double inv = best > 0.0 ? 1.0 / best : 0.0;
+#pragma unroll
+			for (int i = 0; i < RPT; ++i)
+			{
+				const int e = tid + i * BLK;
+				if (kE[i] == k)
+				{
+					const bool anc = uE[i] == bu;
+					if (anc)
+					{
+						hE[i] = 0;
+						cE[i] = 1.0;
+						bb += 1.0;
+					}
+					xp[e] = anc ? 1.0 : s_te[e] * inv;
+					su.invd[off + uE[i]] = cE[i];
+					su.rhs[off + uE[i]] = bp[e] = anc ? 1.0 : 0.0;
+				}
+				if (kR[i] == k)
+				{
+					const bool anc = uR[i] == bu;
+					if (anc)
+					{
+						hR[i] = 0;
+						dR[i] = 1.0;
+						bb += 1.0;
+					}
+					xp[nE + e] = anc ? 1.0 : s_g[e] * inv;
+					su.invd[off + uR[i]] = 1.0 / dR[i];
+					su.rhs[off + uR[i]] = bp[nE + e] = anc ? 1.0 : 0.0;
+				}
+			}
+		}
+		__syncthreads();
+	}
+	else
+	{
+#pragma unroll
+		for (int i = 0; i < RPT; ++i)
+		{
+			const int e = tid + i * BLK;
+			hE[i] = hR[i] = 0;
+			cE[i] = dR[i] = 0.0;
+			for (int cls = 0; cls < 2; ++cls)
+			{
+				if (e >= (cls ? nR : nE))
+					continue;
+				const int q = cls ? nE + e : e, u = G.row[q];
+				const uint32_t h = is_anchor(S, n_seg, b, u) ? 0u : groups_of(q);
+				const double iv = S.invd[off + u], r = rhs[off + u];
+				if (cls)
+				{
+					hR[i] = h;
+					dR[i] = 1.0 / iv;
+				}
+				else
+				{
+					hE[i] = h;
+					cE[i] = iv;
+				}
+				xp[q] = zio[off + u] * iv;
+				bp[q] = r;
+				bb += r * r;
+			}
+		}
+		__syncthreads();
+	}
+	// diag(S): D less what leaves the row and comes straight back (not through an
+	// anchor, whose row takes nothing in)
 #pragma unroll
 	for (int i = 0; i < RPT; ++i)
-	{
-		const int e = tid + i * BLK;
-		hE[i] = 0;
-		cE[i] = 0.0;
-		if (e < nE)
-		{
-			const int u = G.row[e];
-			const bool anc = is_anchor(S, n_seg, b, u);
-			const int g0 = G.ptr[e];
-			hE[i] = anc ? 0u : (uint32_t)g0 | (uint32_t)(G.ptr[e + 1] - g0) << 24;
-			cE[i] = S.invd[off + u];
-			xp[e] = zio[off + u] * cE[i];
-			const double r = rhs[off + u];
-			bp[e] = r;
-			bb += r * r;
-			s_te[e] = anc ? 0.0 : cE[i];
-		}
-	}
+		if (tid + i * BLK < nE)
+			s_te[tid + i * BLK] = hE[i] >> 24 ? cE[i] : 0.0;
 	__syncthreads();
 #pragma unroll
 	for (int i = 0; i < RPT; ++i)
 	{
-		const int o = tid + i * BLK;
-		hR[i] = 0;
-		dR[i] = jR[i] = 0.0;
-		if (o < nR)
+		jR[i] = 0.0;
+		if (tid + i * BLK < nR)
 		{
-			const int u = G.row[nE + o];
-			const int g0 = G.ptr[nE + o];
-			hR[i] = is_anchor(S, n_seg, b, u) ? 0u : (uint32_t)g0 | (uint32_t)(G.ptr[nE + o + 1] - g0) << 24;
-			const double iv = S.invd[off + u];
-			dR[i] = 1.0 / iv;
-			xp[nE + o] = zio[off + u] * iv;
-			const double r = rhs[off + u];
-			bp[nE + o] = r;
-			bb += r * r;
-			// diag(S): D less what leaves the row and comes straight back
 			double d = dR[i];
 			const int g1 = (int)(hR[i] & 0xffffff) + (int)(hR[i] >> 24);
 			for (int g = (int)(hR[i] & 0xffffff); g < g1; ++g)
@@ -542,13 +741,13 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 
 template <int BLK, int RPT, bool LREC>
 __global__ __launch_bounds__(BLK, 4) void k_bicg_set(
-	sys_t S, rb_t G, int n_seg, const double* __restrict__ rhs, double* __restrict__ zio, rb_scratch_t sc, double tol,
-	int max_iters, pgm_out_t out)
+	sys_t S, rb_t G, int n_seg, const double* __restrict__ rhs, double* __restrict__ zio, rb_scratch_t sc, rb_setup_t su,
+	double tol, int max_iters, pgm_out_t out)
 {
-	bicg_set_body<BLK, RPT, LREC>(S, G, n_seg, rhs, zio, sc, tol, max_iters, out);
+	bicg_set_body<BLK, RPT, LREC>(S, G, n_seg, rhs, zio, sc, su, tol, max_iters, out);
 }
 
-using bicg_set_fn = void (*)(sys_t, rb_t, int, const double*, double*, rb_scratch_t, double, int, pgm_out_t);
+using bicg_set_fn = void (*)(sys_t, rb_t, int, const double*, double*, rb_scratch_t, rb_setup_t, double, int, pgm_out_t);
 struct bicg_variant_t
 {
 	bicg_set_fn fn;
@@ -744,11 +943,11 @@ struct rbw_set_t
 
 // ---- start
 
-// c = 1 / D of every row, and the masses the anchor sweeps start from (1 on
-// terminal rows, 0 on ambiguous ones)
+// c = 1 / D of every row, and the masses the anchor sweeps start from (0 on
+// ambiguous rows)
 template <int W>
-__global__ void k_rbw_coef(sys_t S, rb_t G, rbw_geo_t geo, double* __restrict__ c, double* __restrict__ mE,
-						   double* __restrict__ mR)
+__global__ void k_rbw_coef(sys_t S, rb_t G, rbw_geo_t geo, rb_setup_t su, double* __restrict__ c,
+						   double* __restrict__ mE, double* __restrict__ mR)
 {
 	const double* rt = rbw_lds_rates(geo);
 	ESL_RBW_THREAD;
@@ -772,17 +971,14 @@ __global__ void k_rbw_coef(sys_t S, rb_t G, rbw_geo_t geo, double* __restrict__ 
 		for (int w = 0; w < W; ++w)
 		{
 			d.v[w] = 1.0 / d.v[w];
-			m.v[w] = S.ucls[u] >= 0 ? 1.0 : 0.0;
+			m.v[w] = S.ucls[u] >= 0 ? su.mass(b + w, u) : 0.0;
 		}
 		rbw_store<W>(c + q * B + b, d);
 		rbw_store<W>((q < G.nE ? mE + q * B : mR + (q - G.nE) * B) + b, m);
 	}
 }
 
-// Anchor sweeps: the damped Jacobi sweeps of k_anchor_sweep taken class by class.
-// E rows: m = inflow / D; R rows: m = (m + inflow / D) / 2.  One pair moves the mass
-// as far as two sweeps over all rows, so half as many do.
-constexpr int rbw_sweeps = 16;
+// one class of an anchor sweep (rb_sweeps)
 template <int W, bool KEPT>
 __global__ void k_rbw_sweep(rb_t G, rbw_geo_t geo, const double* __restrict__ c, const double* __restrict__ from,
 							double* __restrict__ to)
@@ -968,7 +1164,7 @@ __global__ void k_rbw_start(sys_t S, rb_t G, rbw_geo_t geo, int n_seg, const dou
 
 constexpr int rbw_tile = 32; // rows (and sets) of a transposed tile
 
-// the warm start's counterpart: plan vectors (set-major) -> solver vectors, through
+// or from a system that is set up: plan vectors (set-major) -> solver vectors, through
 // LDS tiles so that both sides are read and written along their rows
 __global__ __launch_bounds__(sblock) void k_rbw_enter(sys_t S, rb_t G, int n_seg, const double* __restrict__ rhs,
 													  const double* __restrict__ z, double* __restrict__ wx,

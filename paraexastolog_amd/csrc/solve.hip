@@ -3920,12 +3920,13 @@ struct bicg_w_t
 
 	// set-up from the rates alone: coefficients, anchors (into anchor[b][seg]), start
 	// vector and right-hand side
-	void enter(const double* x0, const int32_t* seg_off, int segs, int32_t* anchor)
+	void enter(const rb_setup_t& su)
 	{
-		rows(nbU, 0, true, [](auto w) { return k_rbw_coef<decltype(w)::value>; }, S, G, geo, ws.c.get(), TE, P);
+		const int segs = su.n_seg;
+		rows(nbU, 0, true, [](auto w) { return k_rbw_coef<decltype(w)::value>; }, S, G, geo, su, ws.c.get(), TE, P);
 		if (segs)
 		{
-			for (int it = 0; it < rbw_sweeps; ++it)
+			for (int it = 0; it < rb_sweeps; ++it)
 			{
 				timed_launch(c, "k_rbw_sweep", 24.0 * G.nE * B, [&] {
 					rows(nbE, 0, true, [](auto w) { return k_rbw_sweep<decltype(w)::value, false>; }, G, geo, ws.c.get(), P, TE);
@@ -3934,7 +3935,7 @@ struct bicg_w_t
 					rows(nbR, 0, true, [](auto w) { return k_rbw_sweep<decltype(w)::value, true>; }, G, geo, ws.c.get(), TE, P);
 				});
 			}
-			k_rbw_seg_rows<<<ceil_div(segs + 1, sblock), sblock, 0, c.stream>>>(G, segs, seg_off, ws.seg_rows.get());
+			k_rbw_seg_rows<<<ceil_div(segs + 1, sblock), sblock, 0, c.stream>>>(G, segs, su.seg_off, ws.seg_rows.get());
 			const int nt = geo.L * geo.R;
 			const size_t lds = (size_t)W * nt * 12;
 			const dim3 gp(slices * segs, chunks);
@@ -3945,9 +3946,9 @@ struct bicg_w_t
 				k_rbw_pick<1><<<gp, nt, lds, c.stream>>>(G, geo, segs, slices, ws.seg_rows.get(), TE, P, ws.pick_v.get(),
 														 ws.pick_u.get());
 			k_rbw_anchor<<<ceil_div(segs * B, sblock), sblock, 0, c.stream>>>(B, segs, slices, ws.pick_v.get(),
-																			   ws.pick_u.get(), anchor, ws.pa.get());
+																			   ws.pick_u.get(), su.anchor, ws.pa.get());
 		}
-		rows(nbU, 0, false, [](auto w) { return k_rbw_start<decltype(w)::value>; }, S, G, geo, n_seg, x0, TE, P, ws.pa.get(), ws.c.get(), ws.x.get(), ws.b.get());
+		rows(nbU, 0, false, [](auto w) { return k_rbw_start<decltype(w)::value>; }, S, G, geo, n_seg, su.x0, TE, P, ws.pa.get(), ws.c.get(), ws.x.get(), ws.b.get());
 		diag();
 	}
 
@@ -4310,8 +4311,9 @@ const bicg_variant_t* reduced_variant(const ctx_t& c, const sys_t& S, const nbr_
 
 // one launch: the solve of every set, one workgroup per set (no host synchronisation)
 // path: the schedule; path_reduced falls back to path_lds where no reduced variant fits
+// su: the reduced solver's set-up from the rates (x0 null: the plan's vectors are set up)
 void launch_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, int n_seg, const double* rhs, double* z,
-					const esl_solve_opts& o, const pss_view_t& sc, int path)
+					const esl_solve_opts& o, const pss_view_t& sc, int path, const rb_setup_t& su = {})
 {
 	const int B = S.B;
 	const int m = std::min(std::max(o.restart > 0 ? o.restart : 32, 2), pm_max);
@@ -4328,7 +4330,7 @@ void launch_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, int n_seg, 
 			ESL_HIP(hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
 		const rb_scratch_t sp{ sc.r, sc.udiag, sc.t, sc.xk };
 		timed_launch(c, "k_bicg_set", by, [&] {
-			fn<<<B, v->blk, lds, c.stream>>>(S, nb.rview(), nseg1, rhs, z, sp, o.tol, o.max_iters, po);
+			fn<<<B, v->blk, lds, c.stream>>>(S, nb.rview(), nseg1, rhs, z, sp, su, o.tol, o.max_iters, po);
 		});
 		ESL_HIP(hipGetLastError());
 		return;
@@ -4599,6 +4601,11 @@ struct plan_t
 	}
 	~plan_t() { drop_graph(); }
 	sys_t sys(int B, const double* rates) const;
+	rb_setup_t setup(const double* warm) const
+	{
+		return rb_setup_t{ x0.get(), d_seg_off.get(), n_seg, rb.anchor, rb.invd, rb.rhs, n_seg ? warm : nullptr, d_tpos.get(),
+						   g->n_t };
+	}
 };
 
 
@@ -4625,24 +4632,13 @@ int dw_restart(int requested, int64_t nU, int cb)
 	return m;
 }
 
-// what the device-wide reduced solver sets up by itself: anchors [B][n_seg], and
-// from them 1 / D' and the right-hand side that other methods and checks read
-struct rb_setup_t
-{
-	const double* x0;
-	const int32_t* seg_off;
-	int n_seg;
-	int32_t* anchor;
-	double *invd, *rhs;
-};
-
 // throw_on_miss = false leaves sets above the tolerance to the caller (kr.missed);
-// cold: the reduced solver starts from the rates (rhs, z and S.invd need no values)
+// setup: the reduced solver sets itself up (rhs, z and S.invd need no values)
 krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* rhs_p, double* z_p,
 							 const esl_solve_opts& opts, const nbr_store_t* prebuilt = nullptr, bool device_wide = false,
 							 bool throw_on_miss = true, std::vector<double>* set_res = nullptr,
 							 int path = path_reduced, rbw_ws_t* plan_ws = nullptr,
-							 const rb_setup_t* cold = nullptr)
+							 const rb_setup_t* setup = nullptr)
 {
 	krylov_result_t kr;
 	const int64_t nU = S.nU;
@@ -4705,16 +4701,20 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 				rbw_ws_t own;
 				rbw_ws_t& ws = plan_ws ? *plan_ws : own;
 				bicg_w_t gm(c, Sc, nb, ws, nseg1);
-				if (cold)
+				if (setup)
 				{
-					gm.enter(cold->x0, cold->seg_off, cold->n_seg, cold->anchor + (int64_t)b0 * nseg1);
-					k_rhs<<<dim3(ceil_div(nU, sblock), cb), sblock, 0, c.stream>>>(Sc, nseg1, cold->x0,
-																				   cold->rhs + (int64_t)b0 * nU);
+					rb_setup_t su = *setup;
+					su.anchor += (int64_t)b0 * nseg1;
+					if (su.warm)
+						su.warm += (int64_t)b0 * su.n_t;
+					gm.enter(su);
+					k_rhs<<<dim3(ceil_div(nU, sblock), cb), sblock, 0, c.stream>>>(Sc, nseg1, su.x0,
+																				   su.rhs + (int64_t)b0 * nU);
 				}
 				else
 					gm.enter(rhs_c, z_c);
 				done = gm.solve(tol, max_iters);
-				gm.leave(z_c, cold ? cold->invd + (int64_t)b0 * nU : nullptr);
+				gm.leave(z_c, setup ? setup->invd + (int64_t)b0 * nU : nullptr);
 				cres = std::move(gm.h_res);
 				cmax = gm.final_res;
 				it = gm.iters;
@@ -5037,6 +5037,15 @@ sys_t plan_t::sys(int B, const double* rates) const
 	return S;
 }
 
+// whether a per-set run of the plan takes the reduced solver
+bool plan_reduced(const ctx_t& c, const plan_t& P, int B, const esl_solve_opts& o)
+{
+	sys_t S{};
+	S.nU = P.nU;
+	S.B = B;
+	return P.nU > 0 && reduced_variant(c, S, P.nbr, o, P.path) != nullptr;
+}
+
 // The numeric part for B rate sets: anchors, coefficients and start vector
 // (setup), the Krylov solves, then absorption masses and the final vector
 // (post).  No host synchronisation inside, so with the per-set solver the whole
@@ -5178,9 +5187,13 @@ void plan_enqueue(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_f
 		c.stream = main;
 		ESL_HIP(hipEventRecord(c.fill_ev[1], c.fill_s));
 	}
-	plan_enqueue_setup(c, P, B, d_rates, o);
+	rb_setup_t su{};
+	if (plan_reduced(c, P, B, o)) // sets itself up
+		su = P.setup(o.warm_pi);
+	else
+		plan_enqueue_setup(c, P, B, d_rates, o);
 	if (P.nU)
-		launch_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, o, P.rb.ps, P.path);
+		launch_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, o, P.rb.ps, P.path, su);
 	if (fork)
 		ESL_HIP(hipStreamWaitEvent(c.stream, c.fill_ev[1], 0));
 	plan_enqueue_post(c, P, B, d_rates, d_final, !fork);
@@ -5203,15 +5216,6 @@ bool runs_per_set(const plan_t& P, int B, bool tuned)
 	if (P.nU == 0 || (tuned && P.tune.path != path_wide && P.tune.path != path_reduced))
 		return true;
 	return !(tuned && P.tune.path == path_wide) && P.nU <= per_set_max_unknowns(B);
-}
-
-// whether a per-set run of the plan takes the reduced solver
-bool plan_reduced(const ctx_t& c, const plan_t& P, int B, const esl_solve_opts& o)
-{
-	sys_t S{};
-	S.nU = P.nU;
-	S.B = B;
-	return P.nU > 0 && reduced_variant(c, S, P.nbr, o, P.path) != nullptr;
 }
 
 // grows the per-run buffers; a captured graph holds their addresses, so any
@@ -5521,13 +5525,13 @@ void plan_run(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_final
 	{
 		// one large system: device-wide GMRES (host-driven restarts)
 		plan_reserve(P, B, 0, 0, true);
-		const rb_setup_t cold{ P.x0.get(), P.d_seg_off.get(), P.n_seg, P.rb.anchor, P.rb.invd, P.rb.rhs };
-		const bool reduced = P.path == path_reduced && o.preconditioner == 0 && o.warm_pi == nullptr;
+		const rb_setup_t su = P.setup(o.warm_pi);
+		const bool reduced = P.path == path_reduced && o.preconditioner == 0;
 		if (!reduced)
 			plan_enqueue_setup(c, P, B, d_rates, o);
 		set_results_t sr;
 		kr = krylov_solve(c, P.sys(B, d_rates), P.n_seg, P.rb.rhs, P.rb.z, o, &P.nbr, true, false, &sr.res, P.path,
-						  &P.wide_ws, reduced ? &cold : nullptr);
+						  &P.wide_ws, reduced ? &su : nullptr);
 		plan_enqueue_post(c, P, B, d_rates, d_final);
 		if ((int)sr.res.size() != B)
 			sr.res = set_residuals(c, P.sys(B, d_rates), P.n_seg, P.rb.rhs, P.rb.z);
