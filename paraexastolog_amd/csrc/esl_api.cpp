@@ -45,7 +45,7 @@ namespace {
 thread_local std::string tl_error;
 
 template <typename F>
-esl_status guarded(esl_ctx* ctx, F&& f)
+esl_status guarded_call(esl_ctx* ctx, F&& f)
 {
 	try
 	{
@@ -67,6 +67,21 @@ esl_status guarded(esl_ctx* ctx, F&& f)
 		(ctx ? ctx->c.last_error : tl_error) = e.what();
 		return ESL_E_ARG;
 	}
+}
+
+// An entry point's body, its device buffers from the pool of its context.  A call
+// that failed may have left work on the device that nothing waits for: its blocks
+// leave the pool (hipFree waits for the device).
+template <typename F>
+esl_status guarded(esl_ctx* ctx, F&& f)
+{
+	if (!ctx)
+		return guarded_call(ctx, f);
+	const esl::pool_scope_t scope(ctx->c.pool);
+	const esl_status s = guarded_call(ctx, f);
+	if (s != ESL_OK)
+		ctx->c.pool->clear(false);
+	return s;
 }
 
 void require(bool cond, int code, const std::string& what)
@@ -170,6 +185,7 @@ void esl_ctx_destroy(esl_ctx* ctx)
 			(void)hipEventDestroy(e);
 	if (ctx->c.stream)
 		(void)hipStreamDestroy(ctx->c.stream);
+	ctx->c.pool->clear(true);
 	delete ctx;
 }
 

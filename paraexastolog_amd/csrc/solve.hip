@@ -5866,6 +5866,7 @@ void plan_solve_many(ctx_t& c, int np, void* const* plans, const int* B, const d
 			try
 			{
 				const int i = wide[k];
+				const pool_scope_t scope(kids[k]->c.pool);
 				ESL_HIP(hipSetDevice(kids[k]->c.device));
 				plan_run(kids[k]->c, *static_cast<plan_t*>(plans[i]), B[i], d_rates[i], d_final[i], o_in, reps[i]);
 			}
