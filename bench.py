@@ -833,7 +833,7 @@ def workload_n22(a, ctx):
 
 
 def surrogate_gemm_rate(L, ctx, sur, X, T, steps=40, batch=512):
-    """Device time of the surrogate's BF16 GEMM kernels over `steps` training
+    """Device time of the surrogate's kernels with BF16 products over `steps` training
     steps (one esl_mlp_train_steps call at learning rate 0, so the trained
     network is left as it is) on minibatches of 512 rows, timed per launch with
     HIP events: the algorithmic 2 M N K flops of every product over the summed
@@ -853,7 +853,7 @@ def surrogate_gemm_rate(L, ctx, sur, X, T, steps=40, batch=512):
     wall = time.perf_counter() - t
     stats = profile_stats(L, ctx)
     check(L.esl_profile(ctx.handle, 0), ctx.handle)
-    g = [x for x in stats if x[0] == "k_gemm_bf16"]
+    g = [x for x in stats if x[0] in ("k_gemm_bf16", "k_mlp_rows", "k_mlp_update")]
     r = [x for x in stats if x[0] == "k_gemm_reduce"]
     launches = sum(x[1] for x in g)
     ms = sum(x[2] for x in g)

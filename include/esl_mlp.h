@@ -9,7 +9,7 @@
  * from the prediction until the FP64 residual meets its tolerance.
  *
  * All products run on the matrix cores (BF16 operands, FP32 accumulation);
- * parameters, activations and Adam moments are FP32.  Device pointers are
+ * parameters, Adam moments and all between two products are FP32.  Device pointers are
  * row-major [rows][features] FP32.
  */
 #ifndef ESL_MLP_H

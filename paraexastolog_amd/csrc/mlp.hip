@@ -22,7 +22,8 @@
 // so the same kernel serves X W, dZ W^T and X^T dZ.  Products with few output
 // tiles and a long K (dZ W^T of the widest layer) are split over gridDim.z;
 // each split writes FP32 partial tiles that k_gemm_reduce sums in split order
-// (deterministic) before the epilogue.  The epilogues (bias + GELU, bias,
+// (deterministic) before the epilogue.  Networks that fit k_mlp_rows (mlp_rows.hip.hpp) run
+// there instead.  The epilogues (bias + GELU, bias,
 // times GELU'(Z)) are fused, and what they read is loaded before the K loop.
 // Register layout of the instruction (wave64): lane l holds
 // A[l % 32][8 (l / 32) + 0..7], B[8 (l / 32) + 0..7][l % 32] and C rows
@@ -450,6 +451,16 @@ __global__ __launch_bounds__(256) void k_colsum(int rows, int n, const float* __
 	}
 }
 
+// the parameter after an Adam step with gradient g; m, v: its moments, replaced.  Fused
+// multiply-adds are spelled out so that every kernel rounds alike.
+__device__ __forceinline__ float adam_step(float p, float g, float& m, float& v, float lr, float b1, float b2, float eps,
+										   float c1, float c2)
+{
+	m = __builtin_fmaf(1.0f - b1, g, b1 * m);
+	v = __builtin_fmaf(g, (1.0f - b2) * g, b2 * v);
+	return p - lr * (m / c1) / (sqrtf(v / c2) + eps);
+}
+
 __global__ __launch_bounds__(256) void k_adam(int64_t count, float* __restrict__ p, const float* __restrict__ g,
 											  float* __restrict__ m, float* __restrict__ v, float lr, float b1,
 											  float b2, float eps, float c1, float c2)
@@ -457,12 +468,10 @@ __global__ __launch_bounds__(256) void k_adam(int64_t count, float* __restrict__
 	const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
 	if (i >= count)
 		return;
-	const float gi = g[i];
-	const float mi = b1 * m[i] + (1.0f - b1) * gi;
-	const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
+	float mi = m[i], vi = v[i];
+	p[i] = adam_step(p[i], g[i], mi, vi, lr, b1, b2, eps, c1, c2);
 	m[i] = mi;
 	v[i] = vi;
-	p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
 }
 
 // out[0] = sum of x (add: out[0] += sum of x)
@@ -479,6 +488,8 @@ __global__ __launch_bounds__(256) void k_sum_f(int n, const float* __restrict__ 
 
 } // namespace esl
 
+#include "mlp_rows.hip.hpp"
+
 // ============================================================================
 // host side
 
@@ -494,6 +505,12 @@ struct esl_mlp
 	esl::dbuf<float> act, pre, dact, probs, dlog, loss_rows, loss;
 	esl::dbuf<float> part;		  // split-K partial tiles of the GEMMs
 	std::vector<int64_t> act_off; // activations of each layer (input copy at 0)
+	// shapes that k_mlp_rows takes
+	bool by_rows = false;
+	esl::mlp_net_t net{};
+	esl::dbuf<short> ops, frag;
+	esl::dbuf<float> dz;
+	bool ops_stale = true; // parameters were set since the operand copies were written
 };
 
 namespace {
@@ -518,6 +535,132 @@ esl_status mlp_guard(esl_ctx* ctx, const std::function<void()>& f)
 			esl::ctx_impl(ctx).last_error = e.what();
 		return ESL_E_ARG;
 	}
+}
+
+// k per partial sum of an M x N product over K: products with few 64 x 64 output
+// tiles and K >= 512 are split along K so that the launch has up to 256 workgroups
+// of at least 256 k each.  K stages (bk) of 128 (32 for short products) keep enough
+// loads in flight per stage that the few stages of these products are not each a full
+// memory latency.
+int gemm_split(int M, int N, int K, int& bk)
+{
+	const int tiles = esl::ceil_div(M, 64) * esl::ceil_div(N, 64);
+	const int splits = std::max(1, std::min({ K / 256, 256 / tiles, esl::gemm_max_splits }));
+	const int kper = esl::ceil_div(K, splits);
+	bk = kper >= 128 ? 128 : 32;
+	return esl::ceil_div(kper, bk) * bk;
+}
+
+// The rule of the two paths: what k_mlp_rows holds of 16 rows has to fit LDS and its
+// registers.  Where it does, it is 2.3 to 2.7 times as fast (figures there).
+void plan_by_rows(esl::ctx_t& c, esl_mlp* m)
+{
+	esl::mlp_net_t& t = m->net;
+	if (m->n_in > esl::mr_width || m->hidden > esl::mr_width || m->layers > esl::mr_layers || m->n_out > esl::mr_out)
+		return;
+	t.n_in = m->n_in, t.hidden = m->hidden, t.layers = m->layers, t.n_out = m->n_out;
+	t.kt0 = esl::ceil_div(m->n_in, 32);
+	t.kth = m->hidden <= 128 ? 4 : 8;
+	t.kto = esl::ceil_div(m->n_out, 32);
+	const size_t lds = esl::mlp_rows_lds(t, 16, true);
+	if (lds > (size_t)c.lds_per_block)
+		return;
+	int64_t off = 0;
+	for (int y = 0; y <= t.layers; ++y)
+	{
+		const int64_t sz = (int64_t)2 * t.in_tiles(y) * t.out_tiles(y) * esl::mr_tile;
+		t.w[y] = m->w_off[y], t.b[y] = m->b_off[y];
+		t.wf[y] = off, off += sz;
+		if (y > 0)
+			t.wb[y] = off, off += sz;
+	}
+	m->ops.ensure(off);
+	t.params = m->params.get();
+	t.ops = m->ops.get();
+	const void* fns[] = {
+#define ESL_ROWS_FN(E, KT, TPW) \
+	(const void*)esl::k_mlp_rows<E, KT, TPW, false>, (const void*)esl::k_mlp_rows<E, KT, TPW, true>
+		ESL_ROWS_FN(1, 4, 2), ESL_ROWS_FN(1, 4, 8), ESL_ROWS_FN(1, 8, 2), ESL_ROWS_FN(1, 8, 8),
+		ESL_ROWS_FN(4, 4, 2), ESL_ROWS_FN(4, 4, 8), ESL_ROWS_FN(4, 8, 2), ESL_ROWS_FN(4, 8, 8)
+#undef ESL_ROWS_FN
+	};
+	for (const void* f : fns)
+		ESL_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+	m->by_rows = true;
+}
+
+// rows through the network and, with targets, back (enqueued)
+void run_rows(esl::ctx_t& c, esl_mlp* m, esl::mlp_batch_t& q)
+{
+	const esl::mlp_net_t& t = m->net;
+	const bool train = q.tg != nullptr;
+	if (m->ops_stale)
+	{
+		int frags = 0;
+		for (int y = 0; y <= t.layers; ++y)
+			frags += (y > 0 ? 2 : 1) * 2 * t.in_tiles(y) * t.out_tiles(y);
+		esl::k_mlp_operands<<<esl::ceil_div(frags, 4), 256, 0, c.stream>>>(t, frags);
+		ESL_HIP(hipGetLastError());
+		m->ops_stale = false;
+	}
+	q.rt = esl::ceil_div(q.rows, 32);
+	if (train)
+	{
+		int64_t off = 0;
+		int bk;
+		q.zc = gemm_split(q.rows, t.hidden, t.n_out, bk) / 32;
+		for (int y = 0; y <= t.layers; ++y)
+		{
+			q.xc[y] = gemm_split(t.rows_of(y), t.cols_of(y), q.rows, bk) / 32;
+			q.xf[y] = off, off += (int64_t)q.rt * 2 * t.in_tiles(y) * esl::mr_tile;
+			q.zf[y] = off, off += (int64_t)q.rt * 2 * t.out_tiles(y) * esl::mr_tile;
+		}
+		m->frag.ensure(off);
+		m->dz.ensure((size_t)q.rows * t.biases());
+		m->loss_rows.ensure(q.rows);
+		m->loss.ensure(1);
+		q.frag = m->frag.get();
+		q.dz = m->dz.get();
+		q.loss_rows = m->loss_rows.get();
+	}
+	// 4 rows per workgroup while that gives no compute unit a second one, else 16
+	const int e = q.rows <= 4 * 256 ? 1 : 4;
+	const int grid = (train ? 32 * q.rt : q.rows + 4 * e - 1) / (4 * e);
+	const size_t lds = esl::mlp_rows_lds(t, 4 * e, train);
+	const double flops = 2.0 * q.rows * (m->n_params - t.biases()) +
+						 (train ? 2.0 * q.rows * (m->n_params - t.biases() - (int64_t)t.n_in * t.hidden) : 0.0);
+	esl::timed_launch(c, "k_mlp_rows", flops, [&] {
+#define ESL_ROWS_T(E, KT, TPW)                                                                 \
+	(train ? esl::k_mlp_rows<E, KT, TPW, true><<<grid, esl::mr_block, lds, c.stream>>>(t, q) \
+		   : esl::k_mlp_rows<E, KT, TPW, false><<<grid, esl::mr_block, lds, c.stream>>>(t, q))
+#define ESL_ROWS(KT, TPW) (e == 1 ? ESL_ROWS_T(1, KT, TPW) : ESL_ROWS_T(4, KT, TPW))
+		const bool few = t.kto * 2 <= 2 * esl::mr_waves;
+		if (t.kth == 4)
+			few ? ESL_ROWS(4, 2) : ESL_ROWS(4, 8);
+		else
+			few ? ESL_ROWS(8, 2) : ESL_ROWS(8, 8);
+#undef ESL_ROWS
+#undef ESL_ROWS_T
+	});
+	ESL_HIP(hipGetLastError());
+}
+
+// after run_rows with targets: the gradients of the mean cross-entropy into m->grads or,
+// with `adam`, one Adam step; the summed loss of the rows into m->loss[0]
+void run_update(esl::ctx_t& c, esl_mlp* m, const esl::mlp_batch_t& q, esl::mlp_adam_t a, bool adam, bool accumulate)
+{
+	const esl::mlp_net_t& t = m->net;
+	a.m1 = m->m1.get(), a.m2 = m->m2.get(), a.grads = m->grads.get(), a.loss = m->loss.get();
+	a.accumulate = accumulate ? 1 : 0;
+	int tiles = 0;
+	for (int y = 0; y <= t.layers; ++y)
+		tiles += 2 * t.in_tiles(y) * t.out_tiles(y);
+	const int grid = esl::ceil_div(tiles, 4) + esl::ceil_div(t.biases(), 32) + 1;
+	esl::timed_launch(c, "k_mlp_update", 2.0 * q.rows * (m->n_params - t.biases()), [&] {
+		adam ? esl::k_mlp_update<true><<<grid, 256, 0, c.stream>>>(t, q, a, tiles)
+			 : esl::k_mlp_update<false><<<grid, 256, 0, c.stream>>>(t, q, a, tiles);
+	});
+	ESL_HIP(hipGetLastError());
 }
 
 void ensure_rows(esl_mlp* m, int rows)
@@ -571,20 +714,13 @@ bool quad_loads(const float* P, int R, int K, int64_t sr, int64_t sk)
 	return sr == 1 && sk % 4 == 0 && R % 4 == 0;
 }
 
-// C = A B with the given epilogue.  Products with few 64 x 64 output tiles and
-// K >= 512 are split along K so that the launch has up to 256 workgroups of at
-// least 256 k each.  K stages of 128 (32 for short products) keep enough loads
-// in flight per stage that the few stages of these products are not each a
-// full memory latency.
+// C = A B with the given epilogue
 void gemm(esl::ctx_t& c, esl_mlp* m, int M, int N, int K, const float* A, int64_t sam, int64_t sak, const float* B,
 		  int64_t sbk, int64_t sbn, const float* bias, float* C, float* Z, int epi)
 {
-	const int tiles = esl::ceil_div(M, 64) * esl::ceil_div(N, 64);
-	int splits = std::max(1, std::min({ K / 256, 256 / tiles, esl::gemm_max_splits }));
-	const int kper = esl::ceil_div(K, splits);
-	const int bk = kper >= 128 ? 128 : 32;
-	const int k_split = esl::ceil_div(esl::ceil_div(K, splits), bk) * bk;
-	splits = esl::ceil_div(K, k_split);
+	int bk;
+	const int k_split = gemm_split(M, N, K, bk);
+	const int splits = esl::ceil_div(K, k_split);
 	float* part = nullptr;
 	if (splits > 1)
 	{
@@ -685,6 +821,8 @@ esl_status esl_mlp_create(esl_ctx* ctx, int n_in, int hidden, int hidden_layers,
 		ESL_HIP(hipMemcpy(m->params.get(), h.data(), off * sizeof(float), hipMemcpyHostToDevice));
 		ESL_HIP(hipMemset(m->m1.get(), 0, off * sizeof(float)));
 		ESL_HIP(hipMemset(m->m2.get(), 0, off * sizeof(float)));
+		ESL_HIP(hipStreamSynchronize(nullptr)); // the fills run on it, training on the context's stream
+		plan_by_rows(esl::ctx_impl(ctx), m.get());
 		*out = m.release();
 	});
 }
@@ -707,6 +845,7 @@ esl_status esl_mlp_set_params(esl_ctx* ctx, esl_mlp* m, const float* host_in)
 	return mlp_guard(ctx, [&] {
 		if (!ctx || !m || !host_in)
 			throw esl::error(ESL_E_ARG, "null argument");
+		m->ops_stale = true;
 		ESL_HIP(hipMemcpy(m->params.get(), host_in, m->n_params * sizeof(float), hipMemcpyHostToDevice));
 	});
 }
@@ -717,6 +856,14 @@ esl_status esl_mlp_forward(esl_ctx* ctx, esl_mlp* m, int rows, const float* d_x,
 		if (!ctx || !m || !d_x || !d_probs || rows < 1)
 			throw esl::error(ESL_E_ARG, "null argument");
 		esl::ctx_t& c = esl::ctx_impl(ctx);
+		if (m->by_rows)
+		{
+			esl::mlp_batch_t q{};
+			q.rows = rows, q.x = d_x, q.P = d_probs;
+			run_rows(c, m, q);
+			ESL_HIP(hipStreamSynchronize(c.stream));
+			return;
+		}
 		ensure_rows(m, rows);
 		forward(c, m, rows, d_x);
 		const int L = (int)m->dims.size() - 1;
@@ -732,6 +879,14 @@ esl_status esl_mlp_predict_warm(esl_ctx* ctx, esl_mlp* m, int rows, const float*
 		if (!ctx || !m || !d_x || !d_warm || rows < 1)
 			throw esl::error(ESL_E_ARG, "null argument");
 		esl::ctx_t& c = esl::ctx_impl(ctx);
+		if (m->by_rows)
+		{
+			esl::mlp_batch_t q{};
+			q.rows = rows, q.x = d_x, q.Pd = d_warm;
+			run_rows(c, m, q);
+			ESL_HIP(hipStreamSynchronize(c.stream));
+			return;
+		}
 		ensure_rows(m, rows);
 		forward(c, m, rows, d_x);
 		const int L = (int)m->dims.size() - 1;
@@ -784,12 +939,37 @@ static float mlp_read_loss(esl::ctx_t& c, esl_mlp* m)
 	return loss;
 }
 
-// one Adam step on m->grads (beta1 0.9, beta2 0.999, eps 1e-8), enqueued
-static void mlp_enqueue_adam(esl::ctx_t& c, esl_mlp* m, float lr)
+// the gradients of one batch into m->grads, the loss into m->loss, enqueued
+static void mlp_enqueue_gradients(esl::ctx_t& c, esl_mlp* m, int rows, const float* d_x, const float* d_t)
 {
-	m->step++;
+	if (!m->by_rows)
+		return mlp_enqueue_backward(c, m, rows, d_x, d_t, false);
+	esl::mlp_batch_t q{};
+	q.rows = rows, q.x = d_x, q.tg = d_t;
+	run_rows(c, m, q);
+	run_update(c, m, q, {}, false, false);
+}
+
+// one Adam step (beta1 0.9, beta2 0.999, eps 1e-8), enqueued
+static void mlp_enqueue_step(esl::ctx_t& c, esl_mlp* m, int rows, const float* d_x, const float* d_t, float lr,
+							 bool accumulate)
+{
+	const int64_t step = m->step + 1;
 	const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-	const float c1 = 1.0f - std::pow(b1, (float)m->step), c2 = 1.0f - std::pow(b2, (float)m->step);
+	const float c1 = 1.0f - std::pow(b1, (float)step), c2 = 1.0f - std::pow(b2, (float)step);
+	if (m->by_rows)
+	{
+		esl::mlp_batch_t q{};
+		q.rows = rows, q.x = d_x, q.tg = d_t;
+		esl::mlp_adam_t a{};
+		a.lr = lr, a.b1 = b1, a.b2 = b2, a.eps = eps, a.c1 = c1, a.c2 = c2;
+		run_rows(c, m, q);
+		run_update(c, m, q, a, true, accumulate);
+		m->step = step;
+		return;
+	}
+	mlp_enqueue_backward(c, m, rows, d_x, d_t, accumulate);
+	m->step = step;
 	esl::k_adam<<<esl::ceil_div(m->n_params, 256), 256, 0, c.stream>>>(m->n_params, m->params.get(), m->grads.get(),
 																		m->m1.get(), m->m2.get(), lr, b1, b2, eps,
 																		c1, c2);
@@ -803,7 +983,7 @@ esl_status esl_mlp_gradients(esl_ctx* ctx, esl_mlp* m, int rows, const float* d_
 		if (!ctx || !m || !d_x || !d_target || rows < 1)
 			throw esl::error(ESL_E_ARG, "null argument");
 		esl::ctx_t& c = esl::ctx_impl(ctx);
-		mlp_enqueue_backward(c, m, rows, d_x, d_target, false);
+		mlp_enqueue_gradients(c, m, rows, d_x, d_target);
 		const float loss = mlp_read_loss(c, m) / rows;
 		if (loss_out)
 			*loss_out = loss;
@@ -819,8 +999,7 @@ esl_status esl_mlp_train_step(esl_ctx* ctx, esl_mlp* m, int rows, const float* d
 		if (!ctx || !m || !d_x || !d_target || rows < 1)
 			throw esl::error(ESL_E_ARG, "null argument");
 		esl::ctx_t& c = esl::ctx_impl(ctx);
-		mlp_enqueue_backward(c, m, rows, d_x, d_target, false);
-		mlp_enqueue_adam(c, m, lr);
+		mlp_enqueue_step(c, m, rows, d_x, d_target, lr, false);
 		const float loss = mlp_read_loss(c, m) / rows;
 		if (loss_out)
 			*loss_out = loss;
@@ -839,9 +1018,8 @@ esl_status esl_mlp_train_steps(esl_ctx* ctx, esl_mlp* m, int steps, int rows, co
 		{
 			const float lr =
 				steps == 1 || lr_first == 0.0f ? lr_first : (float)(lr_first * std::pow(ratio, (double)j / (steps - 1)));
-			mlp_enqueue_backward(c, m, rows, d_x + (int64_t)j * rows * m->n_in,
-								 d_target + (int64_t)j * rows * m->n_out, j > 0);
-			mlp_enqueue_adam(c, m, lr);
+			mlp_enqueue_step(c, m, rows, d_x + (int64_t)j * rows * m->n_in, d_target + (int64_t)j * rows * m->n_out,
+							 lr, j > 0);
 		}
 		const float loss = mlp_read_loss(c, m) / ((float)rows * steps);
 		if (mean_loss_out)
