@@ -83,7 +83,7 @@ def profile_stats(L, ctx):
 
 
 TABLE_KERNELS = ("k_flip_mask", "k_table_fill")
-MASK_PASS_KERNELS = ("k_trim", "k_color", "k_close", "k_height_check")
+MASK_PASS_KERNELS = ("k_edges", "k_trim", "k_color", "k_height")
 
 
 def stage_bandwidth(stats, n, m, counts=None):

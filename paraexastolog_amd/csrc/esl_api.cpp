@@ -164,6 +164,7 @@ void esl_ctx_destroy(esl_ctx* ctx)
 	if (ctx->c.h_stage)
 		(void)hipHostFree(ctx->c.h_stage);
 	ctx->c.flags.reset();
+	ctx->c.scan_sums.reset();
 	ctx->c.scratch_a.reset();
 	ctx->c.scratch_b.reset();
 	if (ctx->c.multi && ctx->c.multi_free)

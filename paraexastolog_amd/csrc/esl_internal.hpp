@@ -281,6 +281,7 @@ struct ctx_t
 	// reusable scratch
 	dbuf<uint8_t> scratch_a, scratch_b;
 	dbuf<int32_t> flags;	// small device counters / flags
+	dbuf<int32_t> scan_sums; // block sums of exclusive_scan_i32
 	int32_t* h_flags = nullptr; // pinned mirror
 	// pinned staging of the per-set outputs of a launch, read back in one copy
 	// (allocated with the context: calls that may not allocate use it too)

@@ -47,13 +47,14 @@
 #include <atomic>
 #include <chrono>
 #include <cmath>
+#include <cstring>
 #include <cstdio>
 #include <memory>
 #include <mutex>
 #include <thread>
 #include <type_traits>
 
-#include "common.hip.hpp"
+#include "cube.hip.hpp"
 #include "esl_internal.hpp"
 
 namespace esl {
@@ -73,24 +74,34 @@ __global__ __launch_bounds__(sblock) void k_reach_init(int64_t n, const double* 
 }
 
 // v is reached if an in-neighbour is (wave-local fixpoint over bits 0..5).
+template <int HMAX>
 __global__ __launch_bounds__(sblock) void k_reach(int N, int64_t n, const uint32_t* __restrict__ mask,
-												  uint8_t* __restrict__ reach, int32_t* __restrict__ changed)
+												  uint8_t* __restrict__ reach, int32_t* __restrict__ changed,
+												  const int32_t* __restrict__ prev)
 {
+	if (converged(prev))
+		return;
 	const int64_t v = (int64_t)blockIdx.x * sblock + threadIdx.x;
 	const bool valid = v < n;
 	const uint32_t mv = valid ? mask[v] : 0u;
 	const bool r0 = valid && reach[v];
 	bool r = r0;
-	if (valid && !r)
-		for (int i = 6; i < N; ++i)
+	if (HMAX > 0 && __any(valid && !r))
+	{
+		uint32_t mu[HMAX > 0 ? HMAX : 1];
+		uint8_t ru[HMAX > 0 ? HMAX : 1];
+		const int64_t vv = valid ? v : 0; // lanes past n read vertex 0's neighbours, unused
+#pragma unroll
+		for (int j = 0; j < HMAX; ++j)
 		{
-			const int64_t u = v ^ (int64_t(1) << i);
-			if (((mask[u] >> i) & 1u) && reach[u])
-			{
-				r = true;
-				break;
-			}
+			const int64_t u = vv ^ (int64_t(1) << high_bit(j, N));
+			mu[j] = mask[u];
+			ru[j] = reach[u];
 		}
+#pragma unroll
+		for (int j = 0; j < HMAX; ++j)
+			r |= valid && 6 + j < N && ((mu[j] >> (6 + j)) & 1u) && ru[j];
+	}
 	const int lim = N < 6 ? N : 6;
 	for (;;)
 	{
@@ -148,21 +159,32 @@ __global__ __launch_bounds__(sblock) void k_tm_init(int64_t n, const int32_t* __
 }
 
 // pull over out-neighbours: tm[v] |= tm[w] for v -> w (reachable transient v)
+template <int HMAX>
 __global__ __launch_bounds__(sblock) void k_tm(int N, int64_t n, const uint32_t* __restrict__ mask,
 											   const int32_t* __restrict__ rank, int64_t T,
 											   const uint8_t* __restrict__ reach, uint64_t* __restrict__ tm,
-											   int32_t* __restrict__ changed)
+											   int32_t* __restrict__ changed, const int32_t* __restrict__ prev)
 {
+	if (converged(prev))
+		return;
 	const int64_t v = (int64_t)blockIdx.x * sblock + threadIdx.x;
 	const bool valid = v < n;
 	const bool act = valid && reach[v] && rank[v] >= T;
 	const uint32_t mv = valid ? mask[v] : 0u;
 	const uint64_t m0 = valid ? tm[v] : 0ull;
 	uint64_t m = m0;
-	if (act)
-		for (int i = 6; i < N; ++i)
-			if ((mv >> i) & 1u)
-				m |= tm[v ^ (int64_t(1) << i)];
+	if (HMAX > 0 && __any(act))
+	{
+		uint64_t mu[HMAX > 0 ? HMAX : 1];
+		const int64_t vv = valid ? v : 0;
+#pragma unroll
+		for (int j = 0; j < HMAX; ++j)
+			mu[j] = tm[vv ^ (int64_t(1) << high_bit(j, N))];
+#pragma unroll
+		for (int j = 0; j < HMAX; ++j)
+			if (act && 6 + j < N && ((mv >> (6 + j)) & 1u))
+				m |= mu[j];
+	}
 	const int lim = N < 6 ? N : 6;
 	for (;;)
 	{
@@ -239,7 +261,8 @@ __global__ __launch_bounds__(sblock) void k_target_of(int64_t n, const int32_t* 
 													  const int32_t* __restrict__ jmap,
 													  const uint8_t* __restrict__ reach,
 													  const uint64_t* __restrict__ tm, const int32_t* __restrict__ amb,
-													  const double* __restrict__ x0, int Tr, int32_t* __restrict__ tgt)
+													  const double* __restrict__ x0, int Tr, int32_t* __restrict__ tgt,
+													  int32_t* __restrict__ has)
 {
 	const int64_t v = (int64_t)blockIdx.x * sblock + threadIdx.x;
 	if (v >= n)
@@ -256,6 +279,18 @@ __global__ __launch_bounds__(sblock) void k_target_of(int64_t n, const int32_t* 
 			j = __ffsll((unsigned long long)tm[v]) - 1;
 	}
 	tgt[v] = j;
+	has[v] = j >= 0 ? 1 : 0;
+}
+
+__global__ __launch_bounds__(sblock) void k_target_pack(int64_t n, const int32_t* __restrict__ tgt,
+														const int32_t* __restrict__ at, const double* __restrict__ x0,
+														int32_t* __restrict__ j, double* __restrict__ x)
+{
+	const int64_t v = (int64_t)blockIdx.x * sblock + threadIdx.x;
+	if (v >= n || tgt[v] < 0)
+		return;
+	j[at[v]] = tgt[v];
+	x[at[v]] = x0[v];
 }
 
 // ============================================================================
@@ -3294,27 +3329,62 @@ __global__ __launch_bounds__(sblock) void k_lu_store(sys_t S, int b, int64_t u0,
 
 namespace {
 
-struct flags_t
+// Device arrays to the host with one wait, through the context's pinned staging
+// buffer while they fit it.
+struct readback_t
 {
-	ctx_t& c;
-	explicit flags_t(ctx_t& x) : c(x) {}
-	void clear(int k) { ESL_HIP(hipMemsetAsync(c.flags.get() + k, 0, sizeof(int32_t), c.stream)); }
-	int32_t* dev(int k) { return c.flags.get() + k; }
-	int32_t read(int k)
+	struct item_t
 	{
-		ESL_HIP(hipMemcpyAsync(c.h_flags + k, c.flags.get() + k, sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
+		void* to;
+		size_t at, bytes;
+	};
+	ctx_t& c;
+	std::vector<item_t> items;
+	size_t used = 0;
+	explicit readback_t(ctx_t& x) : c(x) {}
+	template <typename T>
+	void add(std::vector<T>& h, const T* d, size_t count)
+	{
+		h.resize(count);
+		if (!count)
+			return;
+		const size_t bytes = count * sizeof(T);
+		void* to = h.data();
+		if (used + bytes <= c.h_stage_bytes)
+		{
+			items.push_back({ to, used, bytes });
+			to = c.h_stage + used;
+			used += (bytes + 15) / 16 * 16;
+		}
+		ESL_HIP(hipMemcpyAsync(to, d, bytes, hipMemcpyDeviceToHost, c.stream));
+	}
+	void wait()
+	{
 		ESL_HIP(hipStreamSynchronize(c.stream));
-		return c.h_flags[k];
+		for (const item_t& i : items)
+			std::memcpy(i.to, c.h_stage + i.at, i.bytes);
+		items.clear();
+		used = 0;
 	}
 };
 
 template <typename T>
 void read_host(ctx_t& c, std::vector<T>& h, const T* d, size_t count)
 {
-	h.resize(count);
-	if (count)
-		ESL_HIP(hipMemcpyAsync(h.data(), d, count * sizeof(T), hipMemcpyDeviceToHost, c.stream));
-	ESL_HIP(hipStreamSynchronize(c.stream));
+	readback_t r(c);
+	r.add(h, d, count);
+	r.wait();
+}
+
+// terminal masks to their fixpoint
+void propagate_masks(ctx_t& c, const graph_t& g, const uint8_t* reach, uint64_t* tmask)
+{
+	int hint = 4;
+	fixpoint(c, hint, 8, 1 << 24, "terminal-mask propagation", [&](int32_t* f, const int32_t* pf) {
+		ESL_HMAX_DISPATCH(g.N, k_tm,
+						  <<<ceil_div(g.n, sblock), sblock, 0, c.stream>>>(g.N, g.n, g.mask.get(), g.rank.get(), g.T,
+																		   reach, tmask, f, pf));
+	});
 }
 
 template <typename T>
@@ -3453,8 +3523,19 @@ void build_nbr(ctx_t& c, const sys_t& S, nbr_store_t& st)
 	k_nbr_fill<<<nb, sblock, 0, c.stream>>>(S, st.ptr.get(), st.nu.get(), st.nr.get(), st.mid.get(), lvl_key.get());
 	build_rb(c, S, st, opos.get(), n_odd, cnt.get());
 	// unknowns grouped by popcount level (counting sort on the host: N + 1 buckets)
-	std::vector<int32_t> h_key;
-	read_host(c, h_key, lvl_key.get(), (size_t)nU);
+	const bool pack = nU <= lds_max_unknowns && nnz < 65536 && S.N < 128;
+	std::vector<int32_t> h_key, h_ptr, h_mid, h_nu;
+	std::vector<uint8_t> h_nr;
+	readback_t rd(c);
+	rd.add(h_key, lvl_key.get(), (size_t)nU);
+	if (pack)
+	{
+		rd.add(h_ptr, st.ptr.get(), (size_t)nU + 1);
+		rd.add(h_mid, st.mid.get(), (size_t)nU);
+		rd.add(h_nu, st.nu.get(), (size_t)nnz);
+		rd.add(h_nr, st.nr.get(), (size_t)nnz);
+	}
+	rd.wait();
 	st.L = levels_t{};
 	st.L.n = S.N + 1;
 	std::vector<int32_t> h_cnt(st.L.n + 1, 0), h_lvl(nU);
@@ -3472,14 +3553,8 @@ void build_nbr(ctx_t& c, const sys_t& S, nbr_store_t& st)
 	// record offsets must fit 16 bits, counts 7 bits (a row has at most N
 	// neighbours)
 	st.packed = false;
-	if (nU <= lds_max_unknowns && nnz < 65536 && S.N < 128)
+	if (pack)
 	{
-		std::vector<int32_t> h_ptr, h_mid, h_nu;
-		std::vector<uint8_t> h_nr;
-		read_host(c, h_ptr, st.ptr.get(), (size_t)nU + 1);
-		read_host(c, h_mid, st.mid.get(), (size_t)nU);
-		read_host(c, h_nu, st.nu.get(), (size_t)nnz);
-		read_host(c, h_nr, st.nr.get(), (size_t)nnz);
 		std::vector<int32_t> pos(nU);
 		for (int64_t p = 0; p < nU; ++p)
 			pos[h_lvl[p]] = (int32_t)p;
@@ -4787,7 +4862,6 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 	const int64_t T = g.T;
 	const int64_t n_t = g.n_t;
 	const int nb = ceil_div(n, sblock);
-	flags_t fl(c);
 	timer_t tm_(c);
 	P.g = &g;
 	P.x0.ensure(n);
@@ -4796,15 +4870,10 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 	// ---- reachability from supp(x0)
 	P.reach.ensure(n);
 	k_reach_init<<<nb, sblock, 0, c.stream>>>(n, P.x0.get(), P.reach.get());
-	for (int p = 0;; ++p)
-	{
-		fl.clear(0);
-		k_reach<<<nb, sblock, 0, c.stream>>>(N, n, g.mask.get(), P.reach.get(), fl.dev(0));
-		if (!fl.read(0))
-			break;
-		if (p > (1 << 24))
-			throw error(ESL_E_DEVICE, "reachability did not converge");
-	}
+	int hint = 4;
+	fixpoint(c, hint, 8, 1 << 24, "reachability", [&](int32_t* f, const int32_t* pf) {
+		ESL_HMAX_DISPATCH(N, k_reach, <<<nb, sblock, 0, c.stream>>>(N, n, g.mask.get(), P.reach.get(), f, pf));
+	});
 	P.ms[0] = tm_.lap();
 
 	// ---- reachable terminal SCCs, compact index j, segments of size >= 2
@@ -4845,16 +4914,7 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 	P.tmask.ensure(n);
 	k_tm_init<<<nb, sblock, 0, c.stream>>>(n, g.rank.get(), T, P.d_jmap.get(), P.reach.get(), P.tmask.get());
 	if (!P.fallback && P.Tr > 1)
-		for (int p = 0;; ++p)
-		{
-			fl.clear(0);
-			k_tm<<<nb, sblock, 0, c.stream>>>(N, n, g.mask.get(), g.rank.get(), T, P.reach.get(), P.tmask.get(),
-											  fl.dev(0));
-			if (!fl.read(0))
-				break;
-			if (p > (1 << 24))
-				throw error(ESL_E_DEVICE, "terminal-mask propagation did not converge");
-		}
+		propagate_masks(c, g, P.reach.get(), P.tmask.get());
 	P.amb.ensure(n);
 	dbuf<int32_t> fpos;
 	fpos.ensure(n + 1);
@@ -4910,18 +4970,30 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 	P.y0.ensure(std::max(P.Tr, 1));
 	if (P.Tr)
 	{
-		dbuf<int32_t> tgt;
+		// the states with such mass, packed in state order: 32,768 of a million with five of
+		// 20 nodes fixed, and 12 MB to the host otherwise (3.6 of 10.5 ms of such a model)
+		dbuf<int32_t> tgt, has, at, mj;
+		dbuf<double> mx;
 		tgt.ensure(n);
+		has.ensure(n);
+		at.ensure(n + 1);
 		k_target_of<<<nb, sblock, 0, c.stream>>>(n, g.rank.get(), T, P.d_jmap.get(), P.reach.get(), P.tmask.get(),
-												  P.amb.get(), P.x0.get(), P.Tr, tgt.get());
+												  P.amb.get(), P.x0.get(), P.Tr, tgt.get(), has.get());
+		exclusive_scan_i32(c, has.get(), at.get(), n);
+		std::vector<int32_t> h_count, h_j;
+		read_host(c, h_count, at.get() + n, 1);
+		const int32_t count = h_count[0];
+		mj.ensure(std::max(count, 1));
+		mx.ensure(std::max(count, 1));
+		k_target_pack<<<nb, sblock, 0, c.stream>>>(n, tgt.get(), at.get(), P.x0.get(), mj.get(), mx.get());
 		ESL_HIP(hipGetLastError());
-		std::vector<int32_t> h_tgt;
-		std::vector<double> h_x0, h_y0(P.Tr, 0.0);
-		read_host(c, h_tgt, tgt.get(), (size_t)n);
-		read_host(c, h_x0, P.x0.get(), (size_t)n);
-		for (int64_t v = 0; v < n; ++v)
-			if (h_tgt[v] >= 0)
-				h_y0[h_tgt[v]] += h_x0[v];
+		std::vector<double> h_x, h_y0(P.Tr, 0.0);
+		readback_t rd(c);
+		rd.add(h_j, mj.get(), (size_t)count);
+		rd.add(h_x, mx.get(), (size_t)count);
+		rd.wait();
+		for (int32_t i = 0; i < count; ++i)
+			h_y0[h_j[i]] += h_x[i];
 		write_dev(c, P.y0.get(), h_y0);
 	}
 	// ---- exit edges of the ambiguous set, by target terminal SCC
@@ -4949,9 +5021,11 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 		ESL_HIP(hipGetLastError());
 		std::vector<int32_t> h_j, h_u;
 		std::vector<uint8_t> h_r;
-		read_host(c, h_j, ej.get(), (size_t)E);
-		read_host(c, h_u, eu.get(), (size_t)E);
-		read_host(c, h_r, er.get(), (size_t)E);
+		readback_t rd(c);
+		rd.add(h_j, ej.get(), (size_t)E);
+		rd.add(h_u, eu.get(), (size_t)E);
+		rd.add(h_r, er.get(), (size_t)E);
+		rd.wait();
 		// stable counting sort by target
 		for (int32_t e = 0; e < E; ++e)
 		{
@@ -6222,7 +6296,6 @@ void solution_full(ctx_t& c, graph_t& g, const double* d_rates, const esl_solve_
 	const int N = g.N;
 	const int64_t n = g.n, T = g.T, n_t = g.n_t;
 	const int nb = ceil_div(n, sblock);
-	flags_t fl(c);
 	solution_t& sol = g.sol;
 	sol = solution_t{};
 	std::vector<int32_t> h_reord;
@@ -6358,16 +6431,7 @@ void solution_full(ctx_t& c, graph_t& g, const double* d_rates, const esl_solve_
 	tmask.ensure(n);
 	k_tm_init<<<nb, sblock, 0, c.stream>>>(n, g.rank.get(), T, d_jmap.get(), reach.get(), tmask.get());
 	if (!fallback)
-		for (int p = 0;; ++p)
-		{
-			fl.clear(0);
-			k_tm<<<nb, sblock, 0, c.stream>>>(N, n, g.mask.get(), g.rank.get(), T, reach.get(), tmask.get(),
-											  fl.dev(0));
-			if (!fl.read(0))
-				break;
-			if (p > (1 << 24))
-				throw error(ESL_E_DEVICE, "terminal-mask propagation did not converge");
-		}
+		propagate_masks(c, g, reach.get(), tmask.get());
 	dbuf<int32_t> amb, fpos;
 	amb.ensure(n);
 	fpos.ensure(n + 1);

@@ -215,13 +215,12 @@ __global__ __launch_bounds__(scan_block) void k_scan_down(const int32_t* __restr
 void exclusive_scan_i32(ctx_t& c, const int32_t* in, int32_t* out, int64_t n)
 {
 	const int nb = ceil_div(n, scan_tile);
-	dbuf<int32_t> sums;
+	dbuf<int32_t>& sums = c.scan_sums;
 	sums.ensure(nb + 1);
 	k_scan_reduce<<<nb, scan_block, 0, c.stream>>>(in, n, sums.get());
 	k_scan_single<<<1, 1024, 0, c.stream>>>(sums.get(), nb);
 	k_scan_down<<<nb, scan_block, 0, c.stream>>>(in, n, sums.get(), out);
 	ESL_HIP(hipGetLastError());
-	ESL_HIP(hipStreamSynchronize(c.stream)); // `sums` is freed on return
 }
 
 // ---- host side -----------------------------------------------------------------
