@@ -32,7 +32,7 @@
 // relaxation from 1 everywhere: a pass of a wave relaxes its sub-cube to a fixpoint,
 // so it advances a chain by several levels.
 //
-// Up to 8192 states one workgroup does all of it in LDS, the order included: there a
+// Up to 4096 states one workgroup does all of it in LDS, the order included: there a
 // pass is a fraction of a microsecond, and launches and round trips were the time.
 //
 // Order: [terminal SCCs by ascending id | transient SCCs by (height desc, id
@@ -360,9 +360,12 @@ __global__ __launch_bounds__(gblock) void k_height_stats(int64_t n, const int32_
 	}
 }
 
-// ---- the whole stage for n <= 8192 states, by one workgroup: state arrays in LDS, up
-// to 8 vertices per thread.  Passes update in place: all relaxations are monotone.
-constexpr int gs_block = 1024, gs_v = 8;
+// ---- the whole stage for n <= 4096 states, by one workgroup: state arrays in LDS, up
+// to 4 vertices per thread.  Passes update in place: all relaxations are monotone.  A
+// pass is vector instructions on one compute unit, some 10 per vertex and bit: with 4096
+// states the stage is 1.7 to 2.4 times as fast as by launches (12 networks), with 8192
+// 0.7 to 1.5 times, so the line lies between.
+constexpr int gs_block = 1024, gs_v = 4, gs_bits = 12;
 constexpr int64_t gs_max = gs_block * gs_v;
 constexpr int gs_none = 0xffff; // no SCC yet
 
@@ -404,10 +407,11 @@ __global__ __launch_bounds__(gs_block) void k_graph_small(int N, const uint32_t*
 			if (v >= n || s_scc[v] != gs_none)
 				continue;
 			const uint32_t mv = s_mask[v], cv = s_cls[v];
-			for (int i = 0; i < N; ++i)
+#pragma unroll
+			for (int i = 0; i < gs_bits; ++i)
 			{
 				const int u = v ^ (1 << i);
-				if (s_scc[u] == gs_none && s_cls[u] == cv)
+				if (i < N && s_scc[u] == gs_none && s_cls[u] == cv)
 				{
 					in[q] |= s_mask[u] & (1u << i);
 					out[q] |= mv & (1u << i);
@@ -426,8 +430,10 @@ __global__ __launch_bounds__(gs_block) void k_graph_small(int N, const uint32_t*
 				if (v >= n || s_scc[v] != gs_none)
 					continue;
 				uint32_t act = 0;
-				for (int i = 0; i < N; ++i)
-					act |= s_scc[v ^ (1 << i)] == gs_none ? 1u << i : 0u;
+#pragma unroll
+				for (int i = 0; i < gs_bits; ++i)
+					if (i < N)
+						act |= s_scc[v ^ (1 << i)] == gs_none ? 1u << i : 0u;
 				if (!(in[q] & act) || !(out[q] & act))
 				{
 					s_scc[v] = (uint16_t)v;
@@ -451,8 +457,11 @@ __global__ __launch_bounds__(gs_block) void k_graph_small(int N, const uint32_t*
 					continue;
 				const uint32_t c0 = s_col[v];
 				uint32_t x = c0 & 0xffffu, y = c0 >> 16;
-				for (int i = 0; i < N; ++i)
+#pragma unroll
+				for (int i = 0; i < gs_bits; ++i)
 				{
+					if (i >= N)
+						continue;
 					const uint32_t cu = s_col[v ^ (1 << i)];
 					if ((in[q] >> i) & 1u)
 						x = min(x, cu & 0xffffu);
@@ -494,8 +503,10 @@ __global__ __launch_bounds__(gs_block) void k_graph_small(int N, const uint32_t*
 		out[q] = 0;
 		if (v >= n)
 			continue;
-		for (int i = 0; i < N; ++i)
-			out[q] |= s_scc[v ^ (1 << i)] != s_scc[v] ? s_mask[v] & (1u << i) : 0u;
+#pragma unroll
+		for (int i = 0; i < gs_bits; ++i)
+			if (i < N)
+				out[q] |= s_scc[v ^ (1 << i)] != s_scc[v] ? s_mask[v] & (1u << i) : 0u;
 		s_col[v] = 1;
 	}
 	__syncthreads();
@@ -512,7 +523,8 @@ __global__ __launch_bounds__(gs_block) void k_graph_small(int N, const uint32_t*
 			const int r = s_scc[v];
 			const uint32_t h0 = s_col[r];
 			uint32_t c = h0;
-			for (int i = 0; i < N; ++i)
+#pragma unroll
+			for (int i = 0; i < gs_bits; ++i)
 				if ((out[q] >> i) & 1u)
 					c = max(c, s_col[s_scc[v ^ (1 << i)]] + 1);
 			if (c > h0)
@@ -544,7 +556,7 @@ __global__ __launch_bounds__(gs_block) void k_graph_small(int N, const uint32_t*
 	{
 		const int r = s_scc[v], hv = (int)s_col[r];
 		const uint64_t hi = hv == 1 ? 0 : H + 1 - hv, lo = hv == 1 ? r : n - 1 - r;
-		s_key[v] = hi << 26 | lo << 13 | (uint64_t)v;
+		s_key[v] = hi << 2 * gs_bits | lo << gs_bits | (uint64_t)v;
 		scc[v] = r;
 		height[v] = hv;
 	}
@@ -567,12 +579,12 @@ __global__ __launch_bounds__(gs_block) void k_graph_small(int N, const uint32_t*
 	const int per = (n + gs_block - 1) / gs_block, p0 = t * per, p1 = min(n, p0 + per);
 	int first = 0, S;
 	for (int p = p0; p < p1; ++p)
-		first += p == 0 || s_key[p] >> 13 != s_key[p - 1] >> 13;
+		first += p == 0 || s_key[p] >> gs_bits != s_key[p - 1] >> gs_bits;
 	int k = block_excl_scan<gs_block>(first, s_red, S) - 1;
 	for (int p = p0; p < p1; ++p)
 	{
-		const int v = (int)(s_key[p] & 8191);
-		if (p == 0 || s_key[p] >> 13 != s_key[p - 1] >> 13)
+		const int v = (int)(s_key[p] & (gs_max - 1));
+		if (p == 0 || s_key[p] >> gs_bits != s_key[p - 1] >> gs_bits)
 			offsets[++k] = p;
 		reordered[p] = v;
 		rank[v] = k;

@@ -1,5 +1,5 @@
 """The graph stage at the sizes where its two forms begin and end (one workgroup up to
-8,192 states, passes over sub-cubes of 64 beyond), bit for bit against the oracle."""
+4,096 states, passes over sub-cubes of 64 beyond), bit for bit against the oracle."""
 import numpy as np
 import pytest
 
