@@ -29,13 +29,14 @@ namespace esl {
 // API calls each 85 times, at 35 and 45 us on average 6.8 of its 17.7 ms (10.5 with the
 // pool; 15 nodes: 4.3 to 3.8 ms).  A block is reused by work on the same context only: calls on
 // one context are serialised on its stream, so what was enqueued on a block comes
-// before what its next owner enqueues.  Blocks below 64 KB are not kept (1 us per
-// call where all are small, a model of 10 nodes), nor above a quarter of the bound; the
-// oldest leave when the bound is exceeded, all when an allocation fails and when
-// the context is destroyed (buffers that outlive it are freed directly).
+// before what its next owner enqueues.  Small blocks cost 1.6 us a pair (115 us
+// of the 1.06 ms of a model of 10 nodes).  Blocks above a quarter of the bound are not
+// kept; the oldest leave when there are more than 512 or the bound is exceeded, all when
+// an allocation fails and when the context is destroyed (buffers that outlive it are
+// freed directly).
 struct buf_pool_t
 {
-	static constexpr size_t bound = (size_t)512 << 20, least = (size_t)64 << 10;
+	static constexpr size_t bound = (size_t)512 << 20, least = 256, most_blocks = 512;
 	struct block_t
 	{
 		void* p;
@@ -73,7 +74,7 @@ struct buf_pool_t
 			{
 				blocks.push_back({ p, bytes });
 				held += bytes;
-				while (held > bound)
+				while (held > bound || blocks.size() > most_blocks)
 				{
 					out.push_back(blocks.front());
 					held -= blocks.front().bytes;

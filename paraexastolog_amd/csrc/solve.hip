@@ -3394,29 +3394,27 @@ void write_dev(ctx_t& c, T* d, const std::vector<T>& h)
 		ESL_HIP(hipMemcpyAsync(d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, c.stream));
 }
 
+// device time between marks on the stream, by the context's events; read once at the end
 struct timer_t
 {
+	static constexpr int first = 4, most = 8;
 	ctx_t& c;
-	hipEvent_t a, b;
-	explicit timer_t(ctx_t& x) : c(x)
+	int marks = 0;
+	explicit timer_t(ctx_t& x) : c(x) { mark(); }
+	void mark()
 	{
-		ESL_HIP(hipEventCreate(&a));
-		ESL_HIP(hipEventCreate(&b));
-		ESL_HIP(hipEventRecord(a, c.stream));
+		if (marks < most)
+			ESL_HIP(hipEventRecord(c.ev[first + marks++], c.stream));
 	}
-	double lap()
+	void read(double* ms)
 	{
-		ESL_HIP(hipEventRecord(b, c.stream));
-		ESL_HIP(hipEventSynchronize(b));
-		float ms = 0;
-		ESL_HIP(hipEventElapsedTime(&ms, a, b));
-		std::swap(a, b);
-		return ms;
-	}
-	~timer_t()
-	{
-		(void)hipEventDestroy(a);
-		(void)hipEventDestroy(b);
+		ESL_HIP(hipEventSynchronize(c.ev[first + marks - 1]));
+		for (int i = 0; i + 1 < marks; ++i)
+		{
+			float t = 0;
+			ESL_HIP(hipEventElapsedTime(&t, c.ev[first + i], c.ev[first + i + 1]));
+			ms[i] = t;
+		}
 	}
 };
 
@@ -3430,7 +3428,7 @@ struct nbr_store_t
 	dbuf<uint32_t> hdr, rec;
 	bool packed = false; // hdr / rec built
 	levels_t L{};
-	int64_t nnz = 0;
+	int64_t nnz = 0, nnz_t = 0; // of all rows, of the terminal rows
 	// the same lists with rows and neighbours in level order (set-minor
 	// device-wide solver), built on first use
 	mutable dbuf<int32_t> wptr, wmid, wnu;
@@ -3487,15 +3485,12 @@ void build_rb(ctx_t& c, const sys_t& S, nbr_store_t& st, const int32_t* opos, in
 	k_rb_place<<<nb, sblock, 0, c.stream>>>(nU, (int)st.nE, elim, S.ulist, opos, st.ptr.get(), st.rrow.get(), inv.get(),
 											cnt);
 	exclusive_scan_i32(c, cnt, st.rptr.get(), nU);
-	int32_t groups = 0;
-	ESL_HIP(hipMemcpyAsync(&groups, st.rptr.get() + nU, sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
-	ESL_HIP(hipStreamSynchronize(c.stream));
-	st.rgroups = groups;
-	st.rrec.ensure((size_t)groups + 1); // a group past the last, for loads ahead
+	// groups of four per row: at most one of each row is not full; and one past the last,
+	// for loads ahead
+	st.rrec.ensure((size_t)(st.nnz / 4 + nU) + 1);
 	k_rb_fill<<<nb, sblock, 0, c.stream>>>(nU, 2 * S.N, st.rrow.get(), inv.get(), st.ptr.get(), st.nu.get(), st.nr.get(),
 										   st.rptr.get(), st.rrec.get());
 	ESL_HIP(hipGetLastError());
-	ESL_HIP(hipStreamSynchronize(c.stream));
 }
 
 void build_nbr(ctx_t& c, const sys_t& S, nbr_store_t& st)
@@ -3513,10 +3508,12 @@ void build_nbr(ctx_t& c, const sys_t& S, nbr_store_t& st)
 	exclusive_scan_i32(c, cnt.get(), opos.get(), nU);
 	k_nbr_count<<<nb, sblock, 0, c.stream>>>(S, cnt.get());
 	exclusive_scan_i32(c, cnt.get(), st.ptr.get(), nU);
-	int32_t nnz = 0, n_odd = 0;
-	ESL_HIP(hipMemcpyAsync(&nnz, st.ptr.get() + nU, sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
-	ESL_HIP(hipMemcpyAsync(&n_odd, opos.get() + nU, sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
-	ESL_HIP(hipStreamSynchronize(c.stream));
+	readback_t rd(c);
+	std::vector<int32_t> h_nnz, h_odd, h_groups, h_nnz_t;
+	rd.add(h_nnz, st.ptr.get() + nU, 1);
+	rd.add(h_odd, opos.get() + nU, 1);
+	rd.wait();
+	const int32_t nnz = h_nnz[0], n_odd = h_odd[0];
 	st.nnz = nnz;
 	st.nu.ensure(std::max(nnz, 1));
 	st.nr.ensure(std::max(nnz, 1));
@@ -3526,7 +3523,8 @@ void build_nbr(ctx_t& c, const sys_t& S, nbr_store_t& st)
 	const bool pack = nU <= lds_max_unknowns && nnz < 65536 && S.N < 128;
 	std::vector<int32_t> h_key, h_ptr, h_mid, h_nu;
 	std::vector<uint8_t> h_nr;
-	readback_t rd(c);
+	rd.add(h_groups, st.rptr.get() + nU, 1);
+	rd.add(h_nnz_t, st.ptr.get() + S.nUt, 1);
 	rd.add(h_key, lvl_key.get(), (size_t)nU);
 	if (pack)
 	{
@@ -3536,6 +3534,8 @@ void build_nbr(ctx_t& c, const sys_t& S, nbr_store_t& st)
 		rd.add(h_nr, st.nr.get(), (size_t)nnz);
 	}
 	rd.wait();
+	st.rgroups = h_groups[0];
+	st.nnz_t = h_nnz_t[0];
 	st.L = levels_t{};
 	st.L.n = S.N + 1;
 	std::vector<int32_t> h_cnt(st.L.n + 1, 0), h_lvl(nU);
@@ -4874,7 +4874,7 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 	fixpoint(c, hint, 8, 1 << 24, "reachability", [&](int32_t* f, const int32_t* pf) {
 		ESL_HMAX_DISPATCH(N, k_reach, <<<nb, sblock, 0, c.stream>>>(N, n, g.mask.get(), P.reach.get(), f, pf));
 	});
-	P.ms[0] = tm_.lap();
+	tm_.mark();
 
 	// ---- reachable terminal SCCs, compact index j, segments of size >= 2
 	dbuf<int32_t> reached;
@@ -4883,8 +4883,13 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 	if (n_t)
 		k_term_reached<<<ceil_div(n_t, sblock), sblock, 0, c.stream>>>(n_t, g.reordered.get(), g.rank.get(),
 																		 P.reach.get(), reached.get());
-	std::vector<int32_t> h_reached;
-	read_host(c, h_reached, reached.get(), (size_t)T);
+	// with few terminal states their order comes along, in the same wait
+	std::vector<int32_t> h_reached, h_reord;
+	readback_t rd(c);
+	rd.add(h_reached, reached.get(), (size_t)T);
+	if (n_t <= 16384)
+		rd.add(h_reord, g.reordered.get(), (size_t)n_t);
+	rd.wait();
 	P.jmap.assign(T, -1);
 	P.segmap.assign(T, -1);
 	P.seg_off.assign(1, 0);
@@ -4918,17 +4923,20 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 	P.amb.ensure(n);
 	dbuf<int32_t> fpos;
 	fpos.ensure(n + 1);
+	int32_t nA = 0;
 	if (P.Tr > 1)
+	{
 		k_amb_flag<<<nb, sblock, 0, c.stream>>>(n, g.rank.get(), T, P.reach.get(), P.tmask.get(), P.fallback ? 1 : 0,
 												P.amb.get());
+		exclusive_scan_i32(c, P.amb.get(), fpos.get(), n);
+		std::vector<int32_t> h_nA;
+		read_host(c, h_nA, fpos.get() + n, 1);
+		nA = h_nA[0];
+	}
 	else
 		ESL_HIP(hipMemsetAsync(P.amb.get(), 0, n * sizeof(int32_t), c.stream));
-	exclusive_scan_i32(c, P.amb.get(), fpos.get(), n);
-	int32_t nA = 0;
-	ESL_HIP(hipMemcpyAsync(&nA, fpos.get() + n, sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
-	ESL_HIP(hipStreamSynchronize(c.stream));
 	P.nA = nA;
-	P.ms[1] = tm_.lap();
+	tm_.mark();
 
 	// ---- unknowns: terminal segments (canonical order) then ambiguous states
 	P.nUt = P.seg_off.back();
@@ -4939,11 +4947,16 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 	P.d_seg_off.ensure(P.seg_off.size());
 	ESL_HIP(hipMemsetAsync(P.pos.get(), 0xff, n * sizeof(int32_t), c.stream));
 	write_dev(c, P.d_seg_off.get(), P.seg_off);
+	// what is copied to the device stays until the wait at the end
+	std::vector<int32_t> states, seg_of, tpos, s_u;
+	std::vector<uint8_t> s_r;
+	std::vector<double> h_y0;
+	dbuf<int32_t> d_states, d_segof;
 	if (P.nUt)
 	{
-		std::vector<int32_t> h_reord;
-		read_host(c, h_reord, g.reordered.get(), (size_t)n_t);
-		std::vector<int32_t> states(P.nUt), seg_of(P.nUt), tpos(P.nUt);
+		if (n_t > 16384)
+			read_host(c, h_reord, g.reordered.get(), (size_t)n_t);
+		states.resize(P.nUt), seg_of.resize(P.nUt), tpos.resize(P.nUt);
 		for (int k = 0; k < P.n_seg; ++k)
 			for (int32_t q = 0; q < P.seg_off[k + 1] - P.seg_off[k]; ++q)
 			{
@@ -4953,14 +4966,12 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 			}
 		P.d_tpos.ensure(P.nUt);
 		write_dev(c, P.d_tpos.get(), tpos);
-		dbuf<int32_t> d_states, d_segof;
 		d_states.ensure(P.nUt);
 		d_segof.ensure(P.nUt);
 		write_dev(c, d_states.get(), states);
 		write_dev(c, d_segof.get(), seg_of);
 		k_fill_term_unknowns<<<ceil_div(P.nUt, sblock), sblock, 0, c.stream>>>(
 			P.nUt, d_states.get(), d_segof.get(), P.ulist.get(), P.ucls.get(), P.pos.get());
-		ESL_HIP(hipStreamSynchronize(c.stream));
 	}
 	if (nA)
 		k_fill_unknowns<<<nb, sblock, 0, c.stream>>>(n, P.amb.get(), fpos.get(), P.nUt, P.ulist.get(), P.ucls.get(),
@@ -4981,18 +4992,27 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 												  P.amb.get(), P.x0.get(), P.Tr, tgt.get(), has.get());
 		exclusive_scan_i32(c, has.get(), at.get(), n);
 		std::vector<int32_t> h_count, h_j;
-		read_host(c, h_count, at.get() + n, 1);
-		const int32_t count = h_count[0];
-		mj.ensure(std::max(count, 1));
-		mx.ensure(std::max(count, 1));
+		std::vector<double> h_x;
+		// few states: packed into arrays for all of them, read with their number in one wait
+		const bool few = n <= 8192;
+		int64_t count = n;
+		if (!few)
+		{
+			read_host(c, h_count, at.get() + n, 1);
+			count = h_count[0];
+		}
+		mj.ensure(std::max<int64_t>(count, 1));
+		mx.ensure(std::max<int64_t>(count, 1));
 		k_target_pack<<<nb, sblock, 0, c.stream>>>(n, tgt.get(), at.get(), P.x0.get(), mj.get(), mx.get());
 		ESL_HIP(hipGetLastError());
-		std::vector<double> h_x, h_y0(P.Tr, 0.0);
-		readback_t rd(c);
+		if (few)
+			rd.add(h_count, at.get() + n, 1);
 		rd.add(h_j, mj.get(), (size_t)count);
 		rd.add(h_x, mx.get(), (size_t)count);
 		rd.wait();
-		for (int32_t i = 0; i < count; ++i)
+		count = h_count[0];
+		h_y0.assign(P.Tr, 0.0);
+		for (int64_t i = 0; i < count; ++i)
 			h_y0[h_j[i]] += h_x[i];
 		write_dev(c, P.y0.get(), h_y0);
 	}
@@ -5008,9 +5028,9 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 		ptr.ensure(nA + 1);
 		k_exit_count<<<gA, sblock, 0, c.stream>>>(S, g.rank.get(), T, P.d_jmap.get(), P.tmask.get(), cnt.get());
 		exclusive_scan_i32(c, cnt.get(), ptr.get(), nA);
-		int32_t E = 0;
-		ESL_HIP(hipMemcpyAsync(&E, ptr.get() + nA, sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
-		ESL_HIP(hipStreamSynchronize(c.stream));
+		std::vector<int32_t> h_E;
+		read_host(c, h_E, ptr.get() + nA, 1);
+		const int32_t E = h_E[0];
 		dbuf<int32_t> ej, eu;
 		dbuf<uint8_t> er;
 		ej.ensure(std::max(E, 1));
@@ -5021,7 +5041,6 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 		ESL_HIP(hipGetLastError());
 		std::vector<int32_t> h_j, h_u;
 		std::vector<uint8_t> h_r;
-		readback_t rd(c);
 		rd.add(h_j, ej.get(), (size_t)E);
 		rd.add(h_u, eu.get(), (size_t)E);
 		rd.add(h_r, er.get(), (size_t)E);
@@ -5035,8 +5054,8 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 		}
 		for (int j = 0; j < P.Tr; ++j)
 			P.ex_off[j + 1] += P.ex_off[j];
-		std::vector<int32_t> fill(P.ex_off.begin(), P.ex_off.end() - 1), s_u(E);
-		std::vector<uint8_t> s_r(E);
+		std::vector<int32_t> fill(P.ex_off.begin(), P.ex_off.end() - 1);
+		s_u.resize(E), s_r.resize(E);
 		for (int32_t e = 0; e < E; ++e)
 		{
 			const int32_t at = fill[h_j[e]]++;
@@ -5049,7 +5068,6 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 		write_dev(c, P.ex_u.get(), s_u);
 		write_dev(c, P.ex_r.get(), s_r);
 		write_dev(c, P.d_ex_off.get(), P.ex_off);
-		ESL_HIP(hipStreamSynchronize(c.stream));
 		P.n_exit = E;
 	}
 	// ---- coupling structure of the per-set solver
@@ -5062,11 +5080,7 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 		build_nbr(c, S, P.nbr);
 		if (P.nUt > 0 && P.nUt <= 4096)
 		{
-			int32_t nnz_t = 0;
-			ESL_HIP(hipMemcpyAsync(&nnz_t, P.nbr.ptr.get() + P.nUt, sizeof(int32_t), hipMemcpyDeviceToHost,
-								   c.stream));
-			ESL_HIP(hipStreamSynchronize(c.stream));
-			const size_t bytes = 24 * (size_t)P.nUt + 4 * (size_t)(P.nUt + 1) + 3 * (size_t)nnz_t + 16;
+			const size_t bytes = 24 * (size_t)P.nUt + 4 * (size_t)(P.nUt + 1) + 3 * (size_t)P.nbr.nnz_t + 16;
 			const size_t static_bytes = 64 * 8 + sblock * 12 + 256;
 			if (bytes + static_bytes <= (size_t)std::min(c.lds_per_block, 160 * 1024))
 			{
@@ -5089,7 +5103,8 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 			}
 		}
 	}
-	P.ms[2] = tm_.lap();
+	tm_.mark();
+	tm_.read(P.ms);
 }
 
 sys_t plan_t::sys(int B, const double* rates) const
@@ -6102,7 +6117,9 @@ void many_per_set(ctx_t& c, const std::vector<int>& conc, void* const* plans, co
 			rep.iterations_sum = kr.iters_sum;
 		}
 	}
-	const double ms = tm_.lap();
+	tm_.mark();
+	double ms = 0.0;
+	tm_.read(&ms);
 	for (int i : conc)
 	{
 		reps[i].ms_stage[3] = ms;
