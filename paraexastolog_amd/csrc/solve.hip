@@ -32,12 +32,12 @@
 //    mass after a few damped Jacobi sweeps of the singular system, chosen per
 //    rate set.
 //
-// Both systems are solved together, for every rate set of a batch, by
-// restarted GMRES with Jacobi (diagonal) right preconditioning: the
-// preconditioned operator is  z -> z - P^T z  with P the jump-chain matrix
-// (P[t, s] = rate(t -> s) / D_t).  Precision 0 runs GMRES in FP64; precision 1
-// runs FP32 GMRES inner solves on the FP64 residual (iterative refinement)
-// until the FP64 residual meets the tolerance.
+// Both systems are solved together, for every rate set of a batch, by BiCGStab on
+// the system reduced by one parity class of the states (reduced.hip.hpp), in FP64.
+// An explicit restart length, a preconditioner or a pinned schedule asks for restarted
+// GMRES with ILU(0) or Jacobi instead, which also finishes the sets that the reduced
+// solver leaves: in FP64, or (precision 1) in FP32 cycles on the FP64 residual
+// (iterative refinement) until that meets the tolerance.
 //
 // Vectors are set-major ([set][unknown]); the shared structure (mask, maps,
 // unknown list) is a few tens of MB and stays in the 256 MB Infinity Cache
