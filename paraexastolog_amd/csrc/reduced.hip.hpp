@@ -227,7 +227,7 @@ constexpr int rb_cycle_products = 500; // products by S per cycle, so that round
 
 // What a solve that starts from the rates alone sets up by itself: the anchors
 // [B][n_seg], and from them 1 / D' and the right-hand side that other methods and
-// checks read.
+// checks read.  Anchors that turn out to be bad are moved there too.
 struct rb_setup_t
 {
 	const double* x0; // [2^N]; null: anchors, 1 / D', right-hand side and start vector are given
@@ -238,6 +238,7 @@ struct rb_setup_t
 	const double* warm;	 // [B][n_t] predicted final vectors on the terminal states, or null
 	const int32_t* tpos; // terminal unknown -> its place there
 	int64_t n_t;
+	const int32_t* only; // per set: whether the per-set kernel solves it; null: all
 	// mass that the sweeps start from on a terminal unknown
 	__device__ __forceinline__ double mass(int b, int32_t u) const
 	{
@@ -299,6 +300,8 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 	__shared__ double s_part[2][rb_part];
 	__shared__ double s_rates[64];
 	const int b = blockIdx.x, tid = threadIdx.x;
+	if (su.only && !su.only[b])
+		return;
 	const uint64_t t_begin = wall_clock64();
 	const int nE = G.nE, nR = G.nR, nU = nE + nR;
 	const int64_t off = (int64_t)b * nU;
@@ -747,6 +750,65 @@ __global__ __launch_bounds__(BLK, 4) void k_bicg_set(
 	bicg_set_body<BLK, RPT, LREC>(S, G, n_seg, rhs, zio, sc, su, tol, max_iters, out);
 }
 
+// Moves bad anchors, for the sets above the tolerance.  A segment's solution is scaled
+// to 1 at its anchor, the row of largest mass after the sweeps.  Where the rates part
+// a segment into regions that exchange little mass, the sweeps can end before the mass
+// has settled; the anchor is then a row with a thousandth of the largest entry or
+// less, and the rounding of D x alone keeps the residual, which is relative to the
+// anchor's 1, above a tolerance of 1e-12 (about two sets in a million of 2,048 unknowns
+// with log-uniform rates in [0.1, 10]: entries of 700 to 6,600 times the anchor's).
+// No method gets below that; the same iterate divided by its largest entry, with the
+// anchor there, has a residual of 1e-15.  Rare, so in a kernel of its own, one
+// workgroup per set, on the set-major vectors.
+constexpr double rb_bad_anchor = 2.0; // an anchor is moved to an entry more than this many times its own
+__global__ __launch_bounds__(sblock) void k_rb_move(sys_t S, rb_setup_t su, const double* __restrict__ res, double tol,
+													double* __restrict__ z, int32_t* __restrict__ moved)
+{
+	__shared__ double s_v[sblock / wave];
+	__shared__ int32_t s_u[sblock / wave];
+	const int b = blockIdx.x, tid = threadIdx.x;
+	const int64_t off = (int64_t)b * S.nU;
+	int any = 0;
+	for (int k = 0; k < su.n_seg && !(res[b] <= tol); ++k)
+	{
+		const int32_t old = su.anchor[(int64_t)b * su.n_seg + k], u1 = su.seg_off[k + 1];
+		double best = -1.0;
+		int32_t bu = INT32_MAX;
+		for (int32_t u = su.seg_off[k] + tid; u < u1; u += sblock)
+		{
+			const double x = z[off + u] * su.invd[off + u];
+			if (x > best)
+			{
+				best = x;
+				bu = u;
+			}
+		}
+		rb_block_argmax<sblock>(best, bu, s_v, s_u);
+		if (!(best > rb_bad_anchor) || !rb_finite(best) || bu == old)
+			continue;
+		any = 1;
+		for (int32_t u = su.seg_off[k] + tid; u < u1; u += sblock)
+		{
+			const double v = z[off + u] / best;
+			z[off + u] = v;
+			if (u == old)
+			{
+				const uint32_t st = (uint32_t)S.ulist[u];
+				const double d = out_rate_s(st, S.mask[st], S.rates + (int64_t)b * S.rate_stride);
+				z[off + u] = v * d; // D' was 1 here
+				su.invd[off + u] = 1.0 / d;
+				su.rhs[off + u] = 0.0;
+			}
+			if (u == bu)
+				z[off + u] = su.invd[off + u] = su.rhs[off + u] = 1.0;
+		}
+		if (tid == 0)
+			su.anchor[(int64_t)b * su.n_seg + k] = bu;
+	}
+	if (tid == 0)
+		moved[b] = any;
+}
+
 using bicg_set_fn = void (*)(sys_t, rb_t, int, const double*, double*, rb_scratch_t, rb_setup_t, double, int, pgm_out_t);
 struct bicg_variant_t
 {
@@ -1093,15 +1155,20 @@ __global__ void k_rbw_pick(rb_t G, rbw_geo_t geo, int n_seg, int slices, const i
 		}
 }
 
-// slices -> anchor[b][seg] and its mass pa[seg][b]
+// slices -> anchor[b][seg] and its mass pa[seg][b].  Where anchors are moved (k_rb_move;
+// `only` null otherwise) for the sets of `only`: bad ones are replaced and the set
+// marked in `moved`, the others' mass is 1.
 __global__ __launch_bounds__(sblock) void k_rbw_anchor(int B, int n_seg, int slices, const double* __restrict__ pv,
 													   const int32_t* __restrict__ pu, int32_t* __restrict__ anchor,
-													   double* __restrict__ pa)
+													   double* __restrict__ pa, const int32_t* __restrict__ only,
+													   int32_t* __restrict__ moved)
 {
 	const int i = blockIdx.x * sblock + threadIdx.x;
 	if (i >= n_seg * B)
 		return;
 	const int k = i / B, b = i - k * B;
+	if (only && !only[b])
+		return;
 	double best = -1.0;
 	int32_t bu = INT32_MAX;
 	for (int s = 0; s < slices; ++s)
@@ -1113,8 +1180,49 @@ __global__ __launch_bounds__(sblock) void k_rbw_anchor(int B, int n_seg, int sli
 			bu = pu[at];
 		}
 	}
+	if (only)
+	{
+		if (!(best > rb_bad_anchor) || !rb_finite(best) || anchor[(int64_t)b * n_seg + k] == bu)
+		{
+			pa[i] = 1.0;
+			return;
+		}
+		moved[b] = 1;
+	}
 	anchor[(int64_t)b * n_seg + k] = bu;
 	pa[i] = best;
+}
+
+// after k_rbw_anchor moved anchors and k_rbw_coef made the coefficients anew: the anchors'
+// coefficients of every set, and the iterate and right-hand side of the sets of `only`
+template <int W>
+__global__ void k_rbw_move(sys_t S, rb_t G, rbw_geo_t geo, int n_seg, const double* __restrict__ pa,
+						   const int32_t* __restrict__ only, double* __restrict__ c, double* __restrict__ x,
+						   double* __restrict__ wb)
+{
+	ESL_RBW_THREAD;
+	int64_t q0, q1;
+	rbw_rows(S.nU, q0, q1);
+	if (!in)
+		return;
+	for (int64_t q = q0 + t_row; q < q1; q += geo.R)
+	{
+		const int32_t u = G.row[q], k = S.ucls[u];
+		if (k < 0)
+			continue;
+		for (int w = 0; w < W; ++w)
+		{
+			const int64_t i = q * B + b + w;
+			const bool anchor = S.anchor[(int64_t)(b + w) * n_seg + k] == u;
+			if (anchor)
+				c[i] = 0.0;
+			if (only[b + w])
+			{
+				x[i] = anchor ? 1.0 : x[i] / pa[(int64_t)k * B + b + w];
+				wb[i] = anchor ? 1.0 : 0.0;
+			}
+		}
+	}
 }
 
 // start vector, right-hand side and anchors (c <- 0: the row is the identity).

@@ -3914,7 +3914,7 @@ struct rbw_ws_t
 		pa.ensure((size_t)n_seg * B);
 		seg_rows.ensure((size_t)2 * (n_seg + 1));
 		st.ensure(B);
-		undo.ensure(B);
+		undo.ensure((size_t)2 * B);
 		if (n_live < (size_t)2 * B)
 		{
 			if (h_live)
@@ -3947,6 +3947,8 @@ struct bicg_w_t
 	std::vector<double> h_res; // relative residuals of the last check
 	int iters = 0, cycles = 0;
 	double final_res = 0.0;
+	rb_setup_t su{};	// segments and anchors, where these may be moved
+	bool moved = false; // anchors were
 
 	bicg_w_t(ctx_t& ctx, const sys_t& sys, const nbr_store_t& nb, rbw_ws_t& w, int nseg)
 		: c(ctx), S(sys), NB(nb), ws(w), n_seg(nseg), B(sys.B), G(nb.rview())
@@ -3999,11 +4001,11 @@ struct bicg_w_t
 
 	// set-up from the rates alone: coefficients, anchors (into anchor[b][seg]), start
 	// vector and right-hand side
-	void enter(const rb_setup_t& su)
+	void enter(const rb_setup_t& setup)
 	{
-		const int segs = su.n_seg;
+		movable(setup);
 		rows(nbU, 0, true, [](auto w) { return k_rbw_coef<decltype(w)::value>; }, S, G, geo, su, ws.c.get(), TE, P);
-		if (segs)
+		if (su.n_seg)
 		{
 			for (int it = 0; it < rb_sweeps; ++it)
 			{
@@ -4014,29 +4016,60 @@ struct bicg_w_t
 					rows(nbR, 0, true, [](auto w) { return k_rbw_sweep<decltype(w)::value, true>; }, G, geo, ws.c.get(), TE, P);
 				});
 			}
-			k_rbw_seg_rows<<<ceil_div(segs + 1, sblock), sblock, 0, c.stream>>>(G, segs, su.seg_off, ws.seg_rows.get());
-			const int nt = geo.L * geo.R;
-			const size_t lds = (size_t)W * nt * 12;
-			const dim3 gp(slices * segs, chunks);
-			if (W == 2)
-				k_rbw_pick<2><<<gp, nt, lds, c.stream>>>(G, geo, segs, slices, ws.seg_rows.get(), TE, P, ws.pick_v.get(),
-														 ws.pick_u.get());
-			else
-				k_rbw_pick<1><<<gp, nt, lds, c.stream>>>(G, geo, segs, slices, ws.seg_rows.get(), TE, P, ws.pick_v.get(),
-														 ws.pick_u.get());
-			k_rbw_anchor<<<ceil_div(segs * B, sblock), sblock, 0, c.stream>>>(B, segs, slices, ws.pick_v.get(),
-																			   ws.pick_u.get(), su.anchor, ws.pa.get());
+			pick(TE, P, nullptr);
 		}
 		rows(nbU, 0, false, [](auto w) { return k_rbw_start<decltype(w)::value>; }, S, G, geo, n_seg, su.x0, TE, P, ws.pa.get(), ws.c.get(), ws.x.get(), ws.b.get());
 		diag();
 	}
 
-	// from the plan's vectors (a warm start, or another system set up set-major)
+	// from the plan's vectors (another system, set up set-major)
 	void enter(const double* rhs, const double* z)
 	{
 		const dim3 gt(ceil_div(S.nU, rbw_tile), ceil_div(B, rbw_tile));
 		k_rbw_enter<<<gt, sblock, 0, c.stream>>>(S, G, n_seg, rhs, z, ws.x.get(), ws.b.get(), ws.c.get());
 		diag();
+	}
+
+	// the segments, so that their anchors can be picked and moved
+	void movable(const rb_setup_t& setup)
+	{
+		su = setup;
+		if (su.n_seg)
+			k_rbw_seg_rows<<<ceil_div(su.n_seg + 1, sblock), sblock, 0, c.stream>>>(G, su.n_seg, su.seg_off,
+																					 ws.seg_rows.get());
+	}
+
+	// the rows of largest value in mE, mR as anchors, of every set or (replacing bad ones) of
+	// the sets of `only`
+	void pick(const double* mE, const double* mR, const int32_t* only)
+	{
+		const int nt = geo.L * geo.R;
+		const size_t lds = (size_t)W * nt * 12;
+		const dim3 gp(slices * su.n_seg, chunks);
+		if (W == 2)
+			k_rbw_pick<2><<<gp, nt, lds, c.stream>>>(G, geo, su.n_seg, slices, ws.seg_rows.get(), mE, mR, ws.pick_v.get(),
+													 ws.pick_u.get());
+		else
+			k_rbw_pick<1><<<gp, nt, lds, c.stream>>>(G, geo, su.n_seg, slices, ws.seg_rows.get(), mE, mR, ws.pick_v.get(),
+													 ws.pick_u.get());
+		k_rbw_anchor<<<ceil_div(su.n_seg * B, sblock), sblock, 0, c.stream>>>(
+			B, su.n_seg, slices, ws.pick_v.get(), ws.pick_u.get(), su.anchor, ws.pa.get(), only, ws.undo.get() + B);
+	}
+
+	// The anchors of the sets with a mark in `which` [B] moved where they are bad (k_rb_move);
+	// returns which sets' were.  Other sets keep their iterates and coefficients, bit for bit.
+	std::vector<int32_t> move_anchors(std::vector<int32_t> which)
+	{
+		which.resize((size_t)2 * B, 0);
+		write_dev(c, ws.undo.get(), which);
+		const int32_t* only = ws.undo.get();
+		pick(ws.x.get(), ws.x.get() + (size_t)G.nE * B, only);
+		rows(nbU, 0, true, [](auto w) { return k_rbw_coef<decltype(w)::value>; }, S, G, geo, su, ws.c.get(), TE, P);
+		rows(nbU, 0, false, [](auto w) { return k_rbw_move<decltype(w)::value>; }, S, G, geo, n_seg, ws.pa.get(), only, ws.c.get(), ws.x.get(), ws.b.get());
+		diag();
+		std::vector<int32_t> got;
+		read_host(c, got, ws.undo.get() + B, (size_t)B);
+		return got;
 	}
 
 	void diag()
@@ -4107,7 +4140,7 @@ struct bicg_w_t
 	{
 		std::vector<double> norms, prev(B, 0.0);
 		std::vector<rbw_set_t> hs(B);
-		std::vector<int32_t> undo(B, 0), fails(B, 0), compare(B, 0);
+		std::vector<int32_t> undo(B, 0), fails(B, 0), compare(B, 0), tried(B, 0);
 		const double* cc = ws.c.get();
 		for (;;)
 		{
@@ -4169,6 +4202,30 @@ struct bicg_w_t
 				}
 				if (more)
 					continue;
+			}
+			if (su.n_seg)
+			{
+				std::vector<int32_t> which(B, 0);
+				for (int b = 0; b < B; ++b)
+					which[b] = !(h_res[b] <= tol) && fails[b] >= rb_max_fails && !tried[b];
+				if (std::any_of(which.begin(), which.end(), [](int32_t v) { return v != 0; }))
+				{
+					const std::vector<int32_t> got = move_anchors(which);
+					bool again = false;
+					for (int b = 0; b < B; ++b)
+					{
+						tried[b] |= which[b];
+						if (!got[b])
+							continue;
+						fails[b] = 0;
+						again = moved = true;
+					}
+					if (again)
+					{
+						std::fill(compare.begin(), compare.end(), 0); // as after an undone cycle
+						continue;
+					}
+				}
 			}
 			if (all || !any_live || iters >= max_iters)
 				return all;
@@ -4530,8 +4587,9 @@ void launch_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, int n_seg, 
 	ESL_HIP(hipGetLastError());
 }
 
-// Reads the per-set results of a launch_per_set.  Sets that missed the tolerance
-// in mixed precision (their FP32 cycles stalled) or in the reduced solver are
+// Reads the per-set results of a launch_per_set.  Sets that the reduced solver leaves
+// above the tolerance get their bad anchors moved (k_rb_move) and another go.  Sets that
+// missed it in mixed precision (their FP32 cycles stalled) or in the reduced solver are
 // finished by FP64 GMRES with ILU(0) from their current iterate; sets that already
 // converged leave it at their first residual check.
 // fp64_view() gives the scratch with an FP64 basis (it may grow it).  Nothing
@@ -4539,14 +4597,43 @@ void launch_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, int n_seg, 
 // marked in `out` (method -1) for the caller's fallback.
 template <typename F>
 krylov_result_t finish_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, int n_seg, const double* rhs,
-							   double* z, esl_solve_opts o, const pss_view_t& sc, bool reduced, F&& fp64_view,
-							   set_results_t* out = nullptr, bool staged = false)
+							   double* z, esl_solve_opts o, const pss_view_t& sc, bool reduced, rb_setup_t su,
+							   F&& fp64_view, set_results_t* out = nullptr, bool staged = false)
 {
 	ESL_HIP(hipStreamSynchronize(c.stream));
 	const int B = S.B;
 	set_results_t sr;
 	sr.method.assign(B, 0);
 	krylov_result_t kr = collect_sets(c, sc, B, o.tol, false, &sr.res, &sr.its, &sr.tspan, staged);
+	if (reduced && su.n_seg && kr.missed > 0)
+	{
+		k_rb_move<<<B, sblock, 0, c.stream>>>(S, su, sc.res, o.tol, z, sc.stl);
+		ESL_HIP(hipGetLastError());
+		std::vector<int32_t> moved;
+		read_host(c, moved, sc.stl, (size_t)B);
+		const int n_moved = (int)std::count(moved.begin(), moved.end(), 1);
+		if (n_moved)
+		{
+			su.x0 = nullptr;
+			su.only = sc.stl;
+			launch_per_set(c, S, nb, n_seg, rhs, z, o, sc, path_reduced, su);
+			std::vector<double> res2;
+			std::vector<int32_t> its2;
+			const krylov_result_t k2 = collect_sets(c, sc, B, o.tol, false, &res2, &its2);
+			for (int b = 0; b < B; ++b)
+				if (moved[b])
+				{
+					sr.res[b] = res2[b];
+					sr.its[b] += its2[b];
+					kr.iters = std::max(kr.iters, sr.its[b]);
+					kr.iters_sum += its2[b];
+				}
+			kr.finished += n_moved;
+			kr.missed = k2.missed;
+			kr.resid = k2.resid;
+			kr.cycles += k2.cycles;
+		}
+	}
 	if ((o.precision == 1 || reduced) && kr.missed > 0)
 	{
 		const bool mixed = o.precision == 1;
@@ -4566,7 +4653,7 @@ krylov_result_t finish_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, 
 			sr.res[b] = res2[b];
 			sr.its[b] += its2[b];
 		}
-		kr.finished = kr.missed;
+		kr.finished += kr.missed;
 		kr.fp64_fallback = mixed ? kr.missed : 0;
 		kr.missed = k2.missed;
 		kr.resid = k2.resid;
@@ -4682,8 +4769,8 @@ struct plan_t
 	sys_t sys(int B, const double* rates) const;
 	rb_setup_t setup(const double* warm) const
 	{
-		return rb_setup_t{ x0.get(), d_seg_off.get(), n_seg, rb.anchor, rb.invd, rb.rhs, n_seg ? warm : nullptr, d_tpos.get(),
-						   g->n_t };
+		return rb_setup_t{ x0.get(), d_seg_off.get(), n_seg,	rb.anchor, rb.invd, rb.rhs, n_seg ? warm : nullptr,
+						   d_tpos.get(), g->n_t, nullptr };
 	}
 };
 
@@ -4712,7 +4799,8 @@ int dw_restart(int requested, int64_t nU, int cb)
 }
 
 // throw_on_miss = false leaves sets above the tolerance to the caller (kr.missed);
-// setup: the reduced solver sets itself up (rhs, z and S.invd need no values)
+// setup: the reduced solver may move anchors, and where it has x0 sets itself up (rhs, z
+// and S.invd need no values)
 krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* rhs_p, double* z_p,
 							 const esl_solve_opts& opts, const nbr_store_t* prebuilt = nullptr, bool device_wide = false,
 							 bool throw_on_miss = true, std::vector<double>* set_res = nullptr,
@@ -4742,7 +4830,7 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 		const bool reduced = reduced_variant(c, S, nb, o, path) != nullptr;
 		sc.reserve(B, nU, m, opts.precision, reduced);
 		launch_per_set(c, S, nb, n_seg, rhs_p, z_p, o, sc.view(), path);
-		kr = finish_per_set(c, S, nb, n_seg, rhs_p, z_p, o, sc.view(), reduced, [&] {
+		kr = finish_per_set(c, S, nb, n_seg, rhs_p, z_p, o, sc.view(), reduced, setup ? *setup : rb_setup_t{}, [&] {
 			sc.reserve(B, nU, m, 0, false);
 			return sc.view();
 		});
@@ -4780,20 +4868,24 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 				rbw_ws_t own;
 				rbw_ws_t& ws = plan_ws ? *plan_ws : own;
 				bicg_w_t gm(c, Sc, nb, ws, nseg1);
-				if (setup)
-				{
-					rb_setup_t su = *setup;
+				rb_setup_t su = setup ? *setup : rb_setup_t{};
+				if (su.n_seg)
 					su.anchor += (int64_t)b0 * nseg1;
-					if (su.warm)
-						su.warm += (int64_t)b0 * su.n_t;
+				if (su.warm)
+					su.warm += (int64_t)b0 * su.n_t;
+				if (su.x0)
 					gm.enter(su);
+				else
+				{
+					gm.enter(rhs_c, z_c);
+					gm.movable(su);
+				}
+				done = gm.solve(tol, max_iters);
+				const bool anew = su.x0 || gm.moved; // anchors, and what goes with them, are the solver's
+				if (anew)
 					k_rhs<<<dim3(ceil_div(nU, sblock), cb), sblock, 0, c.stream>>>(Sc, nseg1, su.x0,
 																				   su.rhs + (int64_t)b0 * nU);
-				}
-				else
-					gm.enter(rhs_c, z_c);
-				done = gm.solve(tol, max_iters);
-				gm.leave(z_c, setup ? setup->invd + (int64_t)b0 * nU : nullptr);
+				gm.leave(z_c, anew ? su.invd + (int64_t)b0 * nU : nullptr);
 				cres = std::move(gm.h_res);
 				cmax = gm.final_res;
 				it = gm.iters;
@@ -5603,7 +5695,7 @@ void plan_run(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_final
 			esl_solve_opts of = o;
 			of.restart = m;
 			set_results_t sr;
-			kr = finish_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, of, P.rb.ps, reduced, [&] {
+			kr = finish_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, of, P.rb.ps, reduced, P.setup(nullptr), [&] {
 				P.scr.reserve(B, P.nU, m, 0, false);
 				P.use_own_bufs();
 				return P.rb.ps;
@@ -5797,7 +5889,7 @@ void plan_solve_noalloc(ctx_t& c, void* p, int B, const double* d_rates, double*
 			const pss_view_t ps = P.rb.ps;
 			set_results_t sr;
 			kr = finish_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, o, ps,
-								plan_reduced(c, P, B, o), [&] { return ps; }, &sr);
+								plan_reduced(c, P, B, o), P.setup(nullptr), [&] { return ps; }, &sr);
 			// no exact fallback here (its dense matrix would need an allocation)
 			plan_finish_sets(c, P, B, d_rates, d_final, o, kr, std::move(sr), kr.finished > 0, false);
 		}
@@ -6106,7 +6198,7 @@ void many_per_set(ctx_t& c, const std::vector<int>& conc, void* const* plans, co
 			set_results_t sr;
 			krylov_result_t kr =
 				finish_per_set(c, P.sys(B[i], d_rates[i]), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, of, P.rb.ps,
-							   plan_reduced(c, P, B[i], of), [&] {
+							   plan_reduced(c, P, B[i], of), P.setup(nullptr), [&] {
 					P.scr.reserve(B[i], P.nU, of.restart, 0, false);
 					P.use_own_bufs();
 					return P.rb.ps;
@@ -6401,7 +6493,8 @@ void solution_full(ctx_t& c, graph_t& g, const double* d_rates, const esl_solve_
 		k_rhs<<<gu, sblock, 0, c.stream>>>(S, n_seg, nullptr, rhs.get());
 		k_zero<double><<<ceil_div(nUt, sblock), sblock, 0, c.stream>>>(nUt, z.get());
 		ESL_HIP(hipGetLastError());
-		krylov_solve(c, S, n_seg, rhs.get(), z.get(), opts, &nb);
+		const rb_setup_t su{ nullptr, d_seg_off.get(), n_seg, anchor.get(), invd.get(), rhs.get(), nullptr, nullptr, 0, nullptr };
+		krylov_solve(c, S, n_seg, rhs.get(), z.get(), opts, &nb, false, true, nullptr, path_reduced, nullptr, &su);
 		k_seg_sum<<<dim3(n_seg, 1), sblock, 0, c.stream>>>(nUt, d_seg_off.get(), z.get(), invd.get(), n_seg,
 														  segsum.get());
 		k_times_invd<<<ceil_div(nUt, sblock), sblock, 0, c.stream>>>(nUt, z.get(), invd.get(), pi.get());
