@@ -5696,8 +5696,7 @@ void plan_run(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_final
 			of.restart = m;
 			set_results_t sr;
 			kr = finish_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, of, P.rb.ps, reduced, P.setup(nullptr), [&] {
-				P.scr.reserve(B, P.nU, m, 0, false);
-				P.use_own_bufs();
+				plan_reserve(P, B, m, 0, false); // captured graphs are told of a basis that moved
 				return P.rb.ps;
 			}, &sr, staged);
 			// the final vectors are rebuilt when a second launch finished sets
@@ -6199,8 +6198,7 @@ void many_per_set(ctx_t& c, const std::vector<int>& conc, void* const* plans, co
 			krylov_result_t kr =
 				finish_per_set(c, P.sys(B[i], d_rates[i]), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, of, P.rb.ps,
 							   plan_reduced(c, P, B[i], of), P.setup(nullptr), [&] {
-					P.scr.reserve(B[i], P.nU, of.restart, 0, false);
-					P.use_own_bufs();
+					plan_reserve(P, B[i], of.restart, 0, false);
 					return P.rb.ps;
 				}, &sr);
 			plan_finish_sets(c, P, B[i], d_rates[i], d_final[i], of, kr, std::move(sr), kr.finished > 0, true);
