@@ -17,9 +17,12 @@
 	{                                                                                                          \
 		hipError_t e_ = (call);                                                                                \
 		if (e_ != hipSuccess)                                                                                  \
+		{                                                                                                      \
+			(void)hipGetLastError(); /* reported here, and not by the next launch's check too */               \
 			throw ::esl::error(e_ == hipErrorOutOfMemory ? ESL_E_OOM : ESL_E_DEVICE,                           \
 							   std::string(#call) + ": " + hipGetErrorString(e_) + " (" + __FILE__ + ":" +    \
 								   std::to_string(__LINE__) + ")");                                            \
+		}                                                                                                      \
 	} while (0)
 
 namespace esl {
