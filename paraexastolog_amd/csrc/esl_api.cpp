@@ -137,8 +137,10 @@ esl_status esl_ctx_create(int device, esl_ctx** out)
 			ctx->c.lds_per_block = lds;
 		for (auto& e : ctx->c.ev)
 			ESL_HIP(hipEventCreate(&e));
-		ctx->c.flags.ensure(64);
-		ESL_HIP(hipHostMalloc((void**)&ctx->c.h_flags, 64 * sizeof(int32_t), hipHostMallocDefault));
+		ctx->c.flags.ensure(esl::flag_words);
+		ESL_HIP(hipHostMalloc((void**)&ctx->c.h_flags, (esl::flag_words + esl::live_words) * sizeof(int32_t),
+							  hipHostMallocDefault));
+		ctx->c.h_live = ctx->c.h_flags + esl::flag_words;
 		ctx->c.h_stage_bytes = esl::stage_bytes;
 		ESL_HIP(hipHostMalloc((void**)&ctx->c.h_stage, ctx->c.h_stage_bytes, hipHostMallocDefault));
 		esl::noalloc_init(ctx->c);
@@ -766,7 +768,7 @@ esl_status esl_device_alloc(esl_ctx* ctx, size_t bytes, void** out)
 	return guarded(ctx, [&] {
 		require(ctx && out, ESL_E_ARG, "null argument");
 		set_device(ctx);
-		ESL_HIP(hipMalloc(out, bytes ? bytes : 1));
+		ESL_HIP(ctx->c.pool->alloc(out, bytes ? bytes : 1));
 	});
 }
 

@@ -101,17 +101,34 @@ struct buf_pool_t
 		for (const block_t& b : out)
 			(void)hipFree(b.p);
 	}
+	// hipMalloc, once more without the kept blocks
+	hipError_t alloc(void** p, size_t bytes)
+	{
+		const hipError_t e = hipMalloc(p, bytes);
+		if (e != hipErrorOutOfMemory)
+			return e;
+		(void)hipGetLastError();
+		clear(false);
+		return hipMalloc(p, bytes);
+	}
 	~buf_pool_t() { clear(true); }
 };
 
 // pool of the context whose call the thread is in (the library's own host threads:
 // of their child context); buffers of another context are freed, not given back
 inline thread_local std::shared_ptr<buf_pool_t> tl_pool;
+// pool that gives its memory back where a call whose buffers do not come from it runs out
+inline thread_local std::shared_ptr<buf_pool_t> tl_spare;
 struct pool_scope_t
 {
+	std::shared_ptr<buf_pool_t>& at;
 	std::shared_ptr<buf_pool_t> before;
-	explicit pool_scope_t(std::shared_ptr<buf_pool_t> p) : before(std::move(tl_pool)) { tl_pool = std::move(p); }
-	~pool_scope_t() { tl_pool = std::move(before); }
+	explicit pool_scope_t(std::shared_ptr<buf_pool_t> p, std::shared_ptr<buf_pool_t>& where = tl_pool)
+		: at(where), before(std::move(where))
+	{
+		at = std::move(p);
+	}
+	~pool_scope_t() { at = std::move(before); }
 };
 
 // Owning device buffer.
@@ -164,13 +181,11 @@ struct dbuf
 				return;
 			}
 		}
-		hipError_t e = hipMalloc(&p, bytes);
-		if (e == hipErrorOutOfMemory && pool)
-		{
-			(void)hipGetLastError();
-			pool->clear(false);
-			e = hipMalloc(&p, bytes);
-		}
+		void* q = nullptr;
+		const hipError_t e = pool		? pool->alloc(&q, bytes)
+							 : tl_spare ? tl_spare->alloc(&q, bytes)
+										: hipMalloc(&q, bytes);
+		p = static_cast<T*>(q);
 		if (e != hipSuccess)
 		{
 			p = nullptr;
@@ -275,6 +290,8 @@ struct prof_t
 	}
 };
 
+constexpr int flag_words = 64, live_words = 2 * 1024;
+
 struct ctx_t
 {
 	int device = 0;
@@ -287,6 +304,7 @@ struct ctx_t
 	dbuf<int32_t> flags;	// small device counters / flags
 	dbuf<int32_t> scan_sums; // block sums of exclusive_scan_i32
 	int32_t* h_flags = nullptr; // pinned mirror
+	int32_t* h_live = nullptr;	// pinned, after the mirror: the device-wide solver's sets, twice
 	// pinned staging of the per-set outputs of a launch, read back in one copy
 	// (allocated with the context: calls that may not allocate use it too)
 	unsigned char* h_stage = nullptr;

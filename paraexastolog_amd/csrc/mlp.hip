@@ -518,6 +518,7 @@ namespace {
 esl_status mlp_guard(esl_ctx* ctx, const std::function<void()>& f)
 {
 	// same contract as the other entry points: no exception crosses the ABI
+	const esl::pool_scope_t scope(ctx ? esl::ctx_impl(ctx).pool : nullptr, esl::tl_spare);
 	try
 	{
 		f();

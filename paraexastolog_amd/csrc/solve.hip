@@ -3867,39 +3867,16 @@ struct gmres_w_t
 	}
 };
 
-// buffers of the device-wide reduced solver, kept with the plan between solves
+// Buffers of a device-wide reduced solve: nine vectors of unknowns x sets (1 GB for 64
+// sets of 221,184 unknowns), so they are the call's, not the plan's; the context's pool
+// keeps its bound of them.  Kept with every plan, they took 1 % off calls of 5 to 50 ms
+// and made several large plans run out of memory.
 struct rbw_ws_t
 {
 	dbuf<double> x, b, c, dj, res, keep, part, norms, pick_v, pa;
 	dbuf<double> vec; // the vectors of the cycle: six on the kept rows, one on the others
 	dbuf<rbw_set_t> st;
 	dbuf<int32_t> undo, pick_u, seg_rows;
-	// liveness after each iteration, written by the device (two iterations deep)
-	int32_t* h_live = nullptr;
-	size_t n_live = 0;
-	hipEvent_t ev[2] = { nullptr, nullptr };
-	rbw_ws_t() = default;
-	rbw_ws_t(const rbw_ws_t&) = delete;
-	rbw_ws_t& operator=(const rbw_ws_t&) = delete;
-	void reset()
-	{
-		for (dbuf<double>* d : { &x, &b, &c, &dj, &res, &keep, &part, &norms, &pick_v, &pa, &vec })
-			d->reset();
-		st.reset();
-		for (dbuf<int32_t>* d : { &undo, &pick_u, &seg_rows })
-			d->reset();
-		if (h_live)
-			(void)hipHostFree(h_live);
-		h_live = nullptr;
-		n_live = 0;
-		for (hipEvent_t& e : ev)
-		{
-			if (e)
-				(void)hipEventDestroy(e);
-			e = nullptr;
-		}
-	}
-	~rbw_ws_t() { reset(); }
 	void reserve(int64_t nE, int64_t nR, int B, int nblk, int n_seg, int slices)
 	{
 		const size_t cU = (size_t)(nE + nR) * B, cR = (size_t)nR * B, cE = (size_t)nE * B;
@@ -3915,17 +3892,6 @@ struct rbw_ws_t
 		seg_rows.ensure((size_t)2 * (n_seg + 1));
 		st.ensure(B);
 		undo.ensure((size_t)2 * B);
-		if (n_live < (size_t)2 * B)
-		{
-			if (h_live)
-				ESL_HIP(hipHostFree(h_live));
-			h_live = nullptr;
-			ESL_HIP(hipHostMalloc((void**)&h_live, (size_t)2 * B * sizeof(int32_t), hipHostMallocDefault));
-			n_live = (size_t)2 * B;
-		}
-		for (hipEvent_t& e : ev)
-			if (!e)
-				ESL_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
 	}
 };
 
@@ -3947,12 +3913,16 @@ struct bicg_w_t
 	std::vector<double> h_res; // relative residuals of the last check
 	int iters = 0, cycles = 0;
 	double final_res = 0.0;
+	static constexpr int live_ev = timer_t::first + timer_t::most; // the context's events of the last two iterations
+	static_assert(live_ev + 2 <= (int)(sizeof(ctx_t::ev) / sizeof(hipEvent_t)), "as many events");
 	rb_setup_t su{};	// segments and anchors, where these may be moved
 	bool moved = false; // anchors were
 
 	bicg_w_t(ctx_t& ctx, const sys_t& sys, const nbr_store_t& nb, rbw_ws_t& w, int nseg)
 		: c(ctx), S(sys), NB(nb), ws(w), n_seg(nseg), B(sys.B), G(nb.rview())
 	{
+		if (2 * B > live_words)
+			throw error(ESL_E_ARG, "the device-wide solver takes at most 1024 rate sets per call");
 		// up to 64 sets (an even share) side by side, two to a lane where the batch is
 		// even, and as many rows as fill the block
 		W = B % 2 ? 1 : 2;
@@ -4087,8 +4057,8 @@ struct bicg_w_t
 
 	bool live_after(int j)
 	{
-		ESL_HIP(hipEventSynchronize(ws.ev[j & 1]));
-		const int32_t* f = ws.h_live + (size_t)(j & 1) * B;
+		ESL_HIP(hipEventSynchronize(c.ev[live_ev + (j & 1)]));
+		const int32_t* f = c.h_live + (size_t)(j & 1) * B;
 		return std::any_of(f, f + B, [](int32_t v) { return v != 0; });
 	}
 
@@ -4098,7 +4068,7 @@ struct bicg_w_t
 		const rbw_set_t* st = ws.st.get();
 		const double *cc = ws.c.get(), *dj = ws.dj.get();
 		double* part = ws.part.get();
-		int32_t* live = ws.h_live + (size_t)(j & 1) * B;
+		int32_t* live = c.h_live + (size_t)(j & 1) * B;
 		// algorithmic bytes: each vector and coefficient the step reads or writes once
 		const double eb = 8.0 * G.nE * B, rb = 8.0 * G.nR * B, st_b = 16.0 * NB.rgroups;
 		for (int half = 0; half < 2; ++half)
@@ -4132,7 +4102,7 @@ struct bicg_w_t
 			}
 		}
 		ESL_HIP(hipGetLastError());
-		ESL_HIP(hipEventRecord(ws.ev[j & 1], c.stream));
+		ESL_HIP(hipEventRecord(c.ev[live_ev + (j & 1)], c.stream));
 	}
 
 	// false when sets are left above the tolerance
@@ -4699,7 +4669,6 @@ struct plan_t
 	dbuf<double> p0, p1, invd, rhs, z, y, segsum;
 	dbuf<int32_t> anchor;
 	per_set_scratch_t scr;
-	rbw_ws_t wide_ws; // device-wide reduced solver
 	// the buffers the run being enqueued uses: the ones above (plan_reserve), or
 	// slices of the library's static scratch (plan_run_noalloc)
 	struct run_bufs_t
@@ -4804,8 +4773,7 @@ int dw_restart(int requested, int64_t nU, int cb)
 krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* rhs_p, double* z_p,
 							 const esl_solve_opts& opts, const nbr_store_t* prebuilt = nullptr, bool device_wide = false,
 							 bool throw_on_miss = true, std::vector<double>* set_res = nullptr,
-							 int path = path_reduced, rbw_ws_t* plan_ws = nullptr,
-							 const rb_setup_t* setup = nullptr)
+							 int path = path_reduced, const rb_setup_t* setup = nullptr)
 {
 	krylov_result_t kr;
 	const int64_t nU = S.nU;
@@ -4865,8 +4833,7 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 			const bool reduced = path == path_reduced && opts.preconditioner == 0;
 			if (reduced)
 			{
-				rbw_ws_t own;
-				rbw_ws_t& ws = plan_ws ? *plan_ws : own;
+				rbw_ws_t ws;
 				bicg_w_t gm(c, Sc, nb, ws, nseg1);
 				rb_setup_t su = setup ? *setup : rb_setup_t{};
 				if (su.n_seg)
@@ -4890,14 +4857,8 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 				cmax = gm.final_res;
 				it = gm.iters;
 				cy = gm.cycles;
-				if (!done)
-				{
-					// sets that stalled: GMRES below, which needs the room
-					ESL_HIP(hipStreamSynchronize(c.stream));
-					ws.reset();
-					if (opts.precision == 1)
-						kr.fp64_fallback += cb;
-				}
+				if (!done && opts.precision == 1)
+					kr.fp64_fallback += cb; // by GMRES below, once the workspace is given back
 			}
 			else if (opts.precision == 1)
 			{
@@ -5384,7 +5345,7 @@ void plan_enqueue(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_f
 	plan_enqueue_post(c, P, B, d_rates, d_final, !fork);
 }
 
-void plan_reserve_(plan_t& P, int B, int m, int precision, bool reduced);
+void plan_reserve_(plan_t& P, int B, int m, int precision, bool reduced, bool masses);
 
 // The schedule of a run: the tuned one when the caller asks for restart 0, else
 // the reduced solver -- unless a restart length asks for GMRES.
@@ -5404,8 +5365,9 @@ bool runs_per_set(const plan_t& P, int B, bool tuned)
 }
 
 // grows the per-run buffers; a captured graph holds their addresses, so any
-// reallocation bumps the plan's epoch (part of every graph key)
-void plan_reserve(plan_t& P, int B, int m, int precision, bool reduced)
+// reallocation bumps the plan's epoch (part of every graph key).  masses: for a run that
+// sets up GMRES (the reduced solvers set themselves up)
+void plan_reserve(plan_t& P, int B, int m, int precision, bool reduced, bool masses)
 {
 	auto ptrs = [&] {
 		return std::vector<const void*>{ P.p0.get(),	 P.p1.get(),	  P.anchor.get(), P.invd.get(),
@@ -5415,16 +5377,19 @@ void plan_reserve(plan_t& P, int B, int m, int precision, bool reduced)
 										 P.scr.tspan.get(), P.scr.xk.get(), P.scr.Vf.get(), P.scr.Vd.get() };
 	};
 	const auto before = ptrs();
-	plan_reserve_(P, B, m, precision, reduced);
+	plan_reserve_(P, B, m, precision, reduced, masses);
 	if (ptrs() != before)
 		++P.epoch;
 }
 
-void plan_reserve_(plan_t& P, int B, int m, int precision, bool reduced)
+void plan_reserve_(plan_t& P, int B, int m, int precision, bool reduced, bool masses)
 {
 	const int64_t nU = std::max<int64_t>(P.nU, 1), nUt = std::max<int64_t>(P.nUt, 1);
-	P.p0.ensure((size_t)B * nUt);
-	P.p1.ensure((size_t)B * nUt);
+	if (masses)
+	{
+		P.p0.ensure((size_t)B * nUt);
+		P.p1.ensure((size_t)B * nUt);
+	}
 	P.anchor.ensure((size_t)B * std::max(P.n_seg, 1));
 	P.invd.ensure((size_t)B * nU);
 	P.rhs.ensure((size_t)B * nU);
@@ -5642,7 +5607,7 @@ void plan_run(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_final
 	if (per_set)
 	{
 		const bool reduced = plan_reduced(c, P, B, o);
-		plan_reserve(P, B, m, o.precision, reduced);
+		plan_reserve(P, B, m, o.precision, reduced, !reduced);
 		const bool use_graph = o.graph != 0;
 		if (use_graph)
 		{
@@ -5696,7 +5661,7 @@ void plan_run(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_final
 			of.restart = m;
 			set_results_t sr;
 			kr = finish_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, of, P.rb.ps, reduced, P.setup(nullptr), [&] {
-				plan_reserve(P, B, m, 0, false); // captured graphs are told of a basis that moved
+				plan_reserve(P, B, m, 0, false, false); // captured graphs are told of a basis that moved
 				return P.rb.ps;
 			}, &sr, staged);
 			// the final vectors are rebuilt when a second launch finished sets
@@ -5707,15 +5672,15 @@ void plan_run(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_final
 	}
 	else
 	{
-		// one large system: device-wide GMRES (host-driven restarts)
-		plan_reserve(P, B, 0, 0, true);
-		const rb_setup_t su = P.setup(o.warm_pi);
+		// one large system: device-wide, driven from the host
 		const bool reduced = P.path == path_reduced && o.preconditioner == 0;
+		plan_reserve(P, B, 0, 0, reduced, !reduced);
+		const rb_setup_t su = P.setup(o.warm_pi);
 		if (!reduced)
 			plan_enqueue_setup(c, P, B, d_rates, o);
 		set_results_t sr;
 		kr = krylov_solve(c, P.sys(B, d_rates), P.n_seg, P.rb.rhs, P.rb.z, o, &P.nbr, true, false, &sr.res, P.path,
-						  &P.wide_ws, reduced ? &su : nullptr);
+						  reduced ? &su : nullptr);
 		plan_enqueue_post(c, P, B, d_rates, d_final);
 		if ((int)sr.res.size() != B)
 			sr.res = set_residuals(c, P.sys(B, d_rates), P.n_seg, P.rb.rhs, P.rb.z);
@@ -5982,8 +5947,9 @@ struct child_ctx_t
 		ESL_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
 		for (auto& e : c.ev)
 			ESL_HIP(hipEventCreate(&e));
-		c.flags.ensure(64);
-		ESL_HIP(hipHostMalloc((void**)&c.h_flags, 64 * sizeof(int32_t), hipHostMallocDefault));
+		c.flags.ensure(flag_words);
+		ESL_HIP(hipHostMalloc((void**)&c.h_flags, (flag_words + live_words) * sizeof(int32_t), hipHostMallocDefault));
+		c.h_live = c.h_flags + flag_words;
 		c.h_stage_bytes = stage_bytes;
 		ESL_HIP(hipHostMalloc((void**)&c.h_stage, c.h_stage_bytes, hipHostMallocDefault));
 	}
@@ -5995,6 +5961,7 @@ struct child_ctx_t
 			(void)hipStreamSynchronize(c.stream);
 			(void)hipStreamDestroy(c.stream);
 		}
+		c.pool->clear(true); // plans may hold buffers of it: freed directly from here on
 		for (auto& e : c.ev)
 			if (e)
 				(void)hipEventDestroy(e);
@@ -6088,8 +6055,11 @@ void many_per_set(ctx_t& c, const std::vector<int>& conc, void* const* plans, co
 	if (conc.empty())
 		return;
 	for (int i : conc)
-		plan_reserve(*static_cast<plan_t*>(plans[i]), B[i], po[i].restart, o.precision,
-					 plan_reduced(c, *static_cast<plan_t*>(plans[i]), B[i], po[i]));
+	{
+		plan_t& P = *static_cast<plan_t*>(plans[i]);
+		const bool reduced = plan_reduced(c, P, B[i], po[i]);
+		plan_reserve(P, B[i], po[i].restart, o.precision, reduced, !reduced);
+	}
 	ensure_aux(c, (int)conc.size());
 	timer_t tm_(c);
 	auto enqueue_all = [&] {
@@ -6198,7 +6168,7 @@ void many_per_set(ctx_t& c, const std::vector<int>& conc, void* const* plans, co
 			krylov_result_t kr =
 				finish_per_set(c, P.sys(B[i], d_rates[i]), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, of, P.rb.ps,
 							   plan_reduced(c, P, B[i], of), P.setup(nullptr), [&] {
-					plan_reserve(P, B[i], of.restart, 0, false);
+					plan_reserve(P, B[i], of.restart, 0, false, false);
 					return P.rb.ps;
 				}, &sr);
 			plan_finish_sets(c, P, B[i], d_rates[i], d_final[i], of, kr, std::move(sr), kr.finished > 0, true);
@@ -6492,7 +6462,7 @@ void solution_full(ctx_t& c, graph_t& g, const double* d_rates, const esl_solve_
 		k_zero<double><<<ceil_div(nUt, sblock), sblock, 0, c.stream>>>(nUt, z.get());
 		ESL_HIP(hipGetLastError());
 		const rb_setup_t su{ nullptr, d_seg_off.get(), n_seg, anchor.get(), invd.get(), rhs.get(), nullptr, nullptr, 0, nullptr };
-		krylov_solve(c, S, n_seg, rhs.get(), z.get(), opts, &nb, false, true, nullptr, path_reduced, nullptr, &su);
+		krylov_solve(c, S, n_seg, rhs.get(), z.get(), opts, &nb, false, true, nullptr, path_reduced, &su);
 		k_seg_sum<<<dim3(n_seg, 1), sblock, 0, c.stream>>>(nUt, d_seg_off.get(), z.get(), invd.get(), n_seg,
 														  segsum.get());
 		k_times_invd<<<ceil_div(nUt, sblock), sblock, 0, c.stream>>>(nUt, z.get(), invd.get(), pi.get());
