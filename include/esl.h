@@ -152,7 +152,8 @@ typedef struct
 	int precision;		 /* 0 = FP64 Krylov solves; 1 = FP32 inner solves + FP64 residual refinement (where
 						  * GMRES runs; the default method holds its vectors in FP64 either way) */
 	double tol;			 /* relative residual target of every linear solve (default 1e-13) */
-	int max_iters;		 /* Krylov iterations per solve before ESL_E_NUMERIC (default 20000) */
+	int max_iters;		 /* Krylov iterations per solve (default 20000); GMRES has as many for the sets that
+						  * the default method leaves, before ESL_E_NUMERIC */
 	int restart;		 /* > 0 asks for restarted GMRES with this restart length: at most 64 for the
 						  * per-set solvers, 128 for the device-wide solver; 0 (default): a plan's
 						  * autotuned schedule, else the default method, BiCGStab on the

@@ -725,11 +725,13 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 		__threadfence_block();
 		__syncthreads();
 	}
-	// z = D' x, back in the unknown order of the caller
+	// z = D' x, back in the unknown order of the caller; zero, whose residual is 1, where a
+	// solve that ran out of products is not there yet
+	const bool keep = rel < 1.0;
 	for (int q = tid; q < nU; q += BLK)
 	{
 		const int u = G.row[q];
-		zio[off + u] = xp[q] / S.invd[off + u];
+		zio[off + u] = keep ? xp[q] / S.invd[off + u] : 0.0;
 	}
 	if (tid == 0)
 	{

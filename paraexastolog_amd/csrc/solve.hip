@@ -4875,10 +4875,14 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 			}
 			if (!done)
 			{
-				// FP64 from the current iterate (also what an FP32 solve that stalled falls back to)
+				// FP64 from the current iterate (also what an FP32 solve that stalled falls back to);
+				// after the reduced solver from zero, whose residual is 1, where that is no worse
+				for (int b = 0; reduced && b < cb; ++b)
+					if (!(cres[b] < 1.0))
+						k_zero<double><<<ceil_div(nU, sblock), sblock, 0, c.stream>>>(nU, z_c + (int64_t)b * nU);
 				gmres_w_t<double> gm(c, Sc, nb, nseg1, dw_restart(opts.restart, nU, cb), ilu);
 				gm.enter(rhs_c, z_c);
-				const bool done64 = gm.solve(tol, std::max(max_iters - it, 1));
+				const bool done64 = gm.solve(tol, reduced ? max_iters : std::max(max_iters - it, 1));
 				gm.leave(z_c);
 				cres = gm.h_res;
 				cmax = gm.final_res;
