@@ -590,6 +590,19 @@ void plan_by_rows(esl::ctx_t& c, esl_mlp* m)
 	m->by_rows = true;
 }
 
+// Whether a forward pass goes by rows.  For narrow networks the time of many rows is
+// that of the vector work, of which a row takes more there (hidden widths are padded to
+// 128); launches no longer matter then.  Layers / rows, us: 16 wide with one hidden layer
+// and 10 outputs 61 / 57 at 32,768 rows, 99 / 101 at 65,536, 332 / 371 at 262,144; with
+// three 73 / 68, 113 / 123, 364 / 460; with three and 300 outputs 128 / 136 at 65,536; with
+// 2,048 outputs 367 / 265.  64 wide with three, at 262,144 rows: 10 outputs 414 / 463, 300
+// outputs 571 / 515.  96 wide with three and 10 outputs 526 / 465.  Training goes by rows
+// always (2.3 to 3.7 times as fast at 65,536 rows).
+bool forward_by_rows(const esl_mlp* m, int rows)
+{
+	return m->by_rows && (rows < 65536 || m->hidden > 64 || m->n_out > (m->hidden > 32 ? 200 : 384));
+}
+
 // rows through the network and, with targets, back (enqueued)
 void run_rows(esl::ctx_t& c, esl_mlp* m, esl::mlp_batch_t& q)
 {
@@ -857,7 +870,7 @@ esl_status esl_mlp_forward(esl_ctx* ctx, esl_mlp* m, int rows, const float* d_x,
 		if (!ctx || !m || !d_x || !d_probs || rows < 1)
 			throw esl::error(ESL_E_ARG, "null argument");
 		esl::ctx_t& c = esl::ctx_impl(ctx);
-		if (m->by_rows)
+		if (forward_by_rows(m, rows))
 		{
 			esl::mlp_batch_t q{};
 			q.rows = rows, q.x = d_x, q.P = d_probs;
@@ -880,7 +893,7 @@ esl_status esl_mlp_predict_warm(esl_ctx* ctx, esl_mlp* m, int rows, const float*
 		if (!ctx || !m || !d_x || !d_warm || rows < 1)
 			throw esl::error(ESL_E_ARG, "null argument");
 		esl::ctx_t& c = esl::ctx_impl(ctx);
-		if (m->by_rows)
+		if (forward_by_rows(m, rows))
 		{
 			esl::mlp_batch_t q{};
 			q.rows = rows, q.x = d_x, q.Pd = d_warm;
