@@ -1,5 +1,5 @@
-"""Benchmark: stationary solves per second at N=20, batched FP32 + FP64
-refinement against the plain per-solve FP64 path, at <= 1e-10 L1.
+"""Benchmark: stationary solves per second at N=20, batched (tuned schedule) against
+the plain per-solve FP64 path, at <= 1e-10 L1.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--sets B] [--seed S] [--no-cpu]
 
@@ -12,7 +12,8 @@ sets (all sharing the topology and its zero pattern) on inputs resident in
 HBM.  `value` = rate sets solved per second.
 
 Also measured (in the same JSON line):
-  plain    the per-solve FP64 path, one rate set per call, graph reused;
+  plain    the per-solve FP64 path with default options, one rate set per call,
+           graph reused; the same with GMRES (restart 32) beside it;
   plain_full  table + graph + FP64 solve per rate set (the reference's flow);
   accuracy L1 and max-relative error of the batched results against the
            plain FP64 results (and the oracle for one set);
@@ -368,17 +369,21 @@ def main():
         check(L.esl_plan_solve(ctx.handle, pl, count, d_r, d_out, C.byref(o), C.byref(rep)), ctx.handle)
         return rep
 
-    # ---- plain FP64, one rate set per call (plan reused)
-    plain_times = []
-    plain_reports = []
-    for k in range(n_check):
-        r_k = C.c_void_p(d_rates.value + 8 * 2 * N * k)
-        out_k = C.c_void_p(d_plain.value + 8 * n * k)
-        t = time.perf_counter()
-        rep = solve_batch(1, r_k, out_k, 0, 1e-13)
-        plain_times.append(time.perf_counter() - t)
-        plain_reports.append(rep.as_dict())
-    plain_s = float(np.median(plain_times[1:] if len(plain_times) > 1 else plain_times))
+    # ---- plain FP64, one rate set per call (plan reused): GMRES, then what a call
+    # with default options does (its results are kept)
+    def plain(restart):
+        times, reps = [], []
+        for k in range(n_check):
+            r_k = C.c_void_p(d_rates.value + 8 * 2 * N * k)
+            out_k = C.c_void_p(d_plain.value + 8 * n * k)
+            t = time.perf_counter()
+            rep = solve_batch(1, r_k, out_k, 0, 1e-13, restart=restart)
+            times.append(time.perf_counter() - t)
+            reps.append(rep.as_dict())
+        return float(np.median(times[1:] if len(times) > 1 else times)), reps
+
+    plain_gmres_s, _ = plain(32)
+    plain_s, plain_reports = plain(0)
 
     # ---- plain, full reference flow per rate set: table + graph + FP64 solve
     full_times = []
@@ -397,7 +402,7 @@ def main():
         full_times.append(time.perf_counter() - t)
         del tb
     # restore set 0's plain result (buffer 0 was reused above)
-    solve_batch(1, d_rates, d_plain, 0, 1e-13)
+    solve_batch(1, d_rates, d_plain, 0, 1e-13, restart=0)
     plain_full_s = float(np.median(full_times))
 
     # ---- batched + refined: the autotuner picks the schedule on this batch, then
@@ -523,6 +528,11 @@ def main():
     oracle_l1 = float(np.abs(xp[0] - xo).sum()) if xo is not None else None
 
     rep0 = reports[-1]
+    # the parity-reduced method holds its vectors in FP64 in both precisions
+    reduced = schedule is not None and schedule["path"] == SCHEDULE_NAMES[5]
+    mixed = a.precision == 1 and not reduced
+    method = ("BiCGStab on the parity-reduced system, FP64" if reduced else
+              "batched FP32 GMRES + FP64 residual refinement" if mixed else "batched FP64 GMRES")
     out = {
         "metric": "stationary solves/sec at N=20 (batched+refined vs plain FP64) at <=1e-10 L1",
         "value": value,
@@ -534,18 +544,19 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "fp32+fp64" if a.precision == 1 else "f64",
+        "dtype": "fp32+fp64" if mixed else "f64",
         "data": "synthetic",
         "config": {
             "workload": f"seeded random Boolean network N=20 (K in {{2,3}}, 5 fixed nodes), generator v1 seed "
-                        f"{a.seed}; {B} log-uniform [0.1,10] rate sets per step, batched FP32 GMRES + FP64 "
-                        f"residual refinement, tol {tol:g}",
+                        f"{a.seed}; {B} log-uniform [0.1,10] rate sets per step, {method}, "
+                        f"tol {tol:g}",
             "states": int(sizes[0]), "transitions": int(sizes[1]), "sccs": int(sizes[2]),
             "terminal_sccs": int(sizes[3]), "rate_sets": B,
             "unknowns_per_set": int(rep0["unknowns"]), "terminals_reached": int(rep0["terminals_reached"]),
         },
         "plain_fp64": {"solves_per_s": 1.0 / plain_s, "ms_per_solve": 1000 * plain_s,
                        "stage_ms": plain_reports[-1]["ms_stage"]},
+        "plain_fp64_gmres": {"solves_per_s": 1.0 / plain_gmres_s, "ms_per_solve": 1000 * plain_gmres_s},
         "plain_full_pipeline": {"solves_per_s": 1.0 / plain_full_s, "ms_per_solve": 1000 * plain_full_s},
         "speedup_vs_plain_fp64": value * plain_s,
         "shared_stages_ms": {"table": float(stage_ms[0]), "graph": float(stage_ms[1]),
@@ -563,7 +574,7 @@ def main():
                      "plain_sets_checked": n_check,
                      "plain_fp64_l1_vs_oracle": oracle_l1, "max_abs_sum_minus_1": float(sums),
                      "max_residual": max(r["residual"] for r in reports),
-                     "gmres_iterations": rep0["iterations"], "refinement_cycles": rep0["refinements"],
+                     "max_iterations": rep0["iterations"], "cycles": rep0["refinements"],
                      "mean_iterations_per_set": rep0["iterations_sum"] / B,
                      "fp64_fallback_sets": rep0["fp64_fallback"]},
         "schedule": schedule,
@@ -644,7 +655,7 @@ def _errors(x, ref):
 
 def workload_n16(a, ctx):
     """One N=16 topology (K=2, generator v1 seed 11: one terminal SCC of 2048
-    states), 1024 rate sets sharing the plan: FP64 and FP32+refinement, HIP graph
+    states), 1024 rate sets sharing the plan: both precisions, HIP graph
     off/on, autotuned schedule; against the plain per-solve FP64 path."""
     from paraexastolog_amd import synth
     from paraexastolog_amd.surrogate import DeviceArray
@@ -670,7 +681,7 @@ def workload_n16(a, ctx):
             sec, rep = _timed(lambda: tp.plan.solve(B, dr.ptr, df.ptr, precision=prec, tol=1e-12, graph=graph),
                               a.steps)
             l1, l1_med, rel = _errors(df.download()[:8], ref)
-            out[f"{'fp32+fp64' if prec else 'fp64'}_graph{graph}"] = {
+            out[f"precision{prec}_graph{graph}"] = {
                 "sets_per_s": B / sec, "ms_per_batch": 1000 * sec, "max_l1_vs_plain": l1, "max_rel_vs_plain": rel,
                 "mean_iterations": rep["iterations_sum"] / B}
     path, restart, best_ms = tp.plan.autotune(B, dr.ptr, df.ptr, precision=1, tol=1e-12, graph=1)
@@ -715,7 +726,7 @@ def workload_uneven(a, ctx):
                                                              [f.ptr for f in dfs], precision=prec, tol=1e-12,
                                                              graph=graph), a.steps)
             diff = max(np.abs(f.download() - s_).sum(axis=1).max() for f, s_ in zip(dfs, seq))
-            res[f"{'fp32+fp64' if prec else 'fp64'}_graph{graph}"] = {
+            res[f"precision{prec}_graph{graph}"] = {
                 "sets_per_s": 8 * per / sec, "ms": 1000 * sec, "sequential_sets_per_s": 8 * per / seq_s,
                 "max_l1_vs_sequential": float(diff), "max_residual": max(r["residual"] for r in reps)}
     best = max(v["sets_per_s"] for v in res.values())
@@ -757,15 +768,15 @@ def workload_seeds(a, ctx):
                 run = lambda: tp.plan.solve(B, dr.ptr, df.ptr, precision=1, tol=1e-12, graph=1, restart=0)  # noqa: E731
                 t_batch, rep = _timed(run, 1)
             else:
-                # device-wide: the faster of restart 32 and 64 (neither wins everywhere)
+                # device-wide: the fastest of the default method and GMRES at restart 32 and 64
                 best = None
-                for m in (32, 64):
+                for m in (0, 32, 64):
                     t_m, rep_m = _timed(lambda: tp.plan.solve(B, dr.ptr, df.ptr, precision=1, tol=1e-12,  # noqa: B023
                                                               restart=m), 1)
                     if best is None or t_m < best[0]:
                         best = (t_m, rep_m, m)
                 t_batch, rep, m = best
-                sched = f"device-wide, restart {m} (best of 32, 64)"
+                sched = f"device-wide, {f'GMRES at restart {m}' if m else 'parity-reduced'} (best of 3)"
             t_plain, _ = _timed(lambda: tp.plan.solve(1, dr.ptr, d1.ptr, precision=0, tol=1e-13), 1)
             xb0 = np.empty(tp.n)  # batched set 0 only
             check(L.esl_memcpy_d2h(ctx.handle, xb0.ctypes.data_as(C.c_void_p), df.ptr, 8 * tp.n), ctx.handle)
@@ -778,7 +789,7 @@ def workload_seeds(a, ctx):
             recs.append(rec)
             print(json.dumps(rec), file=sys.stderr, flush=True)
             del tp, dr, df, d1
-    out = {"metric": "rate sets/s per seed (batched FP32 + FP64 refinement) and speedup vs plain per-solve FP64",
+    out = {"metric": "rate sets/s per seed (batched, precision 1) and speedup vs plain per-solve FP64",
            "workload": "N=20 (K in {2,3}, 5 fixed nodes) seeds 0..7, N=22 (K=3 + 3 spliced 3-cycles) seeds 0..3 "
                        "and N=16 (K=2) seeds 0..3, generator v1; tol 1e-12 batched, 1e-13 plain",
            "seeds": recs}
