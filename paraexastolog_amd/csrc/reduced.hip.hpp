@@ -725,13 +725,11 @@ __device__ __forceinline__ void bicg_set_body(const sys_t& S, const rb_t& G, int
 		__threadfence_block();
 		__syncthreads();
 	}
-	// z = D' x, back in the unknown order of the caller; zero, whose residual is 1, where a
-	// solve that ran out of products is not there yet
-	const bool keep = rel < 1.0;
+	// z = D' x, back in the unknown order of the caller
 	for (int q = tid; q < nU; q += BLK)
 	{
 		const int u = G.row[q];
-		zio[off + u] = keep ? xp[q] / S.invd[off + u] : 0.0;
+		zio[off + u] = xp[q] / S.invd[off + u];
 	}
 	if (tid == 0)
 	{
@@ -809,6 +807,33 @@ __global__ __launch_bounds__(sblock) void k_rb_move(sys_t S, rb_setup_t su, cons
 	}
 	if (tid == 0)
 		moved[b] = any;
+}
+
+// For GMRES to take over the sets above the tolerance: zero for them and, where `invd` is
+// given, 1 / D' as GMRES sets it up (the device-wide solver's differs in the last bit),
+// other iterates kept.  It then starts as where it is asked for by name, so it meets a
+// bound on its iterations, or a tolerance near the rounding, as it does there.
+__global__ __launch_bounds__(sblock) void k_rb_restart(sys_t S, int n_seg, const double* __restrict__ res, double tol,
+													   double* __restrict__ z, double* __restrict__ invd)
+{
+	const int64_t u = (int64_t)blockIdx.x * sblock + threadIdx.x;
+	const int b = blockIdx.y;
+	if (u >= S.nU)
+		return;
+	const int64_t i = (int64_t)b * S.nU + u;
+	const bool left = !(res[b] <= tol);
+	if (!invd)
+	{
+		if (left)
+			z[i] = 0.0;
+		return;
+	}
+	const uint32_t st = (uint32_t)S.ulist[u];
+	const double x = z[i] * invd[i];
+	const double iv =
+		is_anchor(S, n_seg, b, u) ? 1.0 : 1.0 / out_rate_s(st, S.mask[st], S.rates + (int64_t)b * S.rate_stride);
+	invd[i] = iv;
+	z[i] = left ? 0.0 : x / iv;
 }
 
 using bicg_set_fn = void (*)(sys_t, rb_t, int, const double*, double*, rb_scratch_t, rb_setup_t, double, int, pgm_out_t);

@@ -4558,17 +4558,18 @@ void launch_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, int n_seg, 
 }
 
 // Reads the per-set results of a launch_per_set.  Sets that the reduced solver leaves
-// above the tolerance get their bad anchors moved (k_rb_move) and another go.  Sets that
-// missed it in mixed precision (their FP32 cycles stalled) or in the reduced solver are
-// finished by FP64 GMRES with ILU(0) from their current iterate; sets that already
-// converged leave it at their first residual check.
-// fp64_view() gives the scratch with an FP64 basis (it may grow it).  Nothing
-// is thrown here: sets still above the tolerance are counted in kr.missed and
+// above the tolerance get their bad anchors moved (k_rb_move) and another go; what it
+// still leaves starts over with GMRES, as where that is asked for by name (FP32 cycles
+// with refinement in mixed precision).  Sets that missed the tolerance with GMRES in mixed
+// precision (their FP32 cycles stalled) are finished by FP64 GMRES from their current
+// iterate; sets that already converged leave it at their first residual check.
+// basis(precision) gives the scratch with a basis of that precision (it may grow it).
+// Nothing is thrown here: sets still above the tolerance are counted in kr.missed and
 // marked in `out` (method -1) for the caller's fallback.
 template <typename F>
 krylov_result_t finish_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, int n_seg, const double* rhs,
 							   double* z, esl_solve_opts o, const pss_view_t& sc, bool reduced, rb_setup_t su,
-							   F&& fp64_view, set_results_t* out = nullptr, bool staged = false)
+							   F&& basis, set_results_t* out = nullptr, bool staged = false)
 {
 	ESL_HIP(hipStreamSynchronize(c.stream));
 	const int B = S.B;
@@ -4604,13 +4605,33 @@ krylov_result_t finish_per_set(ctx_t& c, const sys_t& S, const nbr_store_t& nb, 
 			kr.cycles += k2.cycles;
 		}
 	}
+	if (reduced && kr.missed > 0)
+		k_rb_restart<<<dim3(ceil_div(S.nU, sblock), B), sblock, 0, c.stream>>>(S, std::max(n_seg, 1), sc.res, o.tol, z,
+																				 nullptr);
+	if (reduced && kr.missed > 0 && o.precision == 1)
+	{
+		const pss_view_t sf = basis(1);
+		launch_per_set(c, S, nb, n_seg, rhs, z, o, sf, path_lds);
+		std::vector<double> res2;
+		std::vector<int32_t> its2;
+		const krylov_result_t k2 = collect_sets(c, sf, B, o.tol, false, &res2, &its2);
+		for (int b = 0; b < B; ++b)
+		{
+			sr.res[b] = res2[b];
+			sr.its[b] += its2[b];
+		}
+		kr.finished += kr.missed;
+		kr.missed = k2.missed;
+		kr.resid = k2.resid;
+		kr.iters += k2.iters;
+		kr.cycles += k2.cycles;
+		kr.iters_sum += k2.iters_sum;
+	}
 	if ((o.precision == 1 || reduced) && kr.missed > 0)
 	{
 		const bool mixed = o.precision == 1;
 		o.precision = 0;
-		if (reduced)
-			o.preconditioner = 2;
-		const pss_view_t sd = fp64_view();
+		const pss_view_t sd = basis(0);
 		launch_per_set(c, S, nb, n_seg, rhs, z, o, sd, path_lds);
 		ESL_HIP(hipStreamSynchronize(c.stream));
 		std::vector<double> res2;
@@ -4798,8 +4819,8 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 		const bool reduced = reduced_variant(c, S, nb, o, path) != nullptr;
 		sc.reserve(B, nU, m, opts.precision, reduced);
 		launch_per_set(c, S, nb, n_seg, rhs_p, z_p, o, sc.view(), path);
-		kr = finish_per_set(c, S, nb, n_seg, rhs_p, z_p, o, sc.view(), reduced, setup ? *setup : rb_setup_t{}, [&] {
-			sc.reserve(B, nU, m, 0, false);
+		kr = finish_per_set(c, S, nb, n_seg, rhs_p, z_p, o, sc.view(), reduced, setup ? *setup : rb_setup_t{}, [&](int prec) {
+			sc.reserve(B, nU, m, prec, false);
 			return sc.view();
 		});
 		if (kr.missed && throw_on_miss)
@@ -4816,6 +4837,7 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 		const bool ilu = opts.preconditioner != 1;
 		const int nseg1 = std::max(n_seg, 1);
 		std::vector<double> res_all;
+		dbuf<double> d_res;
 		for (int b0 = 0; b0 < B; b0 += 1024)
 		{
 			const int cb = std::min(1024, B - b0);
@@ -4857,10 +4879,17 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 				cmax = gm.final_res;
 				it = gm.iters;
 				cy = gm.cycles;
-				if (!done && opts.precision == 1)
-					kr.fp64_fallback += cb; // by GMRES below, once the workspace is given back
 			}
-			else if (opts.precision == 1)
+			const int it_r = it; // products of the reduced solver: GMRES has max_iters beside them
+			if (reduced && !done)
+			{
+				d_res.ensure(cb);
+				write_dev(c, d_res.get(), cres);
+				k_rb_restart<<<dim3(ceil_div(nU, sblock), cb), sblock, 0, c.stream>>>(
+					Sc, nseg1, d_res.get(), tol, z_c, setup ? setup->invd + (int64_t)b0 * nU : nullptr);
+				ESL_HIP(hipStreamSynchronize(c.stream));
+			}
+			if (!done && opts.precision == 1)
 			{
 				gmres_w_t<float> gm(c, Sc, nb, nseg1, dw_restart(opts.restart, nU, cb), ilu);
 				gm.enter(rhs_c, z_c);
@@ -4868,21 +4897,17 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 				gm.leave(z_c);
 				cres = gm.h_res; // the residuals of its last check
 				cmax = gm.final_res;
-				it = gm.iters;
-				cy = gm.cycles;
+				it += gm.iters;
+				cy += gm.cycles;
 				if (!done)
 					kr.fp64_fallback += cb;
 			}
 			if (!done)
 			{
-				// FP64 from the current iterate (also what an FP32 solve that stalled falls back to);
-				// after the reduced solver from zero, whose residual is 1, where that is no worse
-				for (int b = 0; reduced && b < cb; ++b)
-					if (!(cres[b] < 1.0))
-						k_zero<double><<<ceil_div(nU, sblock), sblock, 0, c.stream>>>(nU, z_c + (int64_t)b * nU);
+				// FP64 from the current iterate (also what an FP32 solve that stalled falls back to)
 				gmres_w_t<double> gm(c, Sc, nb, nseg1, dw_restart(opts.restart, nU, cb), ilu);
 				gm.enter(rhs_c, z_c);
-				const bool done64 = gm.solve(tol, reduced ? max_iters : std::max(max_iters - it, 1));
+				const bool done64 = gm.solve(tol, std::max(max_iters - (it - it_r), 1));
 				gm.leave(z_c);
 				cres = gm.h_res;
 				cmax = gm.final_res;
@@ -5664,8 +5689,8 @@ void plan_run(ctx_t& c, plan_t& P, int B, const double* d_rates, double* d_final
 			esl_solve_opts of = o;
 			of.restart = m;
 			set_results_t sr;
-			kr = finish_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, of, P.rb.ps, reduced, P.setup(nullptr), [&] {
-				plan_reserve(P, B, m, 0, false, false); // captured graphs are told of a basis that moved
+			kr = finish_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, of, P.rb.ps, reduced, P.setup(nullptr), [&](int prec) {
+				plan_reserve(P, B, m, prec, false, false); // captured graphs are told of a basis that moved
 				return P.rb.ps;
 			}, &sr, staged);
 			// the final vectors are rebuilt when a second launch finished sets
@@ -5857,7 +5882,7 @@ void plan_solve_noalloc(ctx_t& c, void* p, int B, const double* d_rates, double*
 			const pss_view_t ps = P.rb.ps;
 			set_results_t sr;
 			kr = finish_per_set(c, P.sys(B, d_rates), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, o, ps,
-								plan_reduced(c, P, B, o), P.setup(nullptr), [&] { return ps; }, &sr);
+								plan_reduced(c, P, B, o), P.setup(nullptr), [&](int) { return ps; }, &sr);
 			// no exact fallback here (its dense matrix would need an allocation)
 			plan_finish_sets(c, P, B, d_rates, d_final, o, kr, std::move(sr), kr.finished > 0, false);
 		}
@@ -6171,8 +6196,8 @@ void many_per_set(ctx_t& c, const std::vector<int>& conc, void* const* plans, co
 			set_results_t sr;
 			krylov_result_t kr =
 				finish_per_set(c, P.sys(B[i], d_rates[i]), P.nbr, P.n_seg, P.rb.rhs, P.rb.z, of, P.rb.ps,
-							   plan_reduced(c, P, B[i], of), P.setup(nullptr), [&] {
-					plan_reserve(P, B[i], of.restart, 0, false, false);
+							   plan_reduced(c, P, B[i], of), P.setup(nullptr), [&](int prec) {
+					plan_reserve(P, B[i], of.restart, prec, false, false);
 					return P.rb.ps;
 				}, &sr);
 			plan_finish_sets(c, P, B[i], d_rates[i], d_final[i], of, kr, std::move(sr), kr.finished > 0, true);
