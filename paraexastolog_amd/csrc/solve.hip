@@ -4203,7 +4203,7 @@ struct bicg_w_t
 			write_dev(c, ws.st.get(), hs);
 			const rbw_set_t* st = ws.st.get();
 			rows(nbE, 0, false, [](auto w) { return k_rbw_te0<decltype(w)::value>; }, G, geo, cc, ws.res.get(), TE, st);
-			rows(nbR, 2, true, [](auto w) { return k_rbw_init<decltype(w)::value>; }, G, geo, cc, ws.res.get(), TE, R, RH, P, X, st, ws.part.get());
+			rows(nbR, 3, true, [](auto w) { return k_rbw_init<decltype(w)::value>; }, G, geo, cc, ws.res.get(), TE, R, RH, P, X, st, ws.part.get());
 			k_rbw_reduce<1><<<B, sblock, 0, c.stream>>>(ws.part.get(), nbR, B, ws.st.get(), nullptr, nullptr, 0.0);
 			ESL_HIP(hipGetLastError());
 			for (int j = 0; 2 * j < rb_cycle_products; ++j)
