@@ -80,7 +80,7 @@ esl_status guarded(esl_ctx* ctx, F&& f)
 	const esl::pool_scope_t scope(ctx->c.pool);
 	const esl_status s = guarded_call(ctx, f);
 	if (s != ESL_OK)
-		ctx->c.pool->clear(false);
+		ctx->c.pool->clear_both();
 	return s;
 }
 
@@ -189,6 +189,7 @@ void esl_ctx_destroy(esl_ctx* ctx)
 	if (ctx->c.stream)
 		(void)hipStreamDestroy(ctx->c.stream);
 	ctx->c.pool->clear(true);
+	ctx->c.wide->clear(true);
 	delete ctx;
 }
 

@@ -33,13 +33,16 @@ namespace esl {
 // pool; 15 nodes: 4.3 to 3.8 ms).  A block is reused by work on the same context only: calls on
 // one context are serialised on its stream, so what was enqueued on a block comes
 // before what its next owner enqueues.  Small blocks cost 1.6 us a pair (115 us
-// of the 1.06 ms of a model of 10 nodes).  Blocks above a quarter of the bound are not
-// kept; the oldest leave when there are more than 512 or the bound is exceeded, all when
-// an allocation fails and when the context is destroyed (buffers that outlive it are
-// freed directly).
+// of the 1.06 ms of a model of 10 nodes).  Blocks above a quarter of the bound
+// (of 512 MB) are not kept; the oldest leave when there are more than 512 or the bound is
+// exceeded, all when an allocation fails and when the context is destroyed (buffers that
+// outlive it are freed directly).
 struct buf_pool_t
 {
-	static constexpr size_t bound = (size_t)512 << 20, least = 256, most_blocks = 512;
+	static constexpr size_t least = 256, most_blocks = 512;
+	const size_t bound, largest; // bytes kept, and of one block
+	std::weak_ptr<buf_pool_t> other; // the context's other pool
+	explicit buf_pool_t(size_t most = (size_t)512 << 20, size_t one = (size_t)128 << 20) : bound(most), largest(one) {}
 	struct block_t
 	{
 		void* p;
@@ -71,7 +74,7 @@ struct buf_pool_t
 		std::vector<block_t> out;
 		{
 			std::lock_guard<std::mutex> g(m);
-			if (closed || bytes < least || bytes > bound / 4)
+			if (closed || bytes < least || bytes > largest)
 				out.push_back({ p, bytes });
 			else
 			{
@@ -101,6 +104,13 @@ struct buf_pool_t
 		for (const block_t& b : out)
 			(void)hipFree(b.p);
 	}
+	// frees what this pool and the other one keep
+	void clear_both()
+	{
+		clear(false);
+		if (const auto o = other.lock())
+			o->clear(false);
+	}
 	// hipMalloc, once more without the kept blocks
 	hipError_t alloc(void** p, size_t bytes)
 	{
@@ -108,7 +118,7 @@ struct buf_pool_t
 		if (e != hipErrorOutOfMemory)
 			return e;
 		(void)hipGetLastError();
-		clear(false);
+		clear_both();
 		return hipMalloc(p, bytes);
 	}
 	~buf_pool_t() { clear(true); }
@@ -311,6 +321,17 @@ struct ctx_t
 	size_t h_stage_bytes = 0;
 	prof_t prof;
 	std::shared_ptr<buf_pool_t> pool = std::make_shared<buf_pool_t>();
+	// Pool of device-wide solves' workspaces, with a bound of its own, as they are large: 0.6 GB
+	// for 16 sets of 524,288 unknowns, 2.5 GB for the two device-wide plans of a batch of eight
+	// networks.  Allocated and freed by each call they took 0.6 of 25 and 4 of 65 ms.  A host
+	// thread's context shares the pool of the context that it works for.
+	std::shared_ptr<buf_pool_t> wide = std::make_shared<buf_pool_t>((size_t)2 << 30, (size_t)512 << 20);
+	bool wide_shared = false; // with another context
+	ctx_t()
+	{
+		pool->other = wide;
+		wide->other = pool;
+	}
 	// forked streams (default priority) and fork/join events for plans solved concurrently
 	std::vector<hipStream_t> aux;
 	std::vector<hipEvent_t> aux_ev;

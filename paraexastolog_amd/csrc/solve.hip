@@ -3868,17 +3868,33 @@ struct gmres_w_t
 };
 
 // Buffers of a device-wide reduced solve: nine vectors of unknowns x sets (1 GB for 64
-// sets of 221,184 unknowns), so they are the call's, not the plan's; the context's pool
-// keeps its bound of them.  Kept with every plan, they took 1 % off calls of 5 to 50 ms
-// and made several large plans run out of memory.
+// sets of 221,184 unknowns), so they are the call's, not the plan's; a pool of the context
+// keeps its bound of them.  Kept with every plan, they made several large plans run out
+// of memory.
 struct rbw_ws_t
 {
+	ctx_t& ctx;
 	dbuf<double> x, b, c, dj, res, keep, part, norms, pick_v, pa;
 	dbuf<double> vec; // the vectors of the cycle: six on the kept rows, one on the others
 	dbuf<rbw_set_t> st;
 	dbuf<int32_t> undo, pick_u, seg_rows;
+	explicit rbw_ws_t(ctx_t& c) : ctx(c) {}
+	rbw_ws_t(const rbw_ws_t&) = delete;
+	rbw_ws_t& operator=(const rbw_ws_t&) = delete;
+	~rbw_ws_t()
+	{
+		const pool_scope_t scope(ctx.wide);
+		if (ctx.wide_shared)
+			(void)hipStreamSynchronize(ctx.stream); // the next owner may be on another stream
+		for (dbuf<double>* d : { &x, &b, &c, &dj, &res, &keep, &part, &norms, &pick_v, &pa, &vec })
+			d->reset();
+		st.reset();
+		for (dbuf<int32_t>* d : { &undo, &pick_u, &seg_rows })
+			d->reset();
+	}
 	void reserve(int64_t nE, int64_t nR, int B, int nblk, int n_seg, int slices)
 	{
+		const pool_scope_t scope(ctx.wide);
 		const size_t cU = (size_t)(nE + nR) * B, cR = (size_t)nR * B, cE = (size_t)nE * B;
 		for (dbuf<double>* d : { &x, &b, &c, &res, &keep })
 			d->ensure(cU);
@@ -4855,7 +4871,7 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 			const bool reduced = path == path_reduced && opts.preconditioner == 0;
 			if (reduced)
 			{
-				rbw_ws_t ws;
+				rbw_ws_t ws(c);
 				bicg_w_t gm(c, Sc, nb, ws, nseg1);
 				rb_setup_t su = setup ? *setup : rb_setup_t{};
 				if (su.n_seg)
@@ -5972,6 +5988,9 @@ struct child_ctx_t
 		c.device = parent.device;
 		c.lds_per_block = parent.lds_per_block;
 		c.wall_khz = parent.wall_khz;
+		c.wide = parent.wide;
+		c.wide_shared = true;
+		c.pool->other = c.wide;
 		ESL_HIP(hipSetDevice(c.device));
 		ESL_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
 		for (auto& e : c.ev)
@@ -6037,6 +6056,8 @@ void plan_solve_many(ctx_t& c, int np, void* const* plans, const int* B, const d
 		o.graph = 0;
 	// the device-wide plans, each on a host thread of its own, joined before return
 	std::vector<std::unique_ptr<child_ctx_t>> kids;
+	if (!wide.empty())
+		ESL_HIP(hipStreamSynchronize(c.stream)); // what its solves left in the pool may go to another stream
 	for (size_t k = 0; k < wide.size(); ++k)
 		kids.push_back(std::make_unique<child_ctx_t>(c));
 	std::vector<std::exception_ptr> errs(wide.size());
