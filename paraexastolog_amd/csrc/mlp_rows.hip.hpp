@@ -14,10 +14,13 @@
 // them, one 16-byte load per lane.  The weights have such copies for both directions,
 // rounded to BF16 as the products always did, kept beside the FP32 masters and
 // rewritten by the update; activations and gradients are stored so by k_mlp_rows, with
-// rows as the summed index.  All sums are those of the layer-by-layer kernels bit for
-// bit, their splits of k included: training amplifies a difference in the last bit (an
-// activation on the other side of a BF16 rounding, through Adam's quotient) to 4e-5 of
-// the parameters in 64 steps.
+// rows as the summed index.  The sums that probabilities, gradients and parameters come
+// from are those of the layer-by-layer kernels, their splits of k included, and were the
+// same bits on 13 shapes (widths and outputs that are no multiple of a tile, 1 to 4,096
+// rows, three training steps); a row's loss, which is only reported, is added in another
+// order and differed in its last bit on three.  The order matters: training amplifies a
+// difference in the last bit (an activation on the other side of a BF16 rounding,
+// through Adam's quotient) to 4e-5 of the parameters in 64 steps.
 //
 // What bounds them: a workgroup reads all weights, 2.6 MB there and back, at the 64 bytes
 // per clock of its compute unit's cache (17 us), beside vector work and barriers; the

@@ -10,7 +10,9 @@
 // costs what a product by M costs and has two phases, so two workgroup
 // barriers, where a preconditioned step with ILU(0) has one per popcount level
 // and sweep.  BiCGStab on S, scaled from the left by the inverse of its
-// diagonal, needs no basis: five vectors of half length per set, in registers.
+// diagonal, needs no basis: five vectors of half length per set, in registers (the
+// kernels of 1,024 threads with four and two rows a thread spill 104 and 6 of them, the one
+// of 512 threads with two rows 2).
 //
 // It replaces restarted GMRES with ILU(0) as the default method of the per-set
 // solver (that one stays for sets on which this method stalls, and for callers
@@ -857,8 +859,11 @@ struct bicg_variant_t
 
 // The variants, smallest first.  A batch of more sets than compute units takes
 // two rows per thread, so that several sets share a CU; up to that many sets
-// each has a CU to itself, and one row per thread shortens its chain.
-constexpr int rb_cus = 256;
+// each has a CU to itself, and one row per thread shortens its chain.  One row / two
+// rows, us per call: 2,048 unknowns 390 / 411 for 256 sets, 462 / 417 for 257, 1,107 / 880
+// for 1,024; 936 unknowns, whose sets share a CU either way, 221 / 258 for 256, 230 / 260
+// for 512, 303 / 288 for 1,024; 696 unknowns 227 / 296, 266 / 299, 476 / 428.
+constexpr int rb_cus = 256; // of the MI355X
 constexpr size_t rb_lds_static = 3072; // upper bound of the kernel's static LDS
 // dynamic LDS of one set: the vector being multiplied, its image, the records
 inline size_t rb_lds_bytes(int64_t nU, int64_t groups, bool lrec)

@@ -4252,7 +4252,7 @@ int64_t per_set_max_unknowns(int B)
 	return 4096;
 }
 
-// algorithmic bytes of one per-set GMRES launch: the coupling structure once
+// algorithmic bytes of one per-set launch: the coupling structure once
 // (row pointers, neighbour index and code), then per set the right-hand side,
 // the iterate (read and written) and 1/D'.
 double gmres_set_bytes(const sys_t& S, int64_t nnz)
@@ -4261,7 +4261,7 @@ double gmres_set_bytes(const sys_t& S, int64_t nnz)
 }
 
 // Solves A_p z = rhs for every set of S (z holds the initial guess): one
-// workgroup per set when the system is small, device-wide GMRES otherwise.
+// workgroup per set when the system is small, device-wide otherwise.
 struct krylov_result_t
 {
 	double resid = 0.0;
@@ -4274,7 +4274,7 @@ struct krylov_result_t
 	int exact = 0;		   // sets solved by the exact dense LU
 };
 
-// device scratch of the per-set GMRES kernels (pointers only)
+// device scratch of the per-set kernels (pointers only)
 struct pss_view_t
 {
 	double *r = nullptr, *udiag = nullptr, *res = nullptr, *t = nullptr;
@@ -4367,7 +4367,7 @@ krylov_result_t collect_sets(ctx_t& c, const pss_view_t& sc, int B, double tol, 
 		kr.iters_sum += h_its[b];
 	}
 	if (check && !(kr.resid <= tol))
-		throw error(ESL_E_NUMERIC, "GMRES did not reach the tolerance: relative residual " + sci(kr.resid) +
+		throw error(ESL_E_NUMERIC, "the solve did not reach the tolerance: relative residual " + sci(kr.resid) +
 									   " after " + std::to_string(kr.iters) + " iterations");
 	if (h_res_out)
 		*h_res_out = std::move(h_res);
@@ -4376,7 +4376,7 @@ krylov_result_t collect_sets(ctx_t& c, const pss_view_t& sc, int B, double tol, 
 	return kr;
 }
 
-// scratch of the per-set GMRES kernel, grown on demand and reused
+// scratch of the per-set kernels, grown on demand and reused
 struct per_set_scratch_t
 {
 	dbuf<double> r, udiag, res, t, xk;
@@ -4415,7 +4415,7 @@ enum : int
 {
 	path_lds = 0,	  // per set, GMRES, system in LDS (private per-thread FP32 basis where it fits)
 	path_global = 1,  // per set, GMRES from global memory
-	path_wide = 2,	  // device-wide GMRES
+	path_wide = 2,	  // device-wide, GMRES
 	path_lds_mem = 3, // as 0 with the basis in global memory
 	path_lds_o3 = 4,  // as 0 with 3 workgroups per CU
 	path_reduced = 5  // per set, BiCGStab on the parity-reduced system
@@ -4840,7 +4840,7 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 			return sc.view();
 		});
 		if (kr.missed && throw_on_miss)
-			throw error(ESL_E_NUMERIC, "GMRES did not reach the tolerance: relative residual " + sci(kr.resid) +
+			throw error(ESL_E_NUMERIC, "the solve did not reach the tolerance: relative residual " + sci(kr.resid) +
 										   " after " + std::to_string(kr.iters) + " iterations");
 	}
 	else
@@ -4932,7 +4932,7 @@ krylov_result_t krylov_solve(ctx_t& c, const sys_t& S, int n_seg, const double* 
 				if (!done64)
 				{
 					if (throw_on_miss)
-						throw error(ESL_E_NUMERIC, "GMRES did not reach the tolerance: relative residual " +
+						throw error(ESL_E_NUMERIC, "the solve did not reach the tolerance: relative residual " +
 													   sci(cmax) + " after " + std::to_string(it) + " iterations");
 					kr.missed += cb; // an upper bound: the caller reads every set's residual
 				}
@@ -4985,7 +4985,8 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 	if (n_t)
 		k_term_reached<<<ceil_div(n_t, sblock), sblock, 0, c.stream>>>(n_t, g.reordered.get(), g.rank.get(),
 																		 P.reach.get(), reached.get());
-	// with few terminal states their order comes along, in the same wait
+	// with few terminal states their order comes along, in the same wait (plan of 32,768
+	// terminal states 463 us with, 483 without; 64,512: 587 and 576, most are not needed)
 	std::vector<int32_t> h_reached, h_reord;
 	readback_t rd(c);
 	rd.add(h_reached, reached.get(), (size_t)T);
@@ -5096,6 +5097,8 @@ void plan_build(ctx_t& c, graph_t& g, const double* d_x0, plan_t& P)
 		std::vector<int32_t> h_count, h_j;
 		std::vector<double> h_x;
 		// few states: packed into arrays for all of them, read with their number in one wait
+		// (plan of 10 nodes 430 us so, 507 with a wait for the number; 13 nodes 444 and 506, 17
+		// nodes 937 and 903, 20 nodes 1,358 and 576)
 		const bool few = n <= 8192;
 		int64_t count = n;
 		if (!few)
@@ -6050,8 +6053,9 @@ void plan_solve_many(ctx_t& c, int np, void* const* plans, const int* B, const d
 	}
 	// No capture beside the host threads below, which allocate and free: a program
 	// that alternates between such batches would capture anew on every call while
-	// they run (one such run ended in a host segmentation fault), and what a replay
-	// saves is microseconds beside milliseconds of device-wide solves.
+	// they run.  One such run ended in a host segmentation fault whose cause is not
+	// known, and what a replay saves is microseconds beside milliseconds of device-wide
+	// solves.
 	if (!wide.empty())
 		o.graph = 0;
 	// the device-wide plans, each on a host thread of its own, joined before return
@@ -6267,8 +6271,8 @@ void plan_gather_terminal(ctx_t& c, const void* p, int B, const double* d_final,
 // Times candidate schedules of a plan on the caller's own batch and keeps the
 // fastest one that meets the tolerance: per-set LDS-resident / per-set from
 // global memory / device-wide / per-set LDS-resident with the basis in global
-// memory / per-set LDS-resident with the private basis at 3 or 2 workgroups per
-// CU, restart length 16 / 24 / 32 / 64.  Each candidate runs once untimed
+// memory / per-set LDS-resident with the private basis at 3 workgroups per CU,
+// restart length 16 / 24 / 32 / 64, and the reduced solver.  Each candidate runs once untimed
 // (graph capture, buffer growth), then two timed blocks of four runs (the
 // better block's mean).  The
 // chosen schedule then runs once more, so d_final holds its results.  Later
